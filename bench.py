@@ -11,14 +11,13 @@ pass per conformer axis).  One bench "step" = one exchange interval (100 MC
 steps of all 1,760 replicas + one exchange point), so the default --steps 100 is the whole
 10,000-step job.  FP32 arithmetic, synthetic data (seeded generator).
 
-Prints one JSON line (value = replica-steps/s, on the library's default two
-streams).  The roofline object covers the dominant kernel (gd_pair_kernel<LC>,
-LC ligand atoms per lane) on a pipeline basis: algorithmic FP32 flops of one
-MC step's pair work / the steady-state MC step period, from HIP events at the
-first stream's pair launch of every 16th MC step (the whole step, tail
-kernels and exchange points included, is charged to the pair kernel); the
-half-launch mean, the step's pair span and an isolated one-stream launch
-are reported beside it.  cpu_baseline times the CPU oracle (a restatement of
+Prints one JSON line (value = replica-steps/s).  The roofline object covers
+the dominant kernel (the stepping kernel gd_chain_kernel<LC>, LC ligand atoms
+per lane, one launch per exchange interval): algorithmic FP32 flops of one MC
+step's pair work / the MC step period inside its launches (HIP events around
+each launch over its steps; reduction, accept and proposal are charged to
+it); an isolated launch of the pair work alone (gd_pair_kernel<LC>) is
+reported beside it.  cpu_baseline times the CPU oracle (a restatement of
 the reference CPU backend, in the reference's FP32 expression order) on a
 bounded sample of the same workload.
 
@@ -724,20 +723,17 @@ def main():
     sclk_after = C.c_double()
     g.check(g.lib().gd_measure_sclk(200, C.byref(sclk_after)), "gd_measure_sclk")
     value, jobs_per_s = c2_rates(job.n_rep, steps, wall)
-    # Two streams step the two halves of the replica blocks, so a step's two
-    # pair half-launches overlap each other and the other half's reduce and
-    # finish kernels: the pair kernel's rate is its flops per MC step over the
-    # steady-state step period (HIP events at the pair launches of every 16th
-    # step, on the pair kernel's stream), which charges the whole step -- tail
-    # kernels and exchange points included -- to the pair kernel.
+    # The stepping kernel takes an exchange interval's MC steps in one launch:
+    # its rate is the pair flops of a step over the launch time per step, which
+    # charges the whole step -- reduction, accept, proposal -- to it.
     period_ms = st.ms_step_period
     achieved = flops_step / (period_ms / 1000.0) / 1e12
-    half_ms = st.ms_pair_kernel / max(1, st.n_pair_launch)
-    # the same kernel alone: one stream, one launch per step, event-timed
-    dev.set_streams(1)
-    _, st1 = dev.dock(g.make_mc(400, steps_per_dump=400, steps_per_exchange=STEPS_PER_EXCHANGE,
-                                move_mode="gaussian", seed=SEED, axes=AXES), stats=True)
-    dev.set_streams(2)
+    # the pair work alone: stepped by launches on one stream, event-timed
+    iso_dev = g.DeviceJob(job)
+    iso_dev.set_streams(1)
+    _, st1 = iso_dev.dock(g.make_mc(400, steps_per_dump=400, steps_per_exchange=STEPS_PER_EXCHANGE,
+                                    move_mode="gaussian", seed=SEED, axes=AXES), stats=True)
+    iso_dev.close()
     iso_ms = st1.ms_pair_kernel / max(1, st1.n_pair_launch)
     iso = flops_step / (iso_ms / 1000.0) / 1e12
     traffic = None
@@ -784,20 +780,20 @@ def main():
             "unit": "TFLOP/s",
             "frac": achieved / PEAK_FP32_TFLOPS,
             "traffic": traffic,
-            "kernel": "gd_pair_kernel<%d>" % dev.tiling()[0],
+            "kernel": "gd_chain_kernel<%d>" % dev.tiling()[0],
             "flops_per_launch": flops_step,
             "prt_pairs_per_launch": prt_pairs,
-            "basis": "one launch = one MC step's pair work, two half-launches on two streams; its "
-                     "duration = the steady-state MC step period (events at the pair launches of every "
-                     "16th step on the pair kernel's stream), the whole step charged to the pair kernel",
+            "basis": "one launch = one MC step's pair work inside the stepping kernel; its duration = the "
+                     "kernel's time over its steps (HIP events around each exchange interval's launch), "
+                     "reduction, accept and proposal included",
             "mean_launch_ms": period_ms,
-            "launches_timed": st.n_pair_launch // 2,
-            "half_launch_mean_ms": half_ms,
-            "pair_span_mean_ms": st.ms_pair_span,
+            "launches_timed": st.n_pair_launch,
             "prt_only_tflops": PRT_FLOPS * prt_pairs / (period_ms / 1000.0) / 1e12,
             "isolated": {"streams": 1, "mean_launch_ms": iso_ms, "achieved": iso,
                          "frac": iso / PEAK_FP32_TFLOPS, "launches_timed": st1.n_pair_launch,
-                         "note": "the same launch alone on one stream, 400 MC steps after the timed region"},
+                         "kernel": "gd_pair_kernel<%d>" % dev.tiling()[0],
+                         "note": "the pair work as launches of its own on one stream, 400 MC steps after "
+                                 "the timed region"},
         },
     }
     # the same job in the reference's plain shape: dumps of 200 steps, each

@@ -114,6 +114,42 @@ struct GdItem {           // one 4-wave work group of the pair kernel
   int b;                  // protein tile group: tiles GD_GROUP*b .. GD_GROUP*b + GD_GROUP-1
 };
 
+// Stepping kernel: the slices of a block are reduced two at a time, GD_RT times.
+#define GD_RT (GD_RK * 4 / GD_GROUP)
+// Its counters (32-bit words), a line each: next ticket, queue entries written,
+// the out-of-time mark; then per block the items done and the team's groups done.
+#define GD_SY_TICKET 0
+#define GD_SY_TAIL 32
+#define GD_SY_FAILED 64
+#define GD_SY_HEAD 96
+#define GD_SY_BLOCK 64
+#define GD_CHAIN_WAIT_S 2.0  // seconds until one wait of the stepping kernel gives up
+
+struct GdChainBlock {     // one 64-replica block of the stepping kernel
+  int job;
+  int rb;                 // first replica
+  int item0, n_items;     // its pair items in the launch's list
+};
+
+struct GdChain {          // arguments of one launch of the stepping kernel
+  const GdJob *jobs;
+  const struct GdItem *items;        // each job's (chunk, tile group) items, in its order
+  const struct GdChainBlock *blocks; // [n_blocks]
+  unsigned *sync;
+  unsigned long long *queue;         // entry k at k * stride: epoch << 32 | block << 8 | number
+  int stride;             // 64-bit words from entry to entry
+  int per_entry;          // items of an entry (of a block's last one, what is left)
+  unsigned epoch;         // of this launch: entries of earlier ones do not count
+  int n_blocks;
+  int n_entries;          // queue entries of a step
+  unsigned steps_before;  // steps of the launches before, which the counters hold
+  int n_teams, team;      // finisher teams, groups of a team
+  int n_steps;            // steps of the launch (the initial pass included)
+  int step0;              // launch step of the first one
+  int init;               // the first step is the initial-energy pass
+  long long wait_ticks;   // bound of one wait, in ticks of the constant-rate counter
+};
+
 struct GdBlock {          // one workgroup of the finish / transform kernels
   int job;
   int rb;

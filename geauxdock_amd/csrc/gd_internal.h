@@ -11,6 +11,28 @@
 #include "gd_device.h"
 #include "gd_rng.h"
 
+namespace gdr {
+// Work lists, queue and counters of the stepping kernel for a list of jobs.
+struct ChainList {
+  const GdItem *d_items = nullptr;
+  const GdChainBlock *d_blocks = nullptr;
+  unsigned *d_sync = nullptr;
+  unsigned long long *d_queue = nullptr;
+  int n_blocks = 0, n_items = 0;        // pair items of a step
+  int n_entries = 0, per_entry = 1;     // queue entries of a step
+  int stride = 1;
+  int cap_steps = 0;                    // steps the queue holds
+  int n_teams = 0, team = 0;            // finisher teams, groups of a team
+  unsigned epoch = 0, steps = 0;        // launches and their steps since the counters were zero
+  int lds = 0;                          // LDS added to a group's, which bounds the groups of a CU
+  double wait_s = GD_CHAIN_WAIT_S;      // bound of one wait in the kernel
+  double step_pairs = 0;                // (atom, point) pairs of one step
+  // The host lists (items of each job, blocks) and the launch shape.
+  void shape(const std::vector<const GdJob *> &jobs);
+  size_t queue_bytes() const { return (size_t)n_entries * stride * cap_steps * sizeof(unsigned long long); }
+};
+}  // namespace gdr
+
 struct gd_job {
   GdJob h{};                 // host mirror of the device struct
   GdJob *d_job = nullptr;    // device copy
@@ -34,11 +56,15 @@ struct gd_job {
   // [b0_part[k], b0_part[k] + nb_part[k]), each with its items (the job's items
   // of those blocks, in the job's order) and a stream (part 0: the job's own)
   static constexpr int kMaxParts = 4;
+  bool by_launches = false;  // step by launches on n_streams streams (gd_job_set_streams)
   GdItem *d_items_part[kMaxParts] = {};
   int n_items_part[kMaxParts] = {}, nb_part[kMaxParts] = {}, b0_part[kMaxParts] = {};
   int n_parts = 0;
   int n_streams = 2;         // streams the plain path steps on (1 .. kMaxParts)
   hipStream_t part_stream[kMaxParts] = {};
+  gdr::ChainList chain;      // the stepping kernel's list, its queue and its counters
+  void *d_chain = nullptr;
+  size_t chain_bytes = 0;
   // protein points in source order, laid out on the device per tile count
   std::vector<float4> src_pco;     // [n_prt][P]
   std::vector<float4> src_pattr;   // [P]
@@ -71,6 +97,11 @@ gd_status launch_finish(const GdJob *d_jobs, const GdBlock *d_blocks, int n_bloc
                         int step, hipStream_t s);
 gd_status launch_transform(const GdJob *d_jobs, const GdBlock *d_blocks, int n_blocks, hipStream_t s);
 gd_status launch_exchange(const GdJob *d_jobs, const GdExch *d_ex, int n_ex, hipStream_t s);
+size_t chain_sync_bytes(int n_blocks);
+// Steps that one launch may take (0: this list is stepped by launches).
+int chain_max_steps(const ChainList &c);
+gd_status launch_chain(ChainList &c, const GdJob *d_jobs, int step0, int n_steps, bool init,
+                       hipStream_t s);
 // One conformer swap sub-step along `axis` (0 ligand, 1 protein) for the jobs
 // of the lists whose swr[job] round is >= 0: propose, pair (the caller's
 // launcher), reduce, finish(EVAL), accept.  launch_step / step_base as for the

@@ -64,13 +64,23 @@ __device__ __forceinline__ float gd_exp2(float x) { return __builtin_amdgcn_exp2
 #if defined(__HIP_DEVICE_COMPILE__)
 #define GD_AS_CONST __attribute__((address_space(4)))
 #define GD_AS_GLOBAL __attribute__((address_space(1)))
+#define GD_AS_LDS __attribute__((address_space(3)))
 #else  // host pass of this translation unit: kernels are only declared there
 #define GD_AS_CONST
 #define GD_AS_GLOBAL
+#define GD_AS_LDS
 #endif
 template <class T>
 __device__ __forceinline__ const GD_AS_CONST T *gd_c(const T *p) {
   return (const GD_AS_CONST T *)p;
+}
+// The same pointer, opaque to the compiler: what is read through it is read
+// here, not earlier and not kept for later (scalar registers).
+template <class T>
+__device__ __forceinline__ const GD_AS_CONST T &gd_reread(const GD_AS_CONST T &x) {
+  unsigned long long q = (unsigned long long)&x;
+  asm volatile("" : "+s"(q));
+  return *(const GD_AS_CONST T *)q;
 }
 template <class T>
 __device__ __forceinline__ GD_AS_GLOBAL T *gd_g(T *p) {
@@ -82,6 +92,29 @@ __device__ __forceinline__ const GD_AS_GLOBAL T *gd_g(const T *p) {
   return (const GD_AS_GLOBAL T *)p;
 }
 #endif
+
+// Loads and stores of arrays that other work groups of the same launch write or
+// read (the stepping kernel).  AG: agent scope, relaxed -- the access goes past
+// the CU's and the XCD's caches to where every XCD sees it, so no cache has to
+// be written back or invalidated around it (an agent-scope release fence costs
+// 2 us of L2 writeback per work group here).  A writer waits for its stores
+// (gd_drain) before it announces them; a reader reads after it saw the
+// announcement.
+template <bool AG, class T>
+__device__ __forceinline__ T gd_ld(const GD_AS_GLOBAL T *p) {
+  if constexpr (AG)
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else
+    return *p;
+}
+template <bool AG, class T>
+__device__ __forceinline__ void gd_st(GD_AS_GLOBAL T *p, T v) {
+  if constexpr (AG)
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else
+    *p = v;
+}
+__device__ __forceinline__ void gd_drain() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // FP32 -> FP64 conversions that the compiler may not move (see the H-bond
 // term); _s takes a wave-uniform value held in a scalar register.
@@ -314,12 +347,12 @@ __device__ __forceinline__ void gd_pair_atoms_load(
 // tile holds the same mix of near and far points and waves cost the same.
 template <int LC, int CLS>
 __device__ __forceinline__ void gd_pair_class(
-    const GD_AS_CONST GdJob &J, const int lo, const int hi, const int b, const unsigned pcoff,
-    const GdPairConst &k, const float pmf_a,
+    const GD_AS_CONST GdJob &J0, const int b, const unsigned pcoff, const GdPairConst &k, const float pmf_a,
     const float (&lx)[LC], const float (&ly)[LC], const float (&lz)[LC], const unsigned (&trow)[LC],
     float (&ele)[LC], float (&hpc)[LC], float &evdw, float &epmf, float &epsp, float &ehdb) {
+  const GD_AS_CONST GdJob &J = gd_reread(J0);
   const int P = J.P, nP = J.nP;
-  const int p0 = lo + b;
+  const int hi = J.pcls[CLS + 1], p0 = J.pcls[CLS] + b;
   if (p0 >= hi) return;
   const GD_AS_GLOBAL char *__restrict__ pcb = (const GD_AS_GLOBAL char *)gd_g(J.pcoord);
   const GD_AS_GLOBAL char *__restrict__ pab = (const GD_AS_GLOBAL char *)gd_g(J.pattr);
@@ -389,17 +422,13 @@ __device__ __forceinline__ void gd_pair_points(
   // log2(e)/2 held in a VGPR: a VALU op reads at most one SGPR or literal
   float pmf_a;
   asm("v_mov_b32 %0, 0x3f38aa3b" : "=v"(pmf_a));  // log2(e) / 2
-  gd_pair_class<LC, 0>(J, J.pcls[0], J.pcls[1], b, pc, k, pmf_a, lx, ly, lz, trow, ele, hpc,
-                       evdw, epmf, epsp, ehdb);
-  gd_pair_class<LC, 1>(J, J.pcls[1], J.pcls[2], b, pc, k, pmf_a, lx, ly, lz, trow, ele, hpc,
-                       evdw, epmf, epsp, ehdb);
-  gd_pair_class<LC, 2>(J, J.pcls[2], J.pcls[3], b, pc, k, pmf_a, lx, ly, lz, trow, ele, hpc,
-                       evdw, epmf, epsp, ehdb);
-  gd_pair_class<LC, 3>(J, J.pcls[3], J.pcls[4], b, pc, k, pmf_a, lx, ly, lz, trow, ele, hpc,
-                       evdw, epmf, epsp, ehdb);
+  gd_pair_class<LC, 0>(J, b, pc, k, pmf_a, lx, ly, lz, trow, ele, hpc, evdw, epmf, epsp, ehdb);
+  gd_pair_class<LC, 1>(J, b, pc, k, pmf_a, lx, ly, lz, trow, ele, hpc, evdw, epmf, epsp, ehdb);
+  gd_pair_class<LC, 2>(J, b, pc, k, pmf_a, lx, ly, lz, trow, ele, hpc, evdw, epmf, epsp, ehdb);
+  gd_pair_class<LC, 3>(J, b, pc, k, pmf_a, lx, ly, lz, trow, ele, hpc, evdw, epmf, epsp, ehdb);
 }
 
-template <int LC>
+template <int LC, bool AG = false>
 __device__ __forceinline__ void gd_pair_item(const GdJob *__restrict__ jobs, const GdItem it,
                                              const int lane, const int wave,
                                              float (*__restrict__ red)[GD_NLIN + LC][64]) {
@@ -418,9 +447,9 @@ __device__ __forceinline__ void gd_pair_item(const GdJob *__restrict__ jobs, con
 #pragma unroll
   for (int j = 0; j < LC; ++j) {
     const int l = l0 + min(j, nl - 1);
-    lx[j] = coords[(size_t)(3 * l + 0) * Rp + r];
-    ly[j] = coords[(size_t)(3 * l + 1) * Rp + r];
-    lz[j] = coords[(size_t)(3 * l + 2) * Rp + r];
+    lx[j] = gd_ld<AG>(coords + (size_t)(3 * l + 0) * Rp + r);
+    ly[j] = gd_ld<AG>(coords + (size_t)(3 * l + 1) * Rp + r);
+    lz[j] = gd_ld<AG>(coords + (size_t)(3 * l + 2) * Rp + r);
     trow[j] = (unsigned)atoms[l0 + j].tidx;
     ele[j] = 0.0f;
     hpc[j] = 0.0f;
@@ -485,7 +514,7 @@ __device__ __forceinline__ void gd_pair_item(const GdJob *__restrict__ jobs, con
           d += __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
         }
       }
-      pm[((size_t)m * nL + it.a) * Rp + r_e] = d;
+      gd_st<AG>(pm + ((size_t)m * nL + it.a) * Rp + r_e, d);
     }
   }
 
@@ -514,11 +543,13 @@ __device__ __forceinline__ void gd_pair_item(const GdJob *__restrict__ jobs, con
 #pragma unroll
     for (int w = 1; w < GD_GROUP; ++w) v += red[w][q][lane_e];
     if (q < GD_NLIN)
-      pl[((size_t)q * nS + slot) * Rp + r_e] = v;
+      gd_st<AG>(pl + ((size_t)q * nS + slot) * Rp + r_e, v);
     else if (q - GD_NLIN < nl)
-      ph[((size_t)(l0 + q - GD_NLIN) * nG + it.b) * Rp + r_e] = v;
+      gd_st<AG>(ph + ((size_t)(l0 + q - GD_NLIN) * nG + it.b) * Rp + r_e, v);
   }
-  __syncthreads();  // red[] is reused by the next item of a persistent group
+  // red[] is reused by the next item of a persistent group (the stepping
+  // kernel has its own barrier there)
+  if constexpr (!AG) __syncthreads();
 }
 
 // One work group of GD_GROUP waves per item (grid = items).
@@ -594,11 +625,13 @@ typedef const GD_AS_CONST GdJob GdJobC;
 // One atom of the transform x = R a + t (kernel_cpp_montecarlo_soa.C:274-293),
 // the conformer-relative products summed first and the lab-frame offset t
 // added last, into the [L][3][Rp] coordinate layout.
+template <bool AG = false>
 __device__ __forceinline__ void gd_put_atom(GD_AS_GLOBAL float *co, int Rp, int r, int l,
                                             const float R[9], const float t[3], const float4 a) {
-  co[(size_t)(3 * l + 0) * Rp + r] = __builtin_fmaf(R[0], a.x, __builtin_fmaf(R[1], a.y, R[2] * a.z)) + t[0];
-  co[(size_t)(3 * l + 1) * Rp + r] = __builtin_fmaf(R[3], a.x, __builtin_fmaf(R[4], a.y, R[5] * a.z)) + t[1];
-  co[(size_t)(3 * l + 2) * Rp + r] = __builtin_fmaf(R[6], a.x, __builtin_fmaf(R[7], a.y, R[8] * a.z)) + t[2];
+  GD_AS_GLOBAL float *o = co + (size_t)(3 * l) * Rp + r;
+  gd_st<AG>(o, __builtin_fmaf(R[0], a.x, __builtin_fmaf(R[1], a.y, R[2] * a.z)) + t[0]);
+  gd_st<AG>(o + Rp, __builtin_fmaf(R[3], a.x, __builtin_fmaf(R[4], a.y, R[5] * a.z)) + t[1]);
+  gd_st<AG>(o + (size_t)2 * Rp, __builtin_fmaf(R[6], a.x, __builtin_fmaf(R[7], a.y, R[8] * a.z)) + t[2]);
 }
 
 __device__ __forceinline__ void gd_transform_atoms(GdJobC &J, int r, const float R[9],
@@ -658,75 +691,152 @@ __global__ __launch_bounds__(256) void gd_move_draws_kernel(uint64_t seed, uint3
 }
 
 // ---------------------------------------------------------------------------
-// Sum of n values at stride `st` (floats) with eight loads in flight, the last
-// partial block too (indices clamped to n - 1, masked to zero); element q goes
-// to accumulator q mod 8, so the order depends only on n and is reproducible.
-__device__ __forceinline__ float gd_sum_strided(const GD_AS_GLOBAL float *__restrict__ p, int n,
-                                                size_t st) {
+// The first n rows of 64 partial sums, 1 <= n <= N (the last one is read again
+// for the others): row i at base + i Rp floats, r the lane's column.  The address is a scalar base and a 32-bit lane offset, and the
+// offset and the row count are opaque at each row: scalar bases and tests of all
+// the rows made up front took more scalar registers than there are.
+template <bool AG, int N>
+__device__ __forceinline__ void gd_load_rows_of(const GD_AS_GLOBAL float *base, const int n, const int Rp,
+                                                const int r, float (&v)[N]) {
+  const GD_AS_GLOBAL char *b = (const GD_AS_GLOBAL char *)base;
+  unsigned off = (unsigned)r * 4u;
+  int n_i = n;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    asm volatile("" : "+v"(off), "+s"(n_i));
+    v[i] = gd_ld<AG>((const GD_AS_GLOBAL float *)(b + off));
+    off += i + 1 < n_i ? (unsigned)Rp * 4u : 0u;
+  }
+}
+// Their sum, one after the other.
+template <int N>
+__device__ __forceinline__ float gd_add_rows(const int n, const float (&v)[N]) {
+  float acc = 0.0f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    acc += i < n ? v[i] : 0.0f;
+  }
+  return acc;
+}
+// Their sum by eight accumulators, element q to accumulator q mod 8: the order of
+// long sums, which depends only on n.
+template <int N>
+__device__ __forceinline__ float gd_add_rows8(const int n, const float (&v)[N]) {
+  float a[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) a[i] = 0.0f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) a[i & 7] += i < n ? v[i] : 0.0f;
+  return ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+}
+// The same sum of any number of rows, eight loads in flight.
+template <bool AG>
+__device__ __forceinline__ float gd_sum_strided(const GD_AS_GLOBAL float *__restrict__ base, int n,
+                                                const int Rp, const int r) {
   float a[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) a[i] = 0.0f;
   for (int q = 0; q < n; q += 8) {
     float v[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = p[(size_t)min(q + i, n - 1) * st];
+    gd_load_rows_of<AG, 8>(base + (size_t)q * Rp, n - q, Rp, r, v);
 #pragma unroll
     for (int i = 0; i < 8; ++i) a[i] += q + i < n ? v[i] : 0.0f;
   }
   return ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
 }
 
-// Common shapes of the reduce kernel: at most QL linear slots, one atom and one
-// MCS row per wave, at most QN tile groups and chunks.  Every load of the wave
-// is issued before the first sum, one wait in all.  Indices are clamped into
-// range and the extra values masked to zero; the sums run in slot order, so
-// the result does not depend on QL or QN.
-template <int QL, int QN>
-__device__ __forceinline__ void gd_reduce_common(
-    const GD_AS_GLOBAL float *__restrict__ part_lin, const GD_AS_GLOBAL float *__restrict__ part_hpc,
-    const GD_AS_GLOBAL float *__restrict__ part_mcs, const GD_AS_CONST GdAtom *__restrict__ atoms,
-    const GD_AS_CONST float2 *__restrict__ mcsrow, const int nS, const int nG, const int nL, const int L,
-    const int M, const int Rp, const int r, const int wi, const int q0, const int q1, float (&acc)[8]) {
-  const int ql = max(q1 - 1, q0), l = min(wi, L - 1), m = min(wi, max(M - 1, 0));
+// ---------------------------------------------------------------------------
+// Reduction of a block: 4 GD_RK waves split the partial slots; lanes are
+// replicas.  Wave wi takes a contiguous share of every linear term's slots, atoms
+// l = wi, wi + 4 GD_RK, ... (the hpc sum over tile groups, then the non-linear
+// restraint) and MCS rows m = wi, wi + 4 GD_RK, ... (the sum over chunks, then
+// tcc sqrt(d/n)).  Four waves' values make a slice, summed in a fixed order, and
+// the finish sums the GD_RK slices in a fixed order.  The reduction reads most of
+// the step's partials, and its time is the latency of its loads: as many as the
+// registers hold are issued before the first sum (QL rows of each linear term
+// and QN of the others; BOTH: of both the others together).  SEQ: the sums run
+// one after the other, else by eight accumulators; which depends on the complex
+// and its tiling only, and the result does not depend on QL, QN and BOTH.
+template <bool AG, bool SEQ, bool BOTH, int QL, int QN>
+__device__ __forceinline__ void gd_reduce_shape(GdJobC &J, const int r, const int wi, const int q0,
+                                                const int n, float (&acc)[8]) {
+  const int nG = J.nG, nL = J.nL, nS = nL * nG, L = J.L, M = J.M, Rp = J.Rp, W = 4 * GD_RK;
+  auto sum = [&](int k, auto &v) { return SEQ ? gd_add_rows(k, v) : gd_add_rows8(k, v); };
+  auto hpc = [&](int l, auto &v) {  // hpc of an atom (energy_prt_v1.C:132-133)
+    const GdAtom at = gd_c(J.atoms)[l];
+    const float t = (sum(nG, v) - at.hpl0) / at.hpl1;
+    acc[6] += 0.5f * t * t - at.hpl2;
+  };
+  auto mcs = [&](int m, auto &v) {  // an MCS row (energy_mcs_v1.C:5-29)
+    const float2 row = gd_c(J.mcsrow)[m];
+    acc[7] += row.x * sqrtf(sum(nL, v) / row.y);
+  };
+  auto load_hpc = [&](int l, auto &v) {
+    gd_load_rows_of<AG>(gd_g((const float *)J.part_hpc) + (size_t)min(l, L - 1) * nG * Rp, nG, Rp, r, v);
+  };
+  auto load_mcs = [&](int m, auto &v) {
+    gd_load_rows_of<AG>(gd_g((const float *)J.part_mcs) + (size_t)min(m, max(M - 1, 0)) * nL * Rp, nL, Rp, r,
+                        v);
+  };
   float vl[GD_NLIN][QL], vh[QN], vm[QN];
 #pragma unroll
   for (int c = 0; c < GD_NLIN; ++c)
+    gd_load_rows_of<AG>(gd_g((const float *)J.part_lin) + ((size_t)c * nS + min(q0, nS - 1)) * Rp, n, Rp, r,
+                        vl[c]);
+  load_mcs(wi, vm);
+  if (BOTH) load_hpc(wi, vh);
 #pragma unroll
-    for (int i = 0; i < QL; ++i) vl[c][i] = part_lin[((size_t)c * nS + min(q0 + i, ql)) * Rp + r];
+  for (int c = 0; c < GD_NLIN; ++c) acc[c] = sum(n, vl[c]);
+  if (!BOTH) {
 #pragma unroll
-  for (int i = 0; i < QN; ++i) vh[i] = part_hpc[((size_t)l * nG + min(i, nG - 1)) * Rp + r];
-#pragma unroll
-  for (int i = 0; i < QN; ++i) vm[i] = part_mcs[((size_t)m * nL + min(i, nL - 1)) * Rp + r];
-#pragma unroll
-  for (int c = 0; c < GD_NLIN; ++c)
-#pragma unroll
-    for (int i = 0; i < QL; ++i) acc[c] += q0 + i < q1 ? vl[c][i] : 0.0f;
-  float h = 0.0f, d = 0.0f;
-#pragma unroll
-  for (int i = 0; i < QN; ++i) {
-    h += i < nG ? vh[i] : 0.0f;
-    d += i < nL ? vm[i] : 0.0f;
+    for (int c = 0; c < GD_NLIN; ++c) asm volatile("" : "+v"(acc[c]));  // the rows' registers are free here
+    load_hpc(wi, vh);
   }
-  if (wi < L) {  // hpc per atom (energy_prt_v1.C:132-133)
-    const GdAtom at = atoms[l];
-    const float t = (h - at.hpl0) / at.hpl1;
-    acc[6] += 0.5f * t * t - at.hpl2;
+  if (wi < M) mcs(wi, vm);
+  if (wi < L) hpc(wi, vh);
+  for (int l = wi + W; l < L; l += W) {
+    load_hpc(l, vh);
+    hpc(l, vh);
   }
-  if (wi < M) {  // MCS rows (energy_mcs_v1.C:5-29)
-    const float2 row = mcsrow[m];
-    acc[7] += row.x * sqrtf(d / row.y);
+  for (int m = wi + W; m < M; m += W) {
+    load_mcs(m, vm);
+    mcs(m, vm);
   }
 }
 
-// ---------------------------------------------------------------------------
-// Reduce kernel: GD_RK work groups (4 waves) per 64-replica block; lanes are
-// replicas.  The 4 GD_RK waves of a block split the partial slots: each takes a
-// contiguous share of every linear term's slots, atoms l = w, w + 4 GD_RK, ...
-// (the hpc sum over tile groups, then the non-linear restraint) and MCS rows
-// m = w, w + 4 GD_RK, ... (the sum over chunks, then tcc sqrt(d/n)).  A group
-// sums its 4 waves in a fixed order and writes 8 values per replica; the
-// finish kernel sums the GD_RK slices in a fixed order.  The reduction reads
-// most of the step's partials, so it is spread over many groups: one group per
+template <bool AG>
+__device__ __forceinline__ void gd_reduce_wave(GdJobC &J, const int r, const int wi, float (&acc)[8]) {
+  const int W = 4 * GD_RK, nG = J.nG, nL = J.nL, L = J.L, M = J.M, Rp = J.Rp, nS = nL * nG;
+#pragma unroll
+  for (int c = 0; c < 8; ++c) acc[c] = 0.0f;
+  const int q0 = (int)(((long long)nS * wi) / W), n = (int)(((long long)nS * (wi + 1)) / W) - q0;
+  // short sums run in slot order
+  const bool small = L <= W && M <= W;
+  if (small && nS <= 2 * W && nG <= 12 && nL <= 12) {
+    gd_reduce_shape<AG, true, true, 2, 12>(J, r, wi, q0, n, acc);
+  } else if (small && n <= 4 && nG <= 16 && nL <= 16) {
+    gd_reduce_shape<AG, true, true, 4, 16>(J, r, wi, q0, n, acc);
+  } else if (n <= 4 && nG <= 20 && nL <= 20) {
+    gd_reduce_shape<AG, false, false, 4, 20>(J, r, wi, q0, n, acc);
+  } else {
+#pragma unroll
+    for (int c = 0; c < GD_NLIN; ++c)
+      acc[c] = gd_sum_strided<AG>(gd_g((const float *)J.part_lin) + ((size_t)c * nS + q0) * Rp, n, Rp, r);
+    for (int l = wi; l < L; l += W) {  // hpc per atom (energy_prt_v1.C:132-133)
+      const float h = gd_sum_strided<AG>(gd_g(J.part_hpc) + (size_t)l * nG * Rp, nG, Rp, r);
+      const GdAtom at = gd_c(J.atoms)[l];
+      const float t = (h - at.hpl0) / at.hpl1;
+      acc[6] += 0.5f * t * t - at.hpl2;
+    }
+    for (int m = wi; m < M; m += W) {  // MCS rows (energy_mcs_v1.C:5-29)
+      const float d = gd_sum_strided<AG>(gd_g(J.part_mcs) + (size_t)m * nL * Rp, nL, Rp, r);
+      const float2 row = gd_c(J.mcsrow)[m];
+      acc[7] += row.x * sqrtf(d / row.y);
+    }
+  }
+}
+
+// Reduce kernel: GD_RK work groups (4 waves, one slice) per block; one group per
 // block kept too few loads in flight.
 __global__ __launch_bounds__(256) void gd_reduce_kernel(const GdJob *__restrict__ jobs,
                                                          const GdBlock *__restrict__ blocks) {
@@ -735,42 +845,8 @@ __global__ __launch_bounds__(256) void gd_reduce_kernel(const GdJob *__restrict_
   const GdBlock bk = gd_c(blocks)[bi];
   GdJobC &J = gd_c(jobs)[bk.job];
   const int lane = threadIdx.x & 63, wave = gd_uniform((int)(threadIdx.x >> 6));
-  const int r = bk.rb + lane;
-  const int Rp = J.Rp;
-  const int W = 4 * GD_RK, wi = 4 * k + wave;
-  const int nS = J.nL * J.nG;
-  const GD_AS_GLOBAL float *part_lin = gd_g(J.part_lin);
-  const GD_AS_GLOBAL float *part_hpc = gd_g(J.part_hpc);
-  const GD_AS_GLOBAL float *part_mcs = gd_g(J.part_mcs);
-  const GD_AS_CONST GdAtom *atoms = gd_c(J.atoms);
-  const GD_AS_CONST float2 *mcsrow = gd_c(J.mcsrow);
   float acc[8];
-#pragma unroll
-  for (int c = 0; c < 8; ++c) acc[c] = 0.0f;
-  const int q0 = (int)(((long long)nS * wi) / W), q1 = (int)(((long long)nS * (wi + 1)) / W);
-  const int nG = J.nG, nL = J.nL, L = J.L, M = J.M;
-  if ((nS + W - 1) / W <= 2 && nG <= 12 && nL <= 12 && L <= W && M <= W) {
-    gd_reduce_common<2, 12>(part_lin, part_hpc, part_mcs, atoms, mcsrow, nS, nG, nL, L, M, Rp, r, wi, q0,
-                            q1, acc);
-  } else if (q1 - q0 <= 4 && nG <= 16 && nL <= 16 && L <= W && M <= W) {
-    gd_reduce_common<4, 16>(part_lin, part_hpc, part_mcs, atoms, mcsrow, nS, nG, nL, L, M, Rp, r, wi, q0,
-                            q1, acc);
-  } else {
-#pragma unroll
-    for (int c = 0; c < GD_NLIN; ++c)
-      acc[c] = gd_sum_strided(part_lin + ((size_t)c * nS + q0) * Rp + r, q1 - q0, (size_t)Rp);
-    for (int l = wi; l < L; l += W) {  // hpc per atom (energy_prt_v1.C:132-133)
-      const float h = gd_sum_strided(part_hpc + (size_t)l * nG * Rp + r, nG, (size_t)Rp);
-      const GdAtom at = atoms[l];
-      const float t = (h - at.hpl0) / at.hpl1;
-      acc[6] += 0.5f * t * t - at.hpl2;
-    }
-    for (int m = wi; m < M; m += W) {  // MCS rows (energy_mcs_v1.C:5-29)
-      const float d = gd_sum_strided(part_mcs + (size_t)m * nL * Rp + r, nL, (size_t)Rp);
-      const float2 row = mcsrow[m];
-      acc[7] += row.x * sqrtf(d / row.y);
-    }
-  }
+  gd_reduce_wave<false>(J, bk.rb + lane, 4 * k + wave, acc);
 #pragma unroll
   for (int c = 0; c < 8; ++c) red[wave][c][lane] = acc[c];
   __syncthreads();
@@ -783,82 +859,90 @@ __global__ __launch_bounds__(256) void gd_reduce_kernel(const GdJob *__restrict_
 }
 
 // ---------------------------------------------------------------------------
-// Finish kernel: 1024 threads = 16 waves per 64-replica block; lanes are
-// replicas.  Sums the reduce kernel's slices, assembles and weights the terms,
-// records, accepts, proposes the next move and transforms the atoms.  Only the
-// acceptance waits for the energies: the next step's increments, this step's
-// accept draw and the rotations of both possible next proposals (from the
-// proposal if it is accepted, from the current pose if not) are computed by
-// waves 1-3 while the slices are summed, and wave 0 only selects.
-#define GD_FW 16
+// Finish of a 64-replica block; lanes are replicas.  Sums the reduce slices,
+// assembles and weights the terms, records, accepts, proposes the next move and
+// transforms the atoms.  Only the acceptance waits for the energies: the next
+// step's increments, this step's accept draw and the rotations of both possible
+// next proposals (from the proposal if it is accepted, from the current pose if
+// not) are made before it by waves 1-3 (gd_finish_pre), and wave 0 only
+// selects.  What the next pair items do not need -- the record, the replica
+// state -- is written last.
 #define GD_FPA 4  // conformer atoms per wave prefetched for the transform
-__global__ __launch_bounds__(1024) void gd_finish_kernel(const GdJob *__restrict__ jobs,
-                                                          const GdBlock *__restrict__ blocks,
-                                                          int mode, int launch_step,
-                                                          const int *__restrict__ step_base,
-                                                          int *__restrict__ wq) {
-  if (wq && blockIdx.x == 0 && threadIdx.x == 0) *wq = 0;  // next pair launch's queue
-  if (step_base) launch_step += *step_base;  // graph replays: base step in device memory
-  __shared__ float red[8][64];
-  __shared__ float xf[2][12][64];  // next transform if this step is accepted [0] / rejected [1]
-  __shared__ float inc_s[6][64];
-  __shared__ float u_s[64];
-  __shared__ int acc_s[64];
-  const GdBlock bk = gd_c(blocks)[blockIdx.x];
-  GdJobC &J = gd_c(jobs)[bk.job];
-  const int lane = threadIdx.x & 63, wave = gd_uniform((int)(threadIdx.x >> 6));
-  const int r = bk.rb + lane;
-  const int Rp = J.Rp;
-  const int step = launch_step - J.step0;  // this job's MC step
-  const bool move = mode != GD_MODE_EVAL;
+struct GdFinLds {
+  float red[8][64];
+  float xf[2][12][64];  // next transform if this step is accepted [0] / rejected [1]
+  float inc_s[6][64];
+  float u_s[64];
+  int acc_s[64];
+};
 
-  // (1) the reduce kernel's slices: wave c < 8 sums value c over the GD_RK
-  // slices in slice order (all loads issued first)
-  if (wave < 8) {
-    const GD_AS_GLOBAL float *fp =
-        gd_g(J.fin_part) + (size_t)(bk.rb / 64) * GD_RK * 8 * 64 + (size_t)wave * 64 + lane;
-    float v[GD_RK];
-#pragma unroll
-    for (int k = 0; k < GD_RK; ++k) v[k] = fp[(size_t)k * 8 * 64];
-    float acc = 0.0f;
-#pragma unroll
-    for (int k = 0; k < GD_RK; ++k) acc += v[k];
-    red[wave][lane] = acc;
-  }
-  // (2) off the acceptance path: wave 1 the next step's increments, wave 2 this
-  // step's accept draw (the initial pass draws u = 0, a forced accept)
-  const uint32_t next = mode == GD_MODE_STEP ? (uint32_t)step + 1u : 0u;
-  if (move && wave == 1) {
-    float inc[6], un;
-    gd_move(J, r, next, inc, &un);
-#pragma unroll
-    for (int i = 0; i < 6; ++i) inc_s[i][lane] = inc[i];
-  }
-  if (move && wave == 2)
-    u_s[lane] = mode == GD_MODE_STEP
-                    ? gd_accept_u01(((uint64_t)J.seed_hi << 32) | J.seed_lo, J.job_id, (uint32_t)r,
-                                    (uint32_t)step)
-                    : 0.0f;
-  // the two possible bases of the next proposal, read before wave 0 writes them
-  float base[6];
-  if (move && (wave == 1 || wave == 3)) {
+// Before the energies (mode != EVAL): waves 1-3 of the group; the caller's next
+// barrier makes the results visible.
+__device__ __forceinline__ void gd_finish_pre(GdJobC &J, const int rb, const int mode, const int step,
+                                              const int lane, const int wave, GdFinLds &sh) {
+  const int r = rb + lane;
+  const int Rp = J.Rp;
+  if (wave == 2)  // the initial pass draws u = 0, a forced accept
+    sh.u_s[lane] = mode == GD_MODE_STEP
+                       ? gd_accept_u01(((uint64_t)J.seed_hi << 32) | J.seed_lo, J.job_id, (uint32_t)r,
+                                       (uint32_t)step)
+                       : 0.0f;
+  if (wave == 1 || wave == 3) {
     const GD_AS_GLOBAL float *src = gd_g(wave == 1 ? J.prop : J.mm);
+    float base[6], inc[6], un;
 #pragma unroll
     for (int i = 0; i < 6; ++i) base[i] = src[(size_t)i * Rp + r];
+    gd_move(J, r, mode == GD_MODE_STEP ? (uint32_t)step + 1u : 0u, inc, &un);
+    if (wave == 1)
+#pragma unroll
+      for (int i = 0; i < 6; ++i) sh.inc_s[i][lane] = inc[i];
+    float m[6], R[9];
+#pragma unroll
+    for (int i = 0; i < 6; ++i) m[i] = inc[i] + base[i];
+    gd_rotation(m, R);
+    const int c = wave == 1 ? 0 : 1;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) sh.xf[c][i][lane] = R[i];
+    sh.xf[c][9][lane] = m[0] + J.center[0];
+    sh.xf[c][10][lane] = m[1] + J.center[1];
+    sh.xf[c][11][lane] = m[2] + J.center[2];
+  }
+}
+
+// The energies, the decision and the next coordinates by FW >= 8 waves; step:
+// the job's MC step.  AG: other groups of the launch wrote the slices and read
+// the coordinates; publish() runs once the coordinates are stored.
+template <bool AG, int FW, class Publish>
+__device__ __forceinline__ void gd_finish_post(GdJobC &J, const int rb, const int mode, const int step,
+                                               const int lane, const int wave, GdFinLds &sh,
+                                               Publish &&publish) {
+  const int r = rb + lane;
+  const int Rp = J.Rp;
+  const bool move = mode != GD_MODE_EVAL;
+
+  // the slices: wave c < 8 sums value c over the GD_RK slices in slice order
+  // (all loads issued first)
+  float v[GD_RK];
+  if (wave < 8) {
+    const GD_AS_GLOBAL float *fp =
+        gd_g(J.fin_part) + (size_t)(rb / 64) * GD_RK * 8 * 64 + (size_t)wave * 64 + lane;
+#pragma unroll
+    for (int k = 0; k < GD_RK; ++k) v[k] = gd_ld<AG>(fp + (size_t)k * 8 * 64);
   }
   // loads that do not wait for the energies, issued now: wave 0's replica
   // state, and every wave's first GD_FPA conformer atoms for the transform
-  const GD_AS_GLOBAL float *prop_c = gd_g(J.prop), *en_c = gd_g(J.en), *mm_c = gd_g(J.mm);
+  GD_AS_GLOBAL float *prop = gd_g(J.prop), *en = gd_g(J.en), *mm = gd_g(J.mm);
+  GD_AS_GLOBAL int *acc_r = gd_g(J.acc);
   float m[6], m0[6], en9 = 0.0f, mbv = 0.0f, best0 = 0.0f;
   int nacc0 = 0;
   if (wave == 0) {
 #pragma unroll
-    for (int i = 0; i < 6; ++i) m[i] = prop_c[(size_t)i * Rp + r];
+    for (int i = 0; i < 6; ++i) m[i] = prop[(size_t)i * Rp + r];
     if (move) {
-      en9 = en_c[(size_t)9 * Rp + r];
+      en9 = en[(size_t)9 * Rp + r];
       mbv = gd_g(J.minus_beta)[gd_g(J.tmpi)[r]];
 #pragma unroll
-      for (int i = 0; i < 6; ++i) m0[i] = mm_c[(size_t)i * Rp + r];
+      for (int i = 0; i < 6; ++i) m0[i] = mm[(size_t)i * Rp + r];
       best0 = gd_g(J.best)[r];
       nacc0 = gd_g(J.nacc)[r];
     }
@@ -868,28 +952,23 @@ __global__ __launch_bounds__(1024) void gd_finish_kernel(const GdJob *__restrict
   float4 pa[GD_FPA];
   if (move)
 #pragma unroll
-    for (int q = 0; q < GD_FPA; ++q) pa[q] = lc[min(wave + q * GD_FW, L - 1)];
+    for (int q = 0; q < GD_FPA; ++q) pa[q] = lc[min(wave + q * FW, L - 1)];
+  if (wave < 8) {
+    float acc = 0.0f;
+#pragma unroll
+    for (int k = 0; k < GD_RK; ++k) acc += v[k];
+    sh.red[wave][lane] = acc;
+  }
   __syncthreads();
 
-  if (move && (wave == 1 || wave == 3)) {  // rotation of each candidate next proposal
-    float m[6], R[9];
-#pragma unroll
-    for (int i = 0; i < 6; ++i) m[i] = inc_s[i][lane] + base[i];
-    gd_rotation(m, R);
-    const int c = wave == 1 ? 0 : 1;
-#pragma unroll
-    for (int i = 0; i < 9; ++i) xf[c][i][lane] = R[i];
-    xf[c][9][lane] = m[0] + J.center[0];
-    xf[c][10][lane] = m[1] + J.center[1];
-    xf[c][11][lane] = m[2] + J.center[2];
-  }
+  const bool live = r < J.R;
+  float e[10], tot = 0.0f;
+  bool a = false;
   if (wave == 0) {
-    GD_AS_GLOBAL float *prop = gd_g(J.prop), *en = gd_g(J.en), *mm = gd_g(J.mm);
     float s[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) s[k] = red[k][lane];
+    for (int k = 0; k < 8; ++k) s[k] = sh.red[k][lane];
     // e_s assembly (kernel_cpp_montecarlo_soa.C:318-324), KDE/MCS/DST (:328-359)
-    float e[10];
     e[0] = s[0];
     e[1] = s[1];
     e[2] = J.pmf_all + s[2];
@@ -916,7 +995,6 @@ __global__ __launch_bounds__(1024) void gd_finish_kernel(const GdJob *__restrict
     // normalisation + weights (:363-374)
 #pragma unroll
     for (int i = 0; i < 7; ++i) e[i] = e[i] * J.inv_L;
-    float tot = 0.0f;
 #pragma unroll
     for (int i = 0; i < 9; ++i) {
       e[i] = J.a_para[i] * e[i] + J.b_para[i];
@@ -924,7 +1002,6 @@ __global__ __launch_bounds__(1024) void gd_finish_kernel(const GdJob *__restrict
     }
     e[9] = tot;
 
-    const bool live = r < J.R;
     if (!move) {
       if (live) {
         GD_AS_GLOBAL float *evt = gd_g(J.ev_terms), *evr = gd_g(J.ev_raw);
@@ -932,61 +1009,304 @@ __global__ __launch_bounds__(1024) void gd_finish_kernel(const GdJob *__restrict
         for (int i = 0; i < 9; ++i) evr[(size_t)r * 9 + i] = raw[i];
       }
     } else {
-      GD_AS_GLOBAL int *acc_r = gd_g(J.acc);
-      // record the pre-move state if the previous step was accepted (:224-231)
-      // into the ring half of this step's dump (dump d = step / rec_cap fills
-      // half d mod 2 while the host copies out the other)
-      if (mode == GD_MODE_STEP && J.record && live && acc_r[r]) {
-        const int half = (step / J.rec_cap) & 1;
-        GD_AS_GLOBAL int *rec_n = gd_g(J.rec_n) + (size_t)half * Rp;
-        const int n = rec_n[r];
-        if (n < J.rec_cap) {
-          GD_AS_GLOBAL float *o =
-              gd_g(J.rec) + (((size_t)half * Rp + r) * J.rec_cap + n) * GD_REC_W;
-          o[0] = (float)step;
-          for (int i = 0; i < 6; ++i) o[1 + i] = mm[(size_t)i * Rp + r];
-          for (int i = 0; i < 10; ++i) o[7 + i] = en[(size_t)i * Rp + r];
-          rec_n[r] = n + 1;
-        }
-      }
       // Metropolis (:382-392); the initial pass draws u = 0
-      const float u = u_s[lane];
+      const float u = sh.u_s[lane];
       const float x = (tot - en9) * mbv;
-      const bool a = (u == 0.0f) ? (x >= GD_EXP_UNDERFLOW) : (u < expf(x));
-      acc_s[lane] = live && a;  // padding lanes keep their pose
-      if (live) {
-        acc_r[r] = a;
-        if (a) {
-          for (int i = 0; i < 10; ++i) en[(size_t)i * Rp + r] = e[i];
-          for (int i = 0; i < 6; ++i) mm[(size_t)i * Rp + r] = m[i];
-          if (mode == GD_MODE_STEP) gd_g(J.nacc)[r] = nacc0 + 1;
-          gd_g(J.best)[r] = fminf(best0, tot);
-        }
-      }
-      // the next step's proposal, from the accepted pose (padding lanes keep
-      // theirs: they never accept)
-      const bool took = live && a;
-#pragma unroll
-      for (int i = 0; i < 6; ++i) prop[(size_t)i * Rp + r] = inc_s[i][lane] + (took ? m[i] : m0[i]);
+      a = live && ((u == 0.0f) ? (x >= GD_EXP_UNDERFLOW) : (u < expf(x)));
+      sh.acc_s[lane] = a;  // padding lanes keep their pose
     }
   }
   if (!move) return;
   __syncthreads();
-  const int c = acc_s[lane] ? 0 : 1;
-  float R[9], t[3];
+  {
+    const int c = sh.acc_s[lane] ? 0 : 1;
+    float R[9], t[3];
 #pragma unroll
-  for (int i = 0; i < 9; ++i) R[i] = xf[c][i][lane];
-  t[0] = xf[c][9][lane];
-  t[1] = xf[c][10][lane];
-  t[2] = xf[c][11][lane];
-  // the transform of gd_transform_atoms, the first atoms from the prefetch
-  GD_AS_GLOBAL float *co = gd_g(J.coords);
-  auto put = [&](int l, const float4 a) { gd_put_atom(co, Rp, r, l, R, t, a); };
+    for (int i = 0; i < 9; ++i) R[i] = sh.xf[c][i][lane];
+    t[0] = sh.xf[c][9][lane];
+    t[1] = sh.xf[c][10][lane];
+    t[2] = sh.xf[c][11][lane];
+    // the transform of gd_transform_atoms, the first atoms from the prefetch
+    GD_AS_GLOBAL float *co = gd_g(J.coords);
+    auto put = [&](int l, const float4 q) { gd_put_atom<AG>(co, Rp, r, l, R, t, q); };
 #pragma unroll
-  for (int q = 0; q < GD_FPA; ++q)
-    if (wave + q * GD_FW < L) put(wave + q * GD_FW, pa[q]);
-  for (int l = wave + GD_FPA * GD_FW; l < L; l += GD_FW) put(l, lc[l]);
+    for (int q = 0; q < GD_FPA; ++q)
+      if (wave + q * FW < L) put(wave + q * FW, pa[q]);
+    for (int l = wave + GD_FPA * FW; l < L; l += FW) put(l, lc[l]);
+  }
+  publish();
+  if (wave == 0) {
+    // record the pre-move state if the previous step was accepted (:224-231)
+    // into the ring half of this step's dump (dump d = step / rec_cap fills
+    // half d mod 2 while the host copies out the other)
+    if (mode == GD_MODE_STEP && J.record && live && acc_r[r]) {
+      const int half = (step / J.rec_cap) & 1;
+      GD_AS_GLOBAL int *rec_n = gd_g(J.rec_n) + (size_t)half * Rp;
+      const int n = rec_n[r];
+      if (n < J.rec_cap) {
+        GD_AS_GLOBAL float *o = gd_g(J.rec) + (((size_t)half * Rp + r) * J.rec_cap + n) * GD_REC_W;
+        o[0] = (float)step;
+        for (int i = 0; i < 6; ++i) o[1 + i] = mm[(size_t)i * Rp + r];
+        for (int i = 0; i < 10; ++i) o[7 + i] = en[(size_t)i * Rp + r];
+        rec_n[r] = n + 1;
+      }
+    }
+    if (live) {
+      acc_r[r] = a;
+      if (a) {
+        for (int i = 0; i < 10; ++i) en[(size_t)i * Rp + r] = e[i];
+        for (int i = 0; i < 6; ++i) mm[(size_t)i * Rp + r] = m[i];
+        if (mode == GD_MODE_STEP) gd_g(J.nacc)[r] = nacc0 + 1;
+        gd_g(J.best)[r] = fminf(best0, tot);
+      }
+    }
+    // the next step's proposal, from the accepted pose (padding lanes keep
+    // theirs: they never accept)
+#pragma unroll
+    for (int i = 0; i < 6; ++i) prop[(size_t)i * Rp + r] = sh.inc_s[i][lane] + (a ? m[i] : m0[i]);
+  }
 }
+
+// Finish kernel: one 16-wave group per block.
+#define GD_FW 16
+__global__ __launch_bounds__(64 * GD_FW) void gd_finish_kernel(const GdJob *__restrict__ jobs,
+                                                               const GdBlock *__restrict__ blocks,
+                                                               int mode, int launch_step,
+                                                               const int *__restrict__ step_base,
+                                                               int *__restrict__ wq) {
+  if (wq && blockIdx.x == 0 && threadIdx.x == 0) *wq = 0;  // next pair launch's queue
+  if (step_base) launch_step += *step_base;  // graph replays: base step in device memory
+  __shared__ GdFinLds sh;
+  const GdBlock bk = gd_c(blocks)[blockIdx.x];
+  GdJobC &J = gd_c(jobs)[bk.job];
+  const int lane = threadIdx.x & 63, wave = gd_uniform((int)(threadIdx.x >> 6));
+  const int step = launch_step - J.step0;  // this job's MC step
+  if (mode != GD_MODE_EVAL) gd_finish_pre(J, bk.rb, mode, step, lane, wave, sh);
+  gd_finish_post<false, GD_FW>(J, bk.rb, mode, step, lane, wave, sh, [] {});
+}
+
+// ---------------------------------------------------------------------------
+// Stepping kernel: n_steps MC steps of every replica block of a job list in one
+// launch.  Blocks of 64 replicas do not depend on each other between exchange
+// points, so a block's next step starts as soon as its own last one is
+// finished; nothing waits for the slowest block, and no step pays for launches.
+//
+// The first groups are the blocks' finishers, teams of `team` groups: a team waits
+// for its block's items, each of its groups reduces its share of the slices, and
+// the first runs the finish and queues the block's next step.  Finishers stay for
+// the whole launch, with their code and their blocks: the group that completed a
+// block's last item would have to fetch the finish's instructions first (7 us of
+// finish against 3.5).
+//
+// Every other group is a worker for one pair item.  It takes a ticket, and ticket
+// t is an item of queue entry t / per_entry: an entry is up to per_entry pair
+// items of a block whose coordinates are ready, and entries are in the order in
+// which the blocks became ready, so a worker waits only when no block is.
+// Workers do not stay for a second item: a SIMD issues from its oldest waves
+// first, so that of resident groups the youngest always came last, took three
+// times as long, and held up its block (1,760 replicas, 40 atoms, 3,000 points:
+// 126 us a step, against 106 with a new group for each item, which ages as its
+// item does).
+//
+// A worker waits for an entry that some block's finish will write: the blocks
+// whose items are not all done are held by groups that run.  Finishers have the
+// lowest group numbers, so they run whenever a worker does.  Each wait is bounded
+// in time all the same and ends the launch with `failed` set, for what this
+// launch does not control: launches beside it that hold the slots.
+//
+// What the groups hand each other (coordinates, partial sums, slices) is read
+// and written at agent scope.  The counters run on from launch to launch; the
+// arguments hold the steps taken before this one.
+#define GD_SYNC_LINE 32  // words between two words that different groups poll
+// Wait until done(*p) (thread 0 of a group); false: out of time, or another group
+// ran out of it.
+template <class T, class Done>
+__device__ __forceinline__ bool gd_wait_for(const GD_AS_GLOBAL T *p, Done &&done, GD_AS_GLOBAL unsigned *failed,
+                                            const long long ticks) {
+  if (done(gd_ld<true>(p))) return true;
+  const long long t0 = wall_clock64();
+  for (unsigned k = 1;; ++k) {
+    __builtin_amdgcn_s_sleep(1);
+    if (done(gd_ld<true>(p))) return true;
+    if ((k & 63) == 0) {
+      if (gd_ld<true>((const GD_AS_GLOBAL unsigned *)failed)) return false;
+      if (wall_clock64() - t0 > ticks) {
+        gd_st<true>(failed, 1u);
+        return false;
+      }
+    }
+  }
+}
+
+template <int LC>
+union GdChainLds {
+  float pair[GD_GROUP][GD_NLIN + LC][64];
+  struct {
+    float red[GD_GROUP][8][64];
+    GdFinLds fin;
+    int ok;
+  };
+};
+
+typedef const GD_AS_CONST GdChain GdChainC;
+
+// The counters of block b of the launch's list.
+__device__ __forceinline__ GD_AS_GLOBAL unsigned *gd_block_sync(GdChainC &c, int b) {
+  return gd_g(c.sync) + GD_SY_HEAD + (size_t)b * GD_SY_BLOCK;
+}
+
+// Block b's next items may run: its queue entries, written by one wave.
+__device__ __forceinline__ void gd_chain_push(GdChainC &c, const int b) {
+  const int lane = gd_lane_id();
+  const int n = (gd_c(c.blocks)[b].n_items + c.per_entry - 1) / c.per_entry;
+  unsigned at = 0;
+  if (lane == 0)
+    at = __hip_atomic_fetch_add(gd_g(c.sync) + GD_SY_TAIL, (unsigned)n, __ATOMIC_RELAXED,
+                                __HIP_MEMORY_SCOPE_AGENT) -
+         c.steps_before * (unsigned)c.n_entries;
+  at = (unsigned)gd_uniform((int)at);
+  if (at + (unsigned)n > (unsigned)(c.n_entries * c.n_steps)) return;  // after a launch that failed
+  for (int k = lane; k < n; k += 64)
+    gd_st<true>(gd_g(c.queue) + (size_t)(at + k) * c.stride,
+                (unsigned long long)c.epoch << 32 | (unsigned)(b << 8 | k));
+}
+
+// Not inlined: its registers are its own, and the pair loop's allocation is
+// what it is without it.  lds: the group's GdChainLds.
+template <int LC>
+__device__ __attribute__((noinline)) void gd_chain_finisher(GdChainC *cp, const int wave_in,
+                                                            GD_AS_LDS GdChainLds<LC> *lds) {
+  const unsigned long long cq = (unsigned long long)cp;  // uniform, but passed in vector registers
+  GdChainC &c0 = *(GdChainC *)((unsigned long long)(unsigned)gd_uniform((int)(cq >> 32)) << 32 |
+                               (unsigned)gd_uniform((int)cq));
+  const int wave0 = gd_uniform(wave_in);
+  asm volatile("s_setprio 3");  // before the pair waves of the SIMD
+  GdChainLds<LC> &sh = *(GdChainLds<LC> *)lds;
+  int &s_ok = sh.ok;
+  const int F = c0.team, team = gd_uniform((int)blockIdx.x / F), f = (int)blockIdx.x - team * F;
+  if (f == 0 && wave0 == 1)  // every block is ready for the first step
+    for (int b = team; b < c0.n_blocks; b += c0.n_teams) gd_chain_push(c0, b);
+  int s = 0, b = team;
+  for (;;) {
+    // read and derived again for each block (see the kernel)
+    GdChainC &c = gd_reread(c0);
+    if (b >= c.n_blocks) {
+      b = team;
+      ++s;
+    }
+    if (s >= c.n_steps) return;
+    int wave = wave0;
+    asm volatile("" : "+s"(wave));
+    const int lane = gd_lane_id();
+    const bool first = wave == 0 && lane == 0;
+    GD_AS_GLOBAL unsigned *failed = gd_g(c.sync) + GD_SY_FAILED;
+    const int blk = b;
+    const GdChainBlock bk = gd_c(c.blocks)[blk];
+    GdJobC &J = gd_c(c.jobs)[bk.job];
+    GD_AS_GLOBAL unsigned *sb = gd_block_sync(c, blk);
+    b += c.n_teams;
+    const int mode = c.init && s == 0 ? GD_MODE_INIT : GD_MODE_STEP;
+    const int step = c.step0 + s - c.init - J.step0;
+    if (f == 0) gd_finish_pre(J, bk.rb, mode, step, lane, wave, sh.fin);
+    if (first) {
+      const unsigned want = (unsigned)bk.n_items * (c.steps_before + (unsigned)s + 1u);
+      s_ok = gd_wait_for(sb, [&](unsigned v) { return v == want; }, failed, c.wait_ticks);
+    }
+    __syncthreads();
+    if (!gd_uniform(s_ok)) return;
+    // two slices at a time: waves 0-3 and 4-7
+    for (int k = f; k < GD_RT; k += F) {
+      float acc[8];
+      gd_reduce_wave<true>(J, bk.rb + lane, GD_GROUP * k + wave, acc);
+#pragma unroll
+      for (int q = 0; q < 8; ++q) sh.red[wave][q][lane] = acc[q];
+      __syncthreads();
+      const int h = wave >> 2;  // wave w: values 2 (w mod 4) and the next of slice 2 k + w / 4
+      GD_AS_GLOBAL float *fp = gd_g(J.fin_part) + ((size_t)(bk.rb / 64) * GD_RK + 2 * k + h) * 8 * 64;
+#pragma unroll
+      for (int q = 2 * (wave & 3); q < 2 * (wave & 3) + 2; ++q)
+        gd_st<true>(fp + q * 64 + lane,
+                    ((sh.red[4 * h][q][lane] + sh.red[4 * h + 1][q][lane]) + sh.red[4 * h + 2][q][lane]) +
+                        sh.red[4 * h + 3][q][lane]);
+      __syncthreads();  // red is reused
+    }
+    gd_drain();
+    __syncthreads();
+    if (first && F > 1)
+      __hip_atomic_fetch_add(sb + GD_SYNC_LINE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (f != 0) continue;
+    if (F > 1) {
+      if (first) {
+        const unsigned want = (unsigned)F * (c.steps_before + (unsigned)s + 1u);
+        s_ok = gd_wait_for(sb + GD_SYNC_LINE, [&](unsigned v) { return v == want; }, failed, c.wait_ticks);
+      }
+      __syncthreads();
+      if (!gd_uniform(s_ok)) return;
+    }
+    const bool more = s + 1 < c.n_steps;
+    gd_finish_post<true, GD_GROUP>(J, bk.rb, mode, step, lane, wave, sh.fin, [&] {
+      gd_drain();
+      __syncthreads();
+      if (wave == 1 && more) gd_chain_push(c, blk);
+    });
+    __syncthreads();
+    }
+}
+
+template <int LC>
+__global__ __launch_bounds__(64 * GD_GROUP) __attribute__((amdgpu_waves_per_eu(8))) void gd_chain_kernel(
+    const GdChain chain) {
+  __shared__ GdChainLds<LC> sh;
+  __shared__ int s_blk, s_item;
+  (void)chain;
+  // the arguments are read from the kernarg segment where they are needed: held
+  // across the pair loop they would take scalar registers from it
+  auto args = [&]() -> GdChainC & {
+    unsigned long long q = (unsigned long long)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(q));
+    return *(GdChainC *)q;
+  };
+  const int wave = gd_uniform((int)(threadIdx.x >> 6));
+  if (gd_uniform((int)blockIdx.x) < args().n_teams * args().team) {
+    gd_chain_finisher<LC>(&args(), wave, (GD_AS_LDS GdChainLds<LC> *)&sh);
+    return;
+  }
+  if (threadIdx.x == 0) {
+    GdChainC &c = args();
+    const unsigned t = __hip_atomic_fetch_add(gd_g(c.sync) + GD_SY_TICKET, 1u, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT) -
+                       c.steps_before * (unsigned)(c.n_entries * c.per_entry);
+    // the ticket's queue entry: a block and which per_entry of its items (past
+    // the queue only after a launch that failed)
+    const unsigned e = t / (unsigned)c.per_entry, epoch = c.epoch;
+    const GD_AS_GLOBAL unsigned long long *q = gd_g(c.queue) + (size_t)e * c.stride;
+    s_blk = -1;
+    if (e < (unsigned)(c.n_entries * c.n_steps) &&
+        gd_wait_for(q, [&](unsigned long long v) { return (unsigned)(v >> 32) == epoch; },
+                    gd_g(c.sync) + GD_SY_FAILED, c.wait_ticks)) {
+      const unsigned v = (unsigned)gd_ld<true>(q);
+      s_blk = (int)(v >> 8);
+      s_item = (int)((v & 255u) * (unsigned)c.per_entry + (t - e * (unsigned)c.per_entry));
+    }
+  }
+  __syncthreads();
+  const int blk = gd_uniform(s_blk), k = gd_uniform(s_item);
+  if (blk < 0) return;
+  {
+    GdChainC &c = args();
+    const GdChainBlock bk = gd_c(c.blocks)[blk];
+    if (k >= bk.n_items) return;  // a block's last entry may name items past its last
+    GdItem it = gd_c(c.items)[bk.item0 + k];
+    it.rb = bk.rb;
+    gd_pair_item<LC, true>(c.jobs, it, threadIdx.x & 63, wave, sh.pair);
+  }
+  gd_drain();
+  __syncthreads();
+  if (gd_lane_id() == 0 && wave == 0)
+    __hip_atomic_fetch_add(gd_block_sync(args(), gd_uniform(s_blk)), 1u, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+}
+template __global__ void gd_chain_kernel<4>(const GdChain);
 
 // ---------------------------------------------------------------------------
 // Temperature exchange: one workgroup per (job, round) entry, threads over

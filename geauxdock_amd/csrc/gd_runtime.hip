@@ -12,6 +12,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <limits>
@@ -33,6 +34,8 @@ __global__ void gd_pair_kernel(const GdJob *, const GdItem *, int);
 __global__ void gd_transform_kernel(const GdJob *, const GdBlock *, int *);
 __global__ void gd_reduce_kernel(const GdJob *, const GdBlock *);
 __global__ void gd_finish_kernel(const GdJob *, const GdBlock *, int, int, const int *, int *);
+template <int LC>
+__global__ void gd_chain_kernel(const GdChain);
 __global__ void gd_exchange_kernel(const GdJob *, const GdExch *);
 __global__ void gd_move_draws_kernel(uint64_t, uint32_t, int, GdScale6, int, uint32_t, int, float *);
 __global__ void gd_clock_kernel(long long, float, long long *, float *);
@@ -46,6 +49,7 @@ namespace gdr {
 static thread_local std::string g_err;
 static int g_device = -1;
 static int g_cu = 0;
+static int g_wall_khz = 100000;  // rate of the constant-rate counter
 static std::mutex g_mu;
 
 void set_error(const std::string &s) { g_err = s; }
@@ -779,6 +783,45 @@ gd_status reset_replicas(gd_job *j) {
   return e == hipSuccess ? GD_OK : hip_fail(e, "hipStreamSynchronize");
 }
 
+// The stepping kernel's lists, made at the first run that steps by it and given
+// back with the job's other lists.
+static void chain_drop(gd_job *j) {
+  if (j->d_chain) hipFree(j->d_chain);
+  j->d_chain = nullptr;
+  j->chain_bytes = 0;
+}
+
+static gd_status chain_make(gd_job *j) {
+  if (j->d_chain) return GD_OK;
+  ChainList &cl = j->chain;
+  std::vector<GdItem> items;
+  for (const GdItem &it : j->items)
+    if (it.rb == 0) items.push_back(it);
+  std::vector<GdChainBlock> blocks;
+  for (int rb = 0; rb < j->h.Rp; rb += 64) blocks.push_back({0, rb, 0, (int)items.size()});
+  auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+  const size_t bi = items.size() * sizeof(GdItem), bb = blocks.size() * sizeof(GdChainBlock),
+               bs = chain_sync_bytes(cl.n_blocks), bq = cl.queue_bytes();
+  const size_t all = up(bi) + up(bb) + up(bs) + up(bq);
+  hipError_t e = hipMalloc(&j->d_chain, all);
+  if (e != hipSuccess) return hip_fail(e, "hipMalloc stepping lists");
+  j->chain_bytes = all;
+  char *base = (char *)j->d_chain;
+  cl.d_items = (GdItem *)base;
+  cl.d_blocks = (GdChainBlock *)(base + up(bi));
+  cl.d_sync = (unsigned *)(base + up(bi) + up(bb));
+  cl.d_queue = (unsigned long long *)(base + up(bi) + up(bb) + up(bs));
+  cl.epoch = cl.steps = 0;
+  if ((e = hipMemcpyAsync(base, items.data(), bi, hipMemcpyHostToDevice, j->stream)) != hipSuccess ||
+      (e = hipMemcpyAsync(base + up(bi), blocks.data(), bb, hipMemcpyHostToDevice, j->stream)) != hipSuccess ||
+      (e = hipMemsetAsync(cl.d_sync, 0, up(bs) + up(bq), j->stream)) != hipSuccess ||
+      (e = hipStreamSynchronize(j->stream)) != hipSuccess) {
+    chain_drop(j);
+    return hip_fail(e, "stepping list upload");
+  }
+  return GD_OK;
+}
+
 gd_status sync_job_struct(gd_job *j) {
   hipError_t e = hipMemcpyAsync(j->d_job, &j->h, sizeof(GdJob), hipMemcpyHostToDevice, j->stream);
   if (e != hipSuccess) return hip_fail(e, "hipMemcpyAsync job");
@@ -803,6 +846,7 @@ gd_status sync_job_struct(gd_job *j) {
         ++j->n_items_part[k];
       }
   }
+  chain_drop(j);
   if (j->d_lists) hipFree(j->d_lists);
   j->d_lists = nullptr;
   auto up = [](size_t b) { return (b + 255) / 256 * 256; };
@@ -873,6 +917,93 @@ gd_status launch_exchange(const GdJob *d_jobs, const GdExch *d_ex, int n_ex, hip
   hipLaunchKernelGGL(gd_exchange_kernel, dim3(n_ex), dim3(256), 0, s, d_jobs, d_ex);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? GD_OK : hip_fail(e, "exchange kernel launch");
+}
+
+// ---- stepping kernel ----------------------------------------------------------
+size_t chain_sync_bytes(int n_blocks) {
+  return (GD_SY_HEAD + (size_t)n_blocks * GD_SY_BLOCK) * sizeof(unsigned);
+}
+
+// Finishers: a block's reduction is a chain of latencies, which a team of groups
+// shortens: 8 groups for two blocks, 4 where there are few blocks or a step's items
+// leave slots free (220 replicas, 46 atoms, 4,001 points: 39.0 us a step, with 1
+// group 54.8, with 8 42.2; 1,760 replicas, 24 atoms, 1,200 points: 39.5, with 1
+// 49.2), then one, whose time the other blocks' items cover (1,760 replicas, 40
+// atoms, 3,000 points: 104.8 us, with 4 groups 108.2).  At most 64 finishers, each
+// then with several blocks.
+// Groups of a CU: where the items of a step are fewer than the slots, added LDS
+// keeps a CU from taking four groups while others have none, and keeps groups
+// that only wait from being resident: 128 replicas, 40 atoms, 9,000 points (400
+// items): 50.2 us a step with one group to a CU, 62.9 with four; 440 replicas, 20
+// atoms, 9,000 points (420): 65.9 with two, 70.4 with four.
+// Queue entries: blocks of one job are eight entries each, on lines of their own
+// where there are few blocks (waiting workers then poll different lines); in
+// longer lists an entry is 8 items.  The queue holds up to 1 MB of them.
+void ChainList::shape(const std::vector<const GdJob *> &jobs) {
+  n_blocks = n_items = n_entries = 0;
+  step_pairs = 0.0;
+  int most = 1;
+  for (const GdJob *g : jobs) {
+    n_blocks += g->Rp / 64;
+    n_items += g->Rp / 64 * g->nL * g->nG;
+    step_pairs += (double)g->Rp * g->L * g->P;
+    most = std::max(most, g->nL * g->nG);
+  }
+  per_entry = std::max(jobs.size() == 1 ? (most + 7) / 8 : 8, (most + 255) / 256);
+  for (const GdJob *g : jobs) n_entries += g->Rp / 64 * ((g->nL * g->nG + per_entry - 1) / per_entry);
+  stride = n_blocks <= 8 ? 16 : 1;
+  cap_steps = (int)std::max(2.0, std::min(1024.0, (double)(1 << 17) / ((double)n_entries * stride)));
+  n_teams = std::min(n_blocks, 64);
+  const int cu = g_cu > 0 ? g_cu : 256;
+  team = n_blocks <= 2 ? 8 : n_blocks <= 8 || n_items <= 6 * cu ? 4 : 1;
+  const int groups = n_items + 2 * n_teams * team;
+  lds = groups <= 7 * cu / 4 ? 60 << 10 : groups <= 4 * cu ? 28 << 10 : groups <= 6 * cu ? 14 << 10 : 0;
+}
+
+// One launch stays under about a second and 2^22 groups (2^32 work items is the
+// most): jobs whose single step is a sizeable part of that (10^11 pairs, 50 ms)
+// gain nothing from it and are stepped by launches.  So are jobs of one block,
+// where a step is one chain of latencies and the launches are the shorter one
+// (25 replicas, 24 atoms, 1,200 points: 19.9 us a step against 21.6; 40 atoms,
+// 3,000 points: 25.8 against 29.2), and of two blocks with many items, which the
+// 8 finishers of a block read more slowly than the reduce launch's 16 groups (105
+// replicas, 80 atoms, 9,000 points, 2,840 items: 91 against 111; with 1,480: 82
+// by launches, 76 here).
+int chain_max_steps(const ChainList &c) {
+  if (c.n_blocks < 2 || (c.n_blocks == 2 && c.n_items > 2048) || c.step_pairs > 1e11) return 0;
+  const double by_time = 1e12 / std::max(1.0, c.step_pairs);
+  const double by_count = (double)(1 << 22) / ((double)c.n_entries * c.per_entry);
+  const int n = (int)std::min({(double)c.cap_steps, by_time, by_count});
+  return n >= 2 ? n : 0;  // the first launch takes the initial pass and a step
+}
+
+gd_status launch_chain(ChainList &c, const GdJob *d_jobs, int step0, int n_steps, bool init,
+                       hipStream_t s) {
+  if (n_steps <= 0) return GD_OK;
+  GdChain a;
+  a.jobs = d_jobs;
+  a.items = c.d_items;
+  a.blocks = c.d_blocks;
+  a.sync = c.d_sync;
+  a.queue = c.d_queue;
+  a.stride = c.stride;
+  a.per_entry = c.per_entry;
+  a.epoch = ++c.epoch;
+  a.n_entries = c.n_entries;
+  a.steps_before = c.steps;
+  c.steps += (unsigned)n_steps;
+  a.n_teams = c.n_teams;
+  a.team = c.team;
+  a.n_steps = n_steps;
+  a.step0 = step0;
+  a.init = init ? 1 : 0;
+  a.n_blocks = c.n_blocks;
+  a.wait_ticks = (long long)(c.wait_s * 1e3 * g_wall_khz);
+  // the finishers, then a worker group for each item of every step
+  const int grid = c.n_teams * c.team + c.n_entries * c.per_entry * n_steps;
+  hipLaunchKernelGGL(gd_chain_kernel<4>, dim3(grid), dim3(64 * GD_GROUP), c.lds, s, a);
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? GD_OK : hip_fail(e, "stepping kernel launch");
 }
 
 gd_status launch_swap(int axis, const GdJob *d_jobs, const GdBlock *d_blocks, int n_blocks,
@@ -972,6 +1103,9 @@ gd_status gd_init(int dev) {
   if ((e = hipSetDevice(dev)) != hipSuccess) return hip_fail(e, "hipSetDevice");
   g_device = dev;
   g_cu = prop.multiProcessorCount;
+  int khz = 0;
+  if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) == hipSuccess && khz > 0)
+    g_wall_khz = khz;
   return GD_OK;
 }
 
@@ -1048,6 +1182,7 @@ gd_status gd_job_destroy(gd_job *j) {
   if (j->d_part) hipFree(j->d_part);
   if (j->d_job) hipFree(j->d_job);
   if (j->d_lists) hipFree(j->d_lists);
+  gdr::chain_drop(j);
   if (j->d_rec) hipFree(j->d_rec);
   if (j->h_rec) hipHostFree(j->h_rec);
   if (j->copy_stream) hipStreamDestroy(j->copy_stream);
@@ -1074,7 +1209,7 @@ size_t gd_job_footprint(const gd_job_desc *d) { return footprint(d, false); }
 // lists, the record ring (when a run recorded) and the device job struct.
 size_t gd_job_device_bytes(const gd_job *j) {
   if (!j) return 0;
-  return j->bytes + j->part_bytes + j->lists_bytes + j->rec_bytes + sizeof(GdJob);
+  return j->bytes + j->part_bytes + j->lists_bytes + j->chain_bytes + j->rec_bytes + sizeof(GdJob);
 }
 
 gd_status gd_tiling_get(const gd_job *j, gd_tiling *t) {
@@ -1085,8 +1220,15 @@ gd_status gd_tiling_get(const gd_job *j, gd_tiling *t) {
   return GD_OK;
 }
 
+gd_status gd_job_set_step_wait(gd_job *j, double seconds) {
+  if (!j || !(seconds >= 0.0) || seconds > 60.0) return GD_ERR_ARG;
+  j->chain.wait_s = seconds;
+  return GD_OK;
+}
+
 gd_status gd_job_set_streams(gd_job *j, int n_streams) {
   if (!j || n_streams < 1 || n_streams > gd_job::kMaxParts) return GD_ERR_ARG;
+  j->by_launches = true;
   if (n_streams == j->n_streams) return GD_OK;
   const gd_status st = ensure_device();
   if (st != GD_OK) return st;
@@ -1197,8 +1339,11 @@ struct RecSink {
 // reference's cudaMemcpy after each dump (backend_gpu.cu:110-116), or on the
 // copy stream while the device runs dump k + 1, handed to the sink once
 // copied; dump k + 2 reuses the half only after the host has taken it.
-static gd_status dock_impl(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
-                           gd_replica_out *out, gd_stats *stats) {
+// chain: the stepping kernel may be used.  *again: one of its waits ran out of
+// time, nothing was handed over of this dump or later ones (*handed dumps were,
+// or had been before), and the run is to be repeated without it.
+static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
+                          gd_replica_out *out, gd_stats *stats, const bool chain, int *handed, bool *again) {
   if (!j || !mc || mc->steps_total < 0 || mc->steps_per_exchange < 0) return GD_ERR_ARG;
   gd_status st = ensure_device();
   if (st != GD_OK) return st;
@@ -1229,9 +1374,10 @@ static gd_status dock_impl(gd_job *j, const gd_mc_param *mc, const RecSink *sink
   // host side of a streamed run: pinned halves (records, then counts) and the copy stream
   float *h_half[2] = {nullptr, nullptr};
   int *h_cnt[2] = {nullptr, nullptr};
+  unsigned *h_fail[2] = {nullptr, nullptr};
   hipEvent_t ev_done[2] = {nullptr, nullptr}, ev_copied[2] = {nullptr, nullptr};
   if (sink) {
-    const size_t hb = 2 * (half_floats * sizeof(float) + (size_t)g.Rp * sizeof(int));
+    const size_t hb = 2 * (half_floats * sizeof(float) + (size_t)g.Rp * sizeof(int) + sizeof(unsigned));
     if (hb > j->h_rec_bytes) {
       if (j->h_rec) hipHostFree(j->h_rec);
       j->h_rec = nullptr;
@@ -1243,6 +1389,7 @@ static gd_status dock_impl(gd_job *j, const gd_mc_param *mc, const RecSink *sink
     for (int b = 0; b < 2; ++b) {
       h_half[b] = (float *)j->h_rec + b * half_floats;
       h_cnt[b] = (int *)((float *)j->h_rec + 2 * half_floats) + (size_t)b * g.Rp;
+      h_fail[b] = (unsigned *)((float *)j->h_rec + 2 * half_floats) + 2 * (size_t)g.Rp + b;
     }
     if (!sink->blocking) {
       hipError_t e = hipSuccess;
@@ -1303,10 +1450,29 @@ static gd_status dock_impl(gd_job *j, const gd_mc_param *mc, const RecSink *sink
   const std::function<gd_status()> pair = [&]() {
     return launch_pair(g.lc, j->d_job, j->d_items, j->n_items, s);
   };
-  // hand dump k (ring half b, copied to the host) to the sink
+  // the stepping kernel takes the steps between exchange points and dump ends
+  // in one launch; a job whose streams were set, or with wide ligand chunks, is
+  // stepped by launches
+  int chain_max = 0;
+  if (chain && !j->by_launches && g.lc == 4) {
+    j->chain.shape({&g});
+    chain_max = chain_max_steps(j->chain);
+    if (chain_max > 0 && chain_make(j) != GD_OK) {  // no memory for its lists
+      (void)hipGetLastError();
+      chain_max = 0;
+    }
+  }
+  // hand dump k (ring half b, copied to the host) to the sink, each dump once;
+  // false: the stepping kernel failed in it or before
   const auto deliver = [&](int k, int b) {
-    sink->fn(sink->user, k, k * spd, g.R, spd, h_half[b], h_cnt[b]);
+    if (chain_max > 0 && *h_fail[b]) return false;
+    if (k >= *handed) {
+      sink->fn(sink->user, k, k * spd, g.R, spd, h_half[b], h_cnt[b]);
+      *handed = k + 1;
+    }
+    return true;
   };
+  const unsigned *d_fail = j->chain.d_sync + GD_SY_FAILED;
   KTimer tp;
   SpanTimer tspan;
   const bool timing = stats != nullptr;
@@ -1315,7 +1481,7 @@ static gd_status dock_impl(gd_job *j, const gd_mc_param *mc, const RecSink *sink
   // parts' pair work.  Between exchange points the parts share nothing; they
   // join for every exchange point (which spans the whole job) and at dump ends.
   const int np = j->n_parts;
-  bool multi = np >= 2;
+  bool multi = chain_max == 0 && np >= 2;
   for (int k = 0; k < np; ++k) multi = multi && j->nb_part[k] > 0;
   hipStream_t ps[gd_job::kMaxParts] = {s};
   hipEvent_t ev_fork = nullptr, ev_join[gd_job::kMaxParts] = {};
@@ -1359,10 +1525,15 @@ static gd_status dock_impl(gd_job *j, const gd_mc_param *mc, const RecSink *sink
   const auto t0 = std::chrono::steady_clock::now();
   // initial energies (MonteCarlo_d with s2max = 1)
   if (st == GD_OK) st = launch_transform(j->d_job, j->d_blocks, j->n_blocks, s);
-  if (st == GD_OK) st = launch_pair(g.lc, j->d_job, j->d_items, j->n_items, s);
-  if (st == GD_OK) st = launch_finish(j->d_job, j->d_blocks, j->n_blocks, GD_MODE_INIT, 0, s);
+  if (chain_max > 0) {
+    if (st == GD_OK && mc->steps_total == 0) st = launch_chain(j->chain, j->d_job, 0, 1, true, s);
+  } else {
+    if (st == GD_OK) st = launch_pair(g.lc, j->d_job, j->d_items, j->n_items, s);
+    if (st == GD_OK) st = launch_finish(j->d_job, j->d_blocks, j->n_blocks, GD_MODE_INIT, 0, s);
+  }
   if (st == GD_OK && multi && timing) st = tspan.mark_ref(s);
   int pending = -1;  // streamed dump whose copy is in flight
+  int chain_steps = 0;  // MC steps (and initial pass) taken by the stepping kernel
   for (int s1 = 0, k = 0; s1 < mc->steps_total && st == GD_OK; s1 += spd, ++k) {
     const int b = k & 1;
     if (record) {
@@ -1376,7 +1547,18 @@ static gd_status dock_impl(gd_job *j, const gd_mc_param *mc, const RecSink *sink
     const int s_end = std::min(mc->steps_total, s1 + spd);
     for (int step = s1; step < s_end; ++step) {
       const bool timed = timing && step % kTimedEvery == 0;
-      if (multi) {
+      if (chain_max > 0) {
+        // up to the next exchange point or the dump's end; the initial pass
+        // goes with the first steps
+        const bool init = step == 0;
+        int n = std::min(s_end - step, chain_max - (init ? 1 : 0));
+        if (n_rounds > 0) n = std::min(n, spe - step % spe);
+        if (timing && (st = tp.begin(s)) != GD_OK) break;
+        if ((st = launch_chain(j->chain, j->d_job, step, n + (init ? 1 : 0), init, s)) != GD_OK) break;
+        if (timing && (st = tp.end(s)) != GD_OK) break;
+        step += n - 1;
+        chain_steps += n + (init ? 1 : 0);
+      } else if (multi) {
         for (int k = 0; k < np && st == GD_OK; ++k) {
           if (timed && (st = tspan.record(ps[k])) != GD_OK) break;
           if ((st = launch_pair(g.lc, j->d_job, j->d_items_part[k], j->n_items_part[k], ps[k])) != GD_OK) break;
@@ -1414,11 +1596,13 @@ static gd_status dock_impl(gd_job *j, const gd_mc_param *mc, const RecSink *sink
       if ((e = hipStreamSynchronize(s)) != hipSuccess ||
           (e = hipMemcpy(h_half[b], d_half, half_floats * sizeof(float), hipMemcpyDeviceToHost)) !=
               hipSuccess ||
-          (e = hipMemcpy(h_cnt[b], d_cnt, (size_t)g.Rp * sizeof(int), hipMemcpyDeviceToHost)) != hipSuccess) {
+          (e = hipMemcpy(h_cnt[b], d_cnt, (size_t)g.Rp * sizeof(int), hipMemcpyDeviceToHost)) != hipSuccess ||
+          (chain_max > 0 &&
+           (e = hipMemcpy(h_fail[b], d_fail, sizeof(unsigned), hipMemcpyDeviceToHost)) != hipSuccess)) {
         st = hip_fail(e, "record copy");
         break;
       }
-      deliver(k, b);
+      if (!deliver(k, b)) break;
       continue;
     }
     if ((e = hipEventRecord(ev_done[b], s)) != hipSuccess ||
@@ -1427,6 +1611,8 @@ static gd_status dock_impl(gd_job *j, const gd_mc_param *mc, const RecSink *sink
                             j->copy_stream)) != hipSuccess ||
         (e = hipMemcpyAsync(h_cnt[b], d_cnt, (size_t)g.Rp * sizeof(int), hipMemcpyDeviceToHost,
                             j->copy_stream)) != hipSuccess ||
+        (chain_max > 0 && (e = hipMemcpyAsync(h_fail[b], d_fail, sizeof(unsigned), hipMemcpyDeviceToHost,
+                                              j->copy_stream)) != hipSuccess) ||
         (e = hipEventRecord(ev_copied[b], j->copy_stream)) != hipSuccess) {
       st = hip_fail(e, "record stream");
       break;
@@ -1436,7 +1622,10 @@ static gd_status dock_impl(gd_job *j, const gd_mc_param *mc, const RecSink *sink
         st = hip_fail(e, "record copy");
         break;
       }
-      deliver(pending, pending & 1);
+      if (!deliver(pending, pending & 1)) {
+        pending = -1;
+        break;
+      }
     }
     pending = k;
   }
@@ -1452,11 +1641,22 @@ static gd_status dock_impl(gd_job *j, const gd_mc_param *mc, const RecSink *sink
       if (st == GD_OK && e2 != hipSuccess) st = hip_fail(e2, "record copy");
     }
   }
-  if (st == GD_OK && sink && !sink->blocking && pending >= 0) deliver(pending, pending & 1);
+  if (st == GD_OK && chain_max > 0) {
+    unsigned failed = 0;
+    e = hipMemcpy(&failed, j->chain.d_sync + GD_SY_FAILED, sizeof failed, hipMemcpyDeviceToHost);
+    if (e != hipSuccess) st = hip_fail(e, "stepping kernel status");
+    if (st == GD_OK && failed) {
+      e = hipMemset(j->chain.d_sync, 0, chain_sync_bytes(j->chain.n_blocks));
+      if (e != hipSuccess) st = hip_fail(e, "stepping kernel counters");
+      j->chain.steps = 0;
+      *again = st == GD_OK;
+    }
+  }
+  if (st == GD_OK && !*again && sink && !sink->blocking && pending >= 0) deliver(pending, pending & 1);
   if (st == GD_OK && timing) st = multi ? tspan.collect(np) : tp.collect();
   const auto t1 = std::chrono::steady_clock::now();
   if (d_xt) hipFree(d_xt);
-  if (st != GD_OK) return st;
+  if (st != GD_OK || *again) return st;
   if (stats) {
     stats->ms_total = std::chrono::duration<double, std::milli>(t1 - t0).count();
     stats->ms_pair_kernel = multi ? tspan.parts_ms : tp.ms;
@@ -1470,8 +1670,32 @@ static gd_status dock_impl(gd_job *j, const gd_mc_param *mc, const RecSink *sink
     stats->ms_step_period =
         n_samples >= 2 ? span_first_last / ((double)(n_samples - 1) * kTimedEvery) : 0.0;
     stats->ms_pair_span = multi ? (tspan.n ? tspan.ms / tspan.n : 0.0) : (tp.n ? tp.ms / tp.n : 0.0);
+    if (chain_max > 0 && chain_steps > 0) {
+      // whole MC steps, pair work to next proposal, in the stepping kernel's launches
+      stats->n_pair_launch = chain_steps;
+      stats->ms_step_period = stats->ms_pair_span = tp.ms / chain_steps;
+    }
   }
   return read_out(j, out);
+}
+
+// One run at a time uses the stepping kernel: groups of two such launches that
+// wait for each other's slots could fill the device between them.  Runs that
+// overlap it step by launches, as does a run repeated because a wait ran out of
+// time (another process's launch can hold slots too): the same bits either way.
+static std::atomic<int> g_stepping{0};
+static gd_status dock_impl(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
+                           gd_replica_out *out, gd_stats *stats) {
+  int handed = 0;
+  bool again = false;
+  const bool chain = g_stepping.exchange(1) == 0;
+  gd_status st = dock_run(j, mc, sink, out, stats, chain, &handed, &again);
+  if (chain) g_stepping.store(0);
+  if (st == GD_OK && again) {
+    again = false;
+    st = dock_run(j, mc, sink, out, stats, false, &handed, &again);
+  }
+  return st;
 }
 
 gd_status gd_dock(gd_job *j, const gd_mc_param *mc, gd_replica_out *out, gd_stats *stats) {

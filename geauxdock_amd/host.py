@@ -293,8 +293,12 @@ class DeviceJob:
         return t.atoms_per_lane, t.tile_points
 
     def set_streams(self, n):
-        """Streams gd_dock steps this job on (1 to 4)."""
+        """Step this job by launches, on 1 to 4 streams."""
         check(lib().gd_job_set_streams(self.h, n), "gd_job_set_streams")
+
+    def set_step_wait(self, seconds):
+        """Bound of one wait inside the stepping kernel (default 2 s)."""
+        check(lib().gd_job_set_step_wait(self.h, seconds), "gd_job_set_step_wait")
 
     def set_tiling(self, atoms_per_lane, tile_points):
         t = abi.gd_tiling(atoms_per_lane, tile_points, 0)

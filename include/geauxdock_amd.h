@@ -149,17 +149,21 @@ typedef struct {
 typedef struct {
   double ms_total;          /* wall time of the MC loop (host clock) */
   double ms_pair_kernel;    /* summed HIP-event time of the timed pair-energy launches (on n
-                               streams: of the n part launches of each timed step) */
+                               streams: of the n part launches of each timed step); of the
+                               stepping kernel's launches where the job is stepped by it */
   double ms_finish_kernel;  /* reserved, 0: the tail kernels are not event-timed */
   int n_pair_launch;        /* pair-kernel launches timed (steps 0, 16, 32, ...; n per step on
-                               n streams) */
+                               n streams); steps taken by the stepping kernel, initial pass
+                               included */
   double pair_evals;        /* ligand-atom x protein-point evaluations done */
   double replica_steps;     /* replica x MC steps done (initial pass excluded) */
   double ms_step_period;    /* steady-state MC step period: from the first to the last timed
                                step's pair launch start (HIP events on the pair kernel's
-                               stream) over the steps between */
+                               stream) over the steps between; stepping kernel: launch time
+                               over steps */
   double ms_pair_span;      /* mean time from the first start to the last end of a timed step's
-                               pair launches (the launch itself on one stream) */
+                               pair launches (the launch itself on one stream); stepping
+                               kernel: ms_step_period */
 } gd_stats;
 
 typedef struct gd_job gd_job;         /* device-resident complex */
@@ -269,12 +273,21 @@ typedef struct {
   int waves_per_cu;         /* persistent grid size per CU */
 } gd_tiling;
 gd_status gd_tiling_get(const gd_job *job, gd_tiling *t);
-/* Streams gd_dock steps the job on (1 to 4, default 2): with n, each steps one
- * of n contiguous parts of the replica blocks between exchange points, so one
- * part's reduce and finish kernels and launch tail overlap the other parts'
- * pair work.  The results are the same bits either way.  Waits for the job's
- * stream (the parts' work lists are rebuilt). */
+/* By default gd_dock takes the steps of a job of two or more 64-replica blocks
+ * in launches of the stepping kernel, which run from one exchange point or dump
+ * end to the next; other jobs, and runs that overlap another run's stepping
+ * kernel, take a pair, a reduce and a finish launch for each step.
+ * gd_job_set_streams has the job stepped by those launches from then on, on 1
+ * to 4 streams (default 2): with n, each steps one of n contiguous parts of the
+ * replica blocks between exchange points, so one part's reduce and finish
+ * kernels and launch tail overlap the other parts' pair work.  The results are
+ * the same bits in all cases.  Waits for the job's stream (the parts' work
+ * lists are rebuilt). */
 gd_status gd_job_set_streams(gd_job *job, int n_streams);
+/* Bound of one wait inside the stepping kernel (seconds, 0 to 60, default 2).  A
+ * run that exceeds it, as when other processes' kernels hold the device, is
+ * repeated by launches. */
+gd_status gd_job_set_step_wait(gd_job *job, double seconds);
 gd_status gd_tiling_set(gd_job *job, const gd_tiling *t);
 /* Sweep atoms per lane x protein tile counts on `job` for `steps` MC steps
  * each (33 or more for an event-timed period) on the job's streams, and apply
