@@ -28,10 +28,10 @@
 
 template <int LC>
 __global__ void gd_pair_kernel_wq(const GdJob *, const GdItem *, int, int *);
-__global__ void gd_transform_kernel(const GdJob *, const GdBlock *, int *);
+__global__ void gd_start_kernel(const GdJob *, const GdBlock *, int *);
 __global__ void gd_reduce_kernel(const GdJob *, const GdBlock *);
 __global__ void gd_finish_kernel(const GdJob *, const GdBlock *, int, int, const int *, int *);
-__global__ void gd_exchange_kernel(const GdJob *, const GdExch *);
+__global__ void gd_exchange_kernel(const GdJob *, const GdExch *, int);
 
 using namespace gdr;
 
@@ -172,7 +172,7 @@ struct ExchPoint {
 gd_status exchange_launch(const BatchLists &B, int lc, int grid, int n_ex, int axes, int launch_step,
                           const int *base, hipStream_t s) {
   if (n_ex > 0) {
-    hipLaunchKernelGGL(gd_exchange_kernel, dim3(n_ex), dim3(256), 0, s, B.d_jobs, B.d_ex);
+    hipLaunchKernelGGL(gd_exchange_kernel, dim3(n_ex), dim3(256), 0, s, B.d_jobs, B.d_ex, 0);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "exchange kernel launch");
   }
@@ -182,7 +182,7 @@ gd_status exchange_launch(const BatchLists &B, int lc, int grid, int n_ex, int a
   };
   for (int axis = 0; axis < 2; ++axis)
     if (axes & (GD_EXCH_LIG << axis)) {
-      gd_status st = launch_swap(axis, B.d_jobs, B.d_blocks, B.n_blocks, B.d_swr, launch_step, base,
+      gd_status st = launch_swap(axis, B.d_jobs, B.d_blocks, B.n_blocks, B.d_swr, 0, launch_step, base,
                                  B.d_wq, pair, s);
       if (st != GD_OK) return st;
     }
@@ -220,11 +220,11 @@ gd_status batch_step(const BatchLists &B, int lc, int grid, int launch_step, con
   return GD_OK;
 }
 
+// Start state and initial-energy pass of every job in the lists.
 gd_status batch_init(const BatchLists &B, int lc, int grid, hipStream_t s) {
-  hipLaunchKernelGGL(gd_transform_kernel, dim3(B.n_blocks), dim3(256), 0, s, B.d_jobs, B.d_blocks,
-                     B.d_wq);
+  hipLaunchKernelGGL(gd_start_kernel, dim3(B.n_blocks), dim3(256), 0, s, B.d_jobs, B.d_blocks, B.d_wq);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return hip_fail(e, "transform kernel launch");
+  if (e != hipSuccess) return hip_fail(e, "start kernel launch");
   if ((e = launch_pair_wq(lc, B.d_jobs, B.d_items, B.n_items, B.d_wq, grid, s)) != hipSuccess)
     return hip_fail(e, "pair kernel (queue) launch");
   hipLaunchKernelGGL(gd_reduce_kernel, dim3(B.n_blocks * GD_RK), dim3(256), 0, s, B.d_jobs, B.d_blocks);
@@ -255,7 +255,6 @@ gd_status batch_dock_impl(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, g
     jobs[k]->h.rec = nullptr;
     jobs[k]->h.rec_cap = 0;
     jobs[k]->h.record = 0;
-    if ((st = reset_replicas(jobs[k])) != GD_OK) return st;
     steps_max = std::max(steps_max, mc[k].steps_total);
   }
   // jobs run from launch step 0; a job whose steps are done leaves the lists
@@ -357,6 +356,10 @@ gd_status batch_dock_impl(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, g
     }
     ++step;
   }
+  OutStage res;
+  std::vector<gd_replica_out *> outs(n_jobs, nullptr);
+  for (int k = 0; k < n_jobs && out; ++k) outs[k] = &out[k];
+  if (st == GD_OK) st = out_launch(jobs.data(), outs.data(), n_jobs, nullptr, s, res);
   hipError_t e = hipStreamSynchronize(s);
   if (st == GD_OK && e != hipSuccess) st = hip_fail(e, "hipStreamSynchronize");
   if (st == GD_OK && stats) st = tp.collect();
@@ -375,9 +378,7 @@ gd_status batch_dock_impl(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, g
     stats->ms_step_period = steps_max > 0 ? stats->ms_total / steps_max : 0.0;
     stats->ms_pair_span = tp.n ? tp.ms / tp.n : 0.0;
   }
-  if (out)
-    for (int k = 0; k < n_jobs; ++k)
-      if ((st = read_out(jobs[k], &out[k])) != GD_OK) return st;
+  out_copy(jobs.data(), outs.data(), n_jobs, res);
   return GD_OK;
 }
 
@@ -670,6 +671,7 @@ extern "C" gd_status gd_server_create(const gd_server_config *cfg, gd_server **o
     delete s;
     return hip_fail(e, "hipStreamCreate");
   }
+  gdr::host_pool_users(1);
   *out = s;
   return GD_OK;
 }
@@ -692,6 +694,7 @@ extern "C" gd_status gd_server_destroy(gd_server *s) {
   for (ServJob *j : s->pending) delete j;
   (void)hipStreamDestroy(s->stream);
   delete s;
+  gdr::host_pool_users(-1);
   return GD_OK;
 }
 
@@ -899,7 +902,6 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
       set_mc(j->job->h, &j->mc);
       j->job->h.record = 0;
       j->job->h.step0 = s->launch_step;
-      st = reset_replicas(j->job);
     }
     std::lock_guard<std::mutex> lk(s->mu);
     s->used -= j->foot;
@@ -1004,8 +1006,15 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
       ++it;
     }
   }
+  OutStage res;
+  std::vector<gd_job *> djobs;
+  std::vector<gd_replica_out *> douts;
+  for (ServJob *j : done) djobs.push_back(j->job), douts.push_back(j->out);
+  gd_status rs = out_launch(djobs.data(), douts.data(), (int)done.size(), nullptr, hs, res);
+  e = hipStreamSynchronize(hs);
+  if (rs == GD_OK && e != hipSuccess) rs = hip_fail(e, "results");
+  if (rs == GD_OK) out_copy(djobs.data(), douts.data(), (int)done.size(), res);
   for (ServJob *j : done) {
-    const gd_status rs = read_out(j->job, j->out);
     const double rsteps = (double)j->job->h.R * j->done_steps;
     gd_job_destroy(j->job);
     std::lock_guard<std::mutex> lk(s->mu);

@@ -150,6 +150,21 @@ struct GdChain {          // arguments of one launch of the stepping kernel
   long long wait_ticks;   // bound of one wait, in ticks of the constant-rate counter
 };
 
+struct GdPack {           // one job's results for the host
+  const float *mm, *en, *best;
+  const int *tmpi, *nacc, *nexc, *acc, *nswp;
+  float *dst;             // [R * GD_PACK_W] words
+  int R, Rp;
+};
+#define GD_PACK_W 23
+#define GD_PACK_JOBS 40   // jobs of one launch (its arguments stay under 4 KB)
+struct GdPackList {
+  struct GdPack job[GD_PACK_JOBS];
+  const unsigned *fail;   // a device word copied along (or null)
+  unsigned *fail_out;
+  int n;
+};
+
 struct GdBlock {          // one workgroup of the finish / transform kernels
   int job;
   int rb;

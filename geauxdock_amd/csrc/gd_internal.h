@@ -88,27 +88,52 @@ int pair_waves_per_cu(int lc);       // persistent pair kernel residency
 int lg2_floor(int x);
 gd_status apply_tiling(gd_job *j, int lc, int ptile);
 gd_status sync_job_struct(gd_job *j);
-gd_status reset_replicas(gd_job *j);
 void set_mc(GdJob &g, const gd_mc_param *mc);
-gd_status read_out(gd_job *j, gd_replica_out *out);
+// Host memory that kernels read and write directly, from a pool shared by all
+// threads: it keeps at most kHostPoolBytes of unused buffers, and none once the
+// last job and server are gone (host_pool_users).  A buffer is given back only
+// when no kernel uses it any more.
+constexpr size_t kHostPoolBytes = 16u << 20;
+struct HostBuf {
+  void *p = nullptr;
+  size_t bytes = 0;
+  HostBuf() = default;
+  HostBuf(const HostBuf &) = delete;
+  HostBuf &operator=(const HostBuf &) = delete;
+  ~HostBuf() { release(); }
+  gd_status acquire(size_t n);
+  void release();
+};
+void host_pool_users(int change);
+// Results of jobs whose runs are done in stream order: out_launch queues the
+// kernel that gathers them (and the word *d_fail, if given), out_copy hands them
+// over once the stream was waited for.  out[k] may be null.
+struct OutStage {
+  HostBuf buf;
+  std::vector<size_t> at;    // word offset of each job
+  const unsigned *fail = nullptr;
+};
+gd_status out_launch(gd_job *const *jobs, gd_replica_out *const *out, int n, const unsigned *d_fail, hipStream_t s,
+                     OutStage &o);
+void out_copy(gd_job *const *jobs, gd_replica_out *const *out, int n, const OutStage &o);
 float far_r2_threshold(double pmf0, double el1);
 gd_status launch_pair(int lc, const GdJob *d_jobs, const GdItem *d_items, int n_items, hipStream_t s);
 gd_status launch_finish(const GdJob *d_jobs, const GdBlock *d_blocks, int n_blocks, int mode,
                         int step, hipStream_t s);
 gd_status launch_transform(const GdJob *d_jobs, const GdBlock *d_blocks, int n_blocks, hipStream_t s);
-gd_status launch_exchange(const GdJob *d_jobs, const GdExch *d_ex, int n_ex, hipStream_t s);
+gd_status launch_exchange(const GdJob *d_jobs, int round, hipStream_t s);  // of one job
 size_t chain_sync_bytes(int n_blocks);
 // Steps that one launch may take (0: this list is stepped by launches).
 int chain_max_steps(const ChainList &c);
 gd_status launch_chain(ChainList &c, const GdJob *d_jobs, int step0, int n_steps, bool init,
                        hipStream_t s);
 // One conformer swap sub-step along `axis` (0 ligand, 1 protein) for the jobs
-// of the lists whose swr[job] round is >= 0: propose, pair (the caller's
+// of the lists whose swr[job] round is >= 0 (d_swr null: one job, `round`): propose, pair (the caller's
 // launcher), reduce, finish(EVAL), accept.  launch_step / step_base as for the
 // finish kernel of the step just completed; wq is reset for the next pair
 // launch when given.
 gd_status launch_swap(int axis, const GdJob *d_jobs, const GdBlock *d_blocks, int n_blocks,
-                      const int *d_swr, int launch_step, const int *step_base, int *wq,
+                      const int *d_swr, int round, int launch_step, const int *step_base, int *wq,
                       const std::function<gd_status()> &pair, hipStream_t s);
 
 // HIP-event timer for one kernel over many launches: events are recorded

@@ -16,8 +16,9 @@
 //                    normalises and weights, records, runs the Metropolis
 //                    test, and proposes + transforms the next move
 //                    (Philox4x32-10, counter-based).
-// plus gd_transform_kernel (pose -> ligand coordinates, used before the first
-// pass and for energy evaluation), gd_exchange_kernel (temperature swaps) and
+// plus gd_start_kernel (replica table and ligands of a run's start),
+// gd_transform_kernel (pose -> ligand coordinates, for energy evaluation),
+// gd_pack_kernel (results to the host), gd_exchange_kernel (temperature swaps) and
 // the pose-swap kernels gd_swap_propose_kernel / gd_swap_accept_kernel.
 //
 // The reference computes the same quantities in one CUDA block per replica
@@ -634,12 +635,16 @@ __device__ __forceinline__ void gd_put_atom(GD_AS_GLOBAL float *co, int Rp, int 
   gd_st<AG>(o + (size_t)2 * Rp, __builtin_fmaf(R[6], a.x, __builtin_fmaf(R[7], a.y, R[8] * a.z)) + t[2]);
 }
 
-__device__ __forceinline__ void gd_transform_atoms(GdJobC &J, int r, const float R[9],
-                                                   const float t[3], int wave, int nwave) {
+__device__ __forceinline__ void gd_transform_lig(GdJobC &J, int r, int lig, const float R[9], const float t[3],
+                                                 int wave, int nwave) {
   const int L = J.L, Rp = J.Rp;
-  const GD_AS_GLOBAL float4 *lc = gd_g(J.lig0) + (size_t)gd_g(J.ligi)[r] * L;
+  const GD_AS_GLOBAL float4 *lc = gd_g(J.lig0) + (size_t)lig * L;
   GD_AS_GLOBAL float *co = gd_g(J.coords);
   for (int l = wave; l < L; l += nwave) gd_put_atom(co, Rp, r, l, R, t, lc[l]);
+}
+__device__ __forceinline__ void gd_transform_atoms(GdJobC &J, int r, const float R[9],
+                                                   const float t[3], int wave, int nwave) {
+  gd_transform_lig(J, r, gd_g(J.ligi)[r], R, t, wave, nwave);
 }
 
 // Transform the current proposal (prop) of every replica in the block.
@@ -658,6 +663,93 @@ __global__ __launch_bounds__(256) void gd_transform_kernel(const GdJob *__restri
   gd_rotation(m, R);
   const float t[3] = {m[0] + J.center[0], m[1] + J.center[1], m[2] + J.center[2]};
   gd_transform_atoms(J, r, R, t, wave, 4);
+}
+
+// ---------------------------------------------------------------------------
+// Start of a run: the replica table of SetReplica (util.C:370-406, replica
+// n_tmp n_lig p + n_lig t + l holds ligand conformer l, temperature t, protein
+// conformer p; padding lanes conformer 0), poses, energies and counters zero,
+// and the ligands at the zero pose.  One group of four waves per 64-replica
+// block; one launch in place of 15 uploads (80-210 us a job).
+__device__ __forceinline__ void gd_start_block(GdJobC &J, const int rb) {
+  const int lane = threadIdx.x & 63, wave = gd_uniform((int)(threadIdx.x >> 6));
+  const int r = rb + lane, Rp = J.Rp;
+  const bool live = r < J.R;
+  const int nl = J.n_lig, nt = J.n_tmp;
+  const int q = r / nl, p = live ? q / nt : 0, t = live ? q % nt : 0, l = live ? r % nl : 0;
+  if (wave == 0) {
+    gd_g(J.ligi)[r] = l;
+    gd_g(J.prti)[r] = p;
+    gd_g(J.tmpi)[r] = t;
+    gd_g(J.best)[r] = 1e30f;
+    if (live) gd_g(J.own)[((size_t)p * nl + l) * nt + t] = r;
+  } else if (wave == 1) {
+    gd_g(J.acc)[r] = 0;
+    gd_g(J.nacc)[r] = 0;
+    gd_g(J.nexc)[r] = 0;
+    for (int k = 0; k < 2; ++k) gd_g(J.nswp)[(size_t)k * Rp + r] = 0, gd_g(J.rec_n)[(size_t)k * Rp + r] = 0;
+  } else if (wave == 2) {
+    for (int k = 0; k < 6; ++k) gd_g(J.mm)[(size_t)k * Rp + r] = 0.0f, gd_g(J.prop)[(size_t)k * Rp + r] = 0.0f;
+  } else {
+    for (int k = 0; k < 10; ++k) gd_g(J.en)[(size_t)k * Rp + r] = 0.0f;
+  }
+  float m[6];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) {
+    m[k] = 0.0f;
+    asm volatile("" : "+v"(m[k]));  // the arithmetic of any other pose
+  }
+  float R[9];
+  gd_rotation(m, R);
+  const float t3[3] = {m[0] + J.center[0], m[1] + J.center[1], m[2] + J.center[2]};
+  gd_transform_lig(J, r, l, R, t3, wave, 4);
+}
+
+// Every job of the lists (their device structs are in place).
+__global__ __launch_bounds__(256) void gd_start_kernel(const GdJob *__restrict__ jobs,
+                                                        const GdBlock *__restrict__ blocks, int *__restrict__ wq) {
+  if (wq && blockIdx.x == 0 && threadIdx.x == 0) *wq = 0;  // next pair launch's queue
+  const GdBlock bk = gd_c(blocks)[blockIdx.x];
+  gd_start_block(gd_c(jobs)[bk.job], bk.rb);
+}
+
+// One job, whose struct comes with the launch: the first group stores it.
+__global__ __launch_bounds__(256) void gd_start_job_kernel(const GdJob job, GdJob *__restrict__ d_job) {
+  (void)job;
+  GdJobC &J = *(GdJobC *)__builtin_amdgcn_kernarg_segment_ptr();
+  if (blockIdx.x == 0)
+    for (int k = threadIdx.x; k < (int)(sizeof(GdJob) / 4); k += 256)
+      ((unsigned *)d_job)[k] = ((const GD_AS_CONST unsigned *)&J)[k];
+  gd_start_block(J, 64 * (int)blockIdx.x);
+}
+
+// ---------------------------------------------------------------------------
+// Results of finished runs, to host memory that the device writes directly: per
+// job movematrix [R][6], energy [R][10], then best energy, temperature index,
+// accepts, exchanges, last accept and the two swap counts, [R] each.  One group
+// per 64-replica block (x) and job (y); rows are turned through LDS so that the
+// writes over the link are contiguous.  In place of nine copies, each waited
+// for (200-330 us a job).
+__global__ __launch_bounds__(256) void gd_pack_kernel(const GdPackList list) {
+  __shared__ float s[16 * 64];
+  if (list.fail && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *list.fail_out = *list.fail;
+  if ((int)blockIdx.y >= list.n) return;
+  const GdPack &p = list.job[blockIdx.y];
+  const int rb = 64 * (int)blockIdx.x, Rp = p.Rp, R = p.R;
+  if (rb >= R) return;
+  const int n = min(64, R - rb), lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (int i = wave; i < 16; i += 4) {
+    const float v = (i < 6 ? p.mm + (size_t)i * Rp : p.en + (size_t)(i - 6) * Rp)[rb + lane];
+    s[i < 6 ? 6 * lane + i : 6 * 64 + 10 * lane + i - 6] = v;
+  }
+  __syncthreads();
+  for (int k = threadIdx.x; k < 6 * n; k += 256) p.dst[(size_t)6 * rb + k] = s[k];
+  for (int k = threadIdx.x; k < 10 * n; k += 256) p.dst[(size_t)6 * R + (size_t)10 * rb + k] = s[6 * 64 + k];
+  if (lane >= n) return;
+  const int *rows[7] = {(const int *)p.best, p.tmpi, p.nacc, p.nexc, p.acc, p.nswp, p.nswp + Rp};
+#pragma unroll
+  for (int q = 0; q < 7; ++q)
+    if ((q & 3) == wave) ((int *)p.dst)[(size_t)(16 + q) * R + rb + lane] = rows[q][rb + lane];
 }
 
 // ---------------------------------------------------------------------------
@@ -1312,9 +1404,10 @@ template __global__ void gd_chain_kernel<4>(const GdChain);
 // Temperature exchange: one workgroup per (job, round) entry, threads over
 // the (protein conformer, ligand conformer) ladders; pairs (t, t+1) for
 // t = round mod 2, t+2, ...  Swaps temperature labels, not coordinates.
+// Without a list: job 0 in round `round`.
 __global__ __launch_bounds__(256) void gd_exchange_kernel(const GdJob *__restrict__ jobs,
-                                                           const GdExch *__restrict__ ex) {
-  const GdExch e = ex[blockIdx.x];
+                                                           const GdExch *__restrict__ ex, int round) {
+  const GdExch e = ex ? ex[blockIdx.x] : GdExch{0, round};
   const GdJob &J = jobs[e.job];
   const int nt = J.n_tmp, Rp = J.Rp;
   const uint64_t seed = ((uint64_t)J.seed_hi << 32) | J.seed_lo;
@@ -1347,7 +1440,7 @@ __global__ __launch_bounds__(256) void gd_exchange_kernel(const GdJob *__restric
 //   gd_swap_propose_kernel  (prop := partner's pose, transform)
 //   pair + reduce + finish(EVAL)  (energy of every replica at that pose)
 //   gd_swap_accept_kernel   (joint Metropolis decision, next step's proposal)
-// A job takes part when swr[job] >= 0 (the round) and its exchange axes hold
+// A job takes part when swr[job] >= 0 (the round; without swr, `round`) and its exchange axes hold
 // `axis`; otherwise both kernels leave it untouched, and the evaluation in
 // between changes nothing of its state.
 
@@ -1373,10 +1466,10 @@ __device__ __forceinline__ bool gd_swap_active(GdJobC &J, int rnd, int axis) {
 
 __global__ __launch_bounds__(256) void gd_swap_propose_kernel(const GdJob *__restrict__ jobs,
                                                                const GdBlock *__restrict__ blocks,
-                                                               int axis, const int *__restrict__ swr) {
+                                                               int axis, const int *__restrict__ swr, int round) {
   const GdBlock bk = gd_c(blocks)[blockIdx.x];
   GdJobC &J = gd_c(jobs)[bk.job];
-  const int rnd = gd_c(swr)[bk.job];
+  const int rnd = swr ? gd_c(swr)[bk.job] : round;
   if (!gd_swap_active(J, rnd, axis)) return;
   const int lane = threadIdx.x & 63, wave = gd_uniform((int)(threadIdx.x >> 6));
   const int r = bk.rb + lane;
@@ -1411,12 +1504,12 @@ __global__ __launch_bounds__(256) void gd_swap_propose_kernel(const GdJob *__res
 __global__ __launch_bounds__(256) void gd_swap_accept_kernel(const GdJob *__restrict__ jobs,
                                                               const GdBlock *__restrict__ blocks,
                                                               int axis, const int *__restrict__ swr,
-                                                              int launch_step,
+                                                              int round, int launch_step,
                                                               const int *__restrict__ step_base) {
   __shared__ float xf[12][64];
   const GdBlock bk = gd_c(blocks)[blockIdx.x];
   GdJobC &J = gd_c(jobs)[bk.job];
-  const int rnd = gd_c(swr)[bk.job];
+  const int rnd = swr ? gd_c(swr)[bk.job] : round;
   if (!gd_swap_active(J, rnd, axis)) return;  // uniform over the block
   if (step_base) launch_step += *step_base;
   const int lane = threadIdx.x & 63, wave = gd_uniform((int)(threadIdx.x >> 6));

@@ -36,12 +36,14 @@ __global__ void gd_reduce_kernel(const GdJob *, const GdBlock *);
 __global__ void gd_finish_kernel(const GdJob *, const GdBlock *, int, int, const int *, int *);
 template <int LC>
 __global__ void gd_chain_kernel(const GdChain);
-__global__ void gd_exchange_kernel(const GdJob *, const GdExch *);
+__global__ void gd_start_job_kernel(const GdJob, GdJob *);
+__global__ void gd_pack_kernel(const GdPackList);
+__global__ void gd_exchange_kernel(const GdJob *, const GdExch *, int);
 __global__ void gd_move_draws_kernel(uint64_t, uint32_t, int, GdScale6, int, uint32_t, int, float *);
 __global__ void gd_clock_kernel(long long, float, long long *, float *);
 __global__ void gd_copy_kernel(const float4 *, float4 *, size_t);
-__global__ void gd_swap_propose_kernel(const GdJob *, const GdBlock *, int, const int *);
-__global__ void gd_swap_accept_kernel(const GdJob *, const GdBlock *, int, const int *, int,
+__global__ void gd_swap_propose_kernel(const GdJob *, const GdBlock *, int, const int *, int);
+__global__ void gd_swap_accept_kernel(const GdJob *, const GdBlock *, int, const int *, int, int,
                                       const int *);
 
 namespace gdr {
@@ -706,8 +708,6 @@ static gd_status pack_job(const gd_job_desc *d, gd_job *j) {
   return GD_OK;
 }
 
-// Replica table of SetReplica (util.C:370-406): idx = n_tmp*n_lig*p + n_lig*t + l,
-// zero pose and energies; padding lanes get conformer 0 and never write back.
 // Device bytes gd_job_create allocates for a descriptor (tables, replica
 // state, partial sums under the default tiling, work lists).
 // Device bytes of a complex under the plain tiling, or (shared) under the
@@ -744,43 +744,6 @@ size_t footprint(const gd_job_desc *d, bool shared) {
        a((Rp / 64) * GD_RK * 8 * 64 * 4);
   b += (Rp / 64) * nL * nG * sizeof(GdItem) + (Rp / 64) * sizeof(GdBlock) + 512;
   return b;
-}
-
-gd_status reset_replicas(gd_job *j) {
-  const GdJob &g = j->h;
-  const int Rp = g.Rp, nl = g.n_lig, np = g.n_prt, nt = g.n_tmp;
-  std::vector<int> ligi(Rp, 0), prti(Rp, 0), tmpi(Rp, 0), zero(Rp, 0), own((size_t)nl * np * nt);
-  for (int p = 0; p < np; ++p)
-    for (int t = 0; t < nt; ++t)
-      for (int l = 0; l < nl; ++l) {
-        const int r = nt * nl * p + nl * t + l;
-        ligi[r] = l, prti[r] = p, tmpi[r] = t;
-        own[((size_t)p * nl + l) * nt + t] = r;
-      }
-  std::vector<float> zf((size_t)10 * Rp, 0.0f), best(Rp, 1e30f);
-  hipStream_t s = j->stream;
-  hipError_t e;
-#define GD_UP(dst, src, n)                                                          \
-  if ((e = hipMemcpyAsync(dst, src, n, hipMemcpyHostToDevice, s)) != hipSuccess) \
-    return hip_fail(e, "hipMemcpyAsync");
-  GD_UP(g.ligi, ligi.data(), Rp * sizeof(int));
-  GD_UP(g.prti, prti.data(), Rp * sizeof(int));
-  GD_UP(g.tmpi, tmpi.data(), Rp * sizeof(int));
-  GD_UP(g.acc, zero.data(), Rp * sizeof(int));
-  GD_UP(g.nacc, zero.data(), Rp * sizeof(int));
-  GD_UP(g.nexc, zero.data(), Rp * sizeof(int));
-  GD_UP(g.nswp, zero.data(), Rp * sizeof(int));
-  GD_UP(g.nswp + Rp, zero.data(), Rp * sizeof(int));
-  GD_UP(g.rec_n, zero.data(), Rp * sizeof(int));
-  GD_UP(g.rec_n + Rp, zero.data(), Rp * sizeof(int));
-  GD_UP(g.mm, zf.data(), (size_t)6 * Rp * sizeof(float));
-  GD_UP(g.prop, zf.data(), (size_t)6 * Rp * sizeof(float));
-  GD_UP(g.en, zf.data(), (size_t)10 * Rp * sizeof(float));
-  GD_UP(g.best, best.data(), Rp * sizeof(float));
-  GD_UP(g.own, own.data(), own.size() * sizeof(int));
-#undef GD_UP
-  e = hipStreamSynchronize(s);
-  return e == hipSuccess ? GD_OK : hip_fail(e, "hipStreamSynchronize");
 }
 
 // The stepping kernel's lists, made at the first run that steps by it and given
@@ -912,9 +875,8 @@ gd_status launch_transform(const GdJob *d_jobs, const GdBlock *d_blocks, int n_b
   return e == hipSuccess ? GD_OK : hip_fail(e, "transform kernel launch");
 }
 
-gd_status launch_exchange(const GdJob *d_jobs, const GdExch *d_ex, int n_ex, hipStream_t s) {
-  if (n_ex <= 0) return GD_OK;
-  hipLaunchKernelGGL(gd_exchange_kernel, dim3(n_ex), dim3(256), 0, s, d_jobs, d_ex);
+gd_status launch_exchange(const GdJob *d_jobs, int round, hipStream_t s) {
+  hipLaunchKernelGGL(gd_exchange_kernel, dim3(1), dim3(256), 0, s, d_jobs, (const GdExch *)nullptr, round);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? GD_OK : hip_fail(e, "exchange kernel launch");
 }
@@ -1007,11 +969,11 @@ gd_status launch_chain(ChainList &c, const GdJob *d_jobs, int step0, int n_steps
 }
 
 gd_status launch_swap(int axis, const GdJob *d_jobs, const GdBlock *d_blocks, int n_blocks,
-                      const int *d_swr, int launch_step, const int *step_base, int *wq,
+                      const int *d_swr, int round, int launch_step, const int *step_base, int *wq,
                       const std::function<gd_status()> &pair, hipStream_t s) {
   if (n_blocks <= 0) return GD_OK;
   hipLaunchKernelGGL(gd_swap_propose_kernel, dim3(n_blocks), dim3(256), 0, s, d_jobs, d_blocks, axis,
-                     d_swr);
+                     d_swr, round);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hip_fail(e, "swap propose kernel launch");
   gd_status st = pair();
@@ -1020,7 +982,7 @@ gd_status launch_swap(int axis, const GdJob *d_jobs, const GdBlock *d_blocks, in
   hipLaunchKernelGGL(gd_finish_kernel, dim3(n_blocks), dim3(1024), 0, s, d_jobs, d_blocks, GD_MODE_EVAL,
                      0, (const int *)nullptr, wq);
   hipLaunchKernelGGL(gd_swap_accept_kernel, dim3(n_blocks), dim3(256), 0, s, d_jobs, d_blocks, axis,
-                     d_swr, launch_step, step_base);
+                     d_swr, round, launch_step, step_base);
   e = hipGetLastError();
   return e == hipSuccess ? GD_OK : hip_fail(e, "swap kernel launch");
 }
@@ -1037,45 +999,131 @@ void set_mc(GdJob &g, const gd_mc_param *mc) {
   g.step0 = 0;
 }
 
-gd_status read_out(gd_job *j, gd_replica_out *out) {
-  if (!out) return GD_OK;
-  const GdJob &g = j->h;
-  const int R = g.R, Rp = g.Rp;
-  hipError_t e;
-  std::vector<float> f((size_t)10 * Rp);
-  std::vector<int> iv(Rp);
-  // copies on the job's stream: ordered after every kernel of the run
-  auto down = [&](void *dst, const void *src, size_t n) -> gd_status {
-    e = hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, j->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(j->stream);
-    return e == hipSuccess ? GD_OK : hip_fail(e, "hipMemcpy D2H");
-  };
-  gd_status st;
-  if (out->movematrix) {
-    if ((st = down(f.data(), g.mm, (size_t)6 * Rp * sizeof(float))) != GD_OK) return st;
-    for (int r = 0; r < R; ++r)
-      for (int i = 0; i < 6; ++i) out->movematrix[(size_t)r * 6 + i] = f[(size_t)i * Rp + r];
+// ---- host memory of results ---------------------------------------------------
+namespace {
+struct Pool {
+  std::mutex mu;
+  std::vector<std::pair<void *, size_t>> idle;
+  size_t bytes = 0;  // of idle
+  int users = 0;
+};
+Pool &pool() {
+  static Pool *p = new Pool;  // outlives every caller
+  return *p;
+}
+}  // namespace
+
+void host_pool_users(int change) {
+  Pool &P = pool();
+  std::vector<std::pair<void *, size_t>> gone;
+  {
+    std::lock_guard<std::mutex> lk(P.mu);
+    P.users += change;
+    if (P.users > 0) return;
+    gone.swap(P.idle);
+    P.bytes = 0;
   }
-  if (out->energy) {
-    if ((st = down(f.data(), g.en, (size_t)10 * Rp * sizeof(float))) != GD_OK) return st;
-    for (int r = 0; r < R; ++r)
-      for (int i = 0; i < 10; ++i) out->energy[(size_t)r * 10 + i] = f[(size_t)i * Rp + r];
-  }
-  if (out->best_energy) {
-    if ((st = down(f.data(), g.best, (size_t)Rp * sizeof(float))) != GD_OK) return st;
-    std::memcpy(out->best_energy, f.data(), (size_t)R * sizeof(float));
-  }
-  struct {
-    int *dst;
-    int *src;
-  } ints[] = {{out->idx_tmp, g.tmpi}, {out->n_accept, g.nacc}, {out->n_exchange, g.nexc},
-              {out->is_accept, g.acc}, {out->n_swap_lig, g.nswp}, {out->n_swap_prt, g.nswp + Rp}};
-  for (auto &q : ints)
-    if (q.dst) {
-      if ((st = down(iv.data(), q.src, (size_t)Rp * sizeof(int))) != GD_OK) return st;
-      std::memcpy(q.dst, iv.data(), (size_t)R * sizeof(int));
+  for (auto &b : gone) hipHostFree(b.first);
+}
+
+gd_status HostBuf::acquire(size_t n) {
+  release();
+  size_t want = 64 << 10;
+  while (want < n) want *= 2;
+  Pool &P = pool();
+  {
+    std::lock_guard<std::mutex> lk(P.mu);
+    int best = -1;
+    for (int k = 0; k < (int)P.idle.size(); ++k)
+      if (P.idle[k].second >= want && (best < 0 || P.idle[k].second < P.idle[best].second)) best = k;
+    if (best >= 0) {
+      p = P.idle[best].first, bytes = P.idle[best].second;
+      P.bytes -= bytes;
+      P.idle.erase(P.idle.begin() + best);
+      return GD_OK;
     }
+  }
+  const hipError_t e = hipHostMalloc(&p, want, hipHostMallocPortable);
+  if (e != hipSuccess) {
+    p = nullptr;
+    return hip_fail(e, "hipHostMalloc");
+  }
+  bytes = want;
   return GD_OK;
+}
+
+void HostBuf::release() {
+  if (!p) return;
+  Pool &P = pool();
+  {
+    std::lock_guard<std::mutex> lk(P.mu);
+    if (P.users > 0 && P.bytes + bytes <= kHostPoolBytes) {
+      P.idle.push_back({p, bytes});
+      P.bytes += bytes;
+      p = nullptr;
+    }
+  }
+  if (p) hipHostFree(p);
+  p = nullptr, bytes = 0;
+}
+
+gd_status out_launch(gd_job *const *jobs, gd_replica_out *const *out, int n, const unsigned *d_fail, hipStream_t s,
+                     OutStage &o) {
+  size_t words = 16;  // the failure word, on its own
+  o.at.assign(n, 0);
+  o.fail = nullptr;
+  for (int k = 0; k < n; ++k)
+    if (out[k]) {
+      o.at[k] = words;
+      words += ((size_t)jobs[k]->h.R * GD_PACK_W + 15) / 16 * 16;
+    }
+  if (words == 16 && !d_fail) return GD_OK;
+  gd_status st = o.buf.acquire(words * sizeof(float));
+  if (st != GD_OK) return st;
+  float *base = (float *)o.buf.p;
+  if (d_fail) o.fail = (unsigned *)base;
+  GdPackList list;
+  std::memset(&list, 0, sizeof list);
+  list.fail = d_fail;
+  list.fail_out = (unsigned *)base;
+  int blocks = 1;
+  const auto send = [&]() -> gd_status {
+    hipLaunchKernelGGL(gd_pack_kernel, dim3(blocks, std::max(1, list.n)), dim3(256), 0, s, list);
+    const hipError_t e = hipGetLastError();
+    list.fail = nullptr;
+    list.n = 0;
+    blocks = 1;
+    return e == hipSuccess ? GD_OK : hip_fail(e, "pack kernel launch");
+  };
+  for (int k = 0; k < n; ++k) {
+    if (!out[k]) continue;
+    const GdJob &g = jobs[k]->h;
+    list.job[list.n++] = {g.mm, g.en, g.best, g.tmpi, g.nacc, g.nexc, g.acc, g.nswp, base + o.at[k], g.R, g.Rp};
+    blocks = std::max(blocks, g.Rp / 64);
+    if (list.n == GD_PACK_JOBS && (st = send()) != GD_OK) return st;
+  }
+  return list.n > 0 || list.fail ? send() : GD_OK;
+}
+
+void out_copy(gd_job *const *jobs, gd_replica_out *const *out, int n, const OutStage &o) {
+  for (int k = 0; k < n; ++k) {
+    if (!out[k]) continue;
+    const size_t R = jobs[k]->h.R;
+    const float *p = (const float *)o.buf.p + o.at[k];
+    const gd_replica_out &q = *out[k];
+    const auto cp = [](void *dst, const float *src, size_t words) {
+      if (dst) std::memcpy(dst, src, words * 4);
+    };
+    cp(q.movematrix, p, 6 * R);
+    cp(q.energy, p + 6 * R, 10 * R);
+    cp(q.best_energy, p + 16 * R, R);
+    cp(q.idx_tmp, p + 17 * R, R);
+    cp(q.n_accept, p + 18 * R, R);
+    cp(q.n_exchange, p + 19 * R, R);
+    cp(q.is_accept, p + 20 * R, R);
+    cp(q.n_swap_lig, p + 21 * R, R);
+    cp(q.n_swap_prt, p + 22 * R, R);
+  }
 }
 
 }  // namespace gdr
@@ -1152,8 +1200,10 @@ gd_status gd_job_create(const gd_job_desc *desc, gd_job **out) {
   gd_status st = ensure_device();
   if (st != GD_OK) return st;
   gd_job *j = new gd_job();
+  gdr::host_pool_users(1);
   hipError_t e = hipStreamCreateWithFlags(&j->stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
+    gdr::host_pool_users(-1);
     delete j;
     return hip_fail(e, "hipStreamCreate");
   }
@@ -1190,6 +1240,7 @@ gd_status gd_job_destroy(gd_job *j) {
     if (ps) hipStreamDestroy(ps);
   if (j->stream) hipStreamDestroy(j->stream);
   delete j;
+  gdr::host_pool_users(-1);
   return GD_OK;
 }
 
@@ -1416,37 +1467,13 @@ static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
       }
     }
   } ev_guard{ev_done, ev_copied};
-  if ((st = reset_replicas(j)) != GD_OK) return st;
-  hipError_t e = hipMemcpyAsync(j->d_job, &g, sizeof(GdJob), hipMemcpyHostToDevice, s);
-  if (e != hipSuccess) return hip_fail(e, "hipMemcpyAsync job");
-  if ((e = hipStreamSynchronize(s)) != hipSuccess) return hip_fail(e, "hipStreamSynchronize");
+  hipError_t e = hipSuccess;
   // exchange points: after MC steps spe-1, 2spe-1, ...; round k uses table entry k
   const int spe = mc->steps_per_exchange;
   const bool tx = spe > 0 && (g.xaxes & GD_EXCH_TEMP) && g.n_tmp > 1;
   const bool lx = spe > 0 && (g.xaxes & GD_EXCH_LIG) && g.n_lig > 1;
   const bool px = spe > 0 && (g.xaxes & GD_EXCH_PRT) && g.n_prt > 1;
   const int n_rounds = (tx || lx || px) ? mc->steps_total / spe : 0;
-  void *d_xt = nullptr;  // GdExch [n_rounds], then the swap rounds int [n_rounds]
-  GdExch *d_ex = nullptr;
-  int *d_swr = nullptr;
-  if (n_rounds > 0) {
-    const size_t be = ((size_t)n_rounds * sizeof(GdExch) + 255) / 256 * 256;
-    std::vector<char> xt(be + (size_t)n_rounds * sizeof(int));
-    for (int k = 0; k < n_rounds; ++k) {
-      const GdExch x = {0, k};
-      std::memcpy(xt.data() + k * sizeof(GdExch), &x, sizeof x);
-      std::memcpy(xt.data() + be + k * sizeof(int), &k, sizeof k);
-    }
-    e = hipMalloc(&d_xt, xt.size());
-    if (e != hipSuccess) return hip_fail(e, "hipMalloc exch");
-    e = hipMemcpy(d_xt, xt.data(), xt.size(), hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-      hipFree(d_xt);
-      return hip_fail(e, "hipMemcpy exch");
-    }
-    d_ex = (GdExch *)d_xt;
-    d_swr = (int *)((char *)d_xt + be);
-  }
   const std::function<gd_status()> pair = [&]() {
     return launch_pair(g.lc, j->d_job, j->d_items, j->n_items, s);
   };
@@ -1503,7 +1530,6 @@ static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
     for (int k = 1; k < np && e == hipSuccess; ++k)
       e = hipEventCreateWithFlags(&ev_join[k], hipEventDisableTiming);
     if (e != hipSuccess) {
-      if (d_xt) hipFree(d_xt);
       return hip_fail(e, "part streams");
     }
   }
@@ -1524,7 +1550,8 @@ static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
   };
   const auto t0 = std::chrono::steady_clock::now();
   // initial energies (MonteCarlo_d with s2max = 1)
-  if (st == GD_OK) st = launch_transform(j->d_job, j->d_blocks, j->n_blocks, s);
+  hipLaunchKernelGGL(gd_start_job_kernel, dim3(j->n_blocks), dim3(256), 0, s, g, j->d_job);
+  if ((e = hipGetLastError()) != hipSuccess) st = hip_fail(e, "start kernel launch");
   if (chain_max > 0) {
     if (st == GD_OK && mc->steps_total == 0) st = launch_chain(j->chain, j->d_job, 0, 1, true, s);
   } else {
@@ -1576,10 +1603,10 @@ static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
       if (n_rounds > 0 && (step + 1) % spe == 0 && (step + 1) / spe <= n_rounds) {
         const int r = (step + 1) / spe - 1;
         if (multi && (st = join()) != GD_OK) break;
-        if (tx && (st = launch_exchange(j->d_job, d_ex + r, 1, s)) != GD_OK) break;
+        if (tx && (st = launch_exchange(j->d_job, r, s)) != GD_OK) break;
         for (int axis = 0; axis < 2; ++axis)
           if ((axis ? px : lx) &&
-              (st = launch_swap(axis, j->d_job, j->d_blocks, j->n_blocks, d_swr + r, step, nullptr,
+              (st = launch_swap(axis, j->d_job, j->d_blocks, j->n_blocks, nullptr, r, step, nullptr,
                                 nullptr, pair, s)) != GD_OK)
             break;
         if (st != GD_OK) break;
@@ -1629,6 +1656,8 @@ static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
     }
     pending = k;
   }
+  OutStage res;
+  if (st == GD_OK) st = out_launch(&j, &out, 1, chain_max > 0 ? d_fail : nullptr, s, res);
   {
     hipError_t e2 = hipStreamSynchronize(s);  // also covers steps_total == 0
     if (st == GD_OK && e2 != hipSuccess) st = hip_fail(e2, "hipStreamSynchronize");
@@ -1642,10 +1671,7 @@ static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
     }
   }
   if (st == GD_OK && chain_max > 0) {
-    unsigned failed = 0;
-    e = hipMemcpy(&failed, j->chain.d_sync + GD_SY_FAILED, sizeof failed, hipMemcpyDeviceToHost);
-    if (e != hipSuccess) st = hip_fail(e, "stepping kernel status");
-    if (st == GD_OK && failed) {
+    if (*res.fail) {
       e = hipMemset(j->chain.d_sync, 0, chain_sync_bytes(j->chain.n_blocks));
       if (e != hipSuccess) st = hip_fail(e, "stepping kernel counters");
       j->chain.steps = 0;
@@ -1655,7 +1681,6 @@ static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
   if (st == GD_OK && !*again && sink && !sink->blocking && pending >= 0) deliver(pending, pending & 1);
   if (st == GD_OK && timing) st = multi ? tspan.collect(np) : tp.collect();
   const auto t1 = std::chrono::steady_clock::now();
-  if (d_xt) hipFree(d_xt);
   if (st != GD_OK || *again) return st;
   if (stats) {
     stats->ms_total = std::chrono::duration<double, std::milli>(t1 - t0).count();
@@ -1676,7 +1701,8 @@ static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
       stats->ms_step_period = stats->ms_pair_span = tp.ms / chain_steps;
     }
   }
-  return read_out(j, out);
+  out_copy(&j, &out, 1, res);
+  return GD_OK;
 }
 
 // One run at a time uses the stepping kernel: groups of two such launches that
@@ -1711,7 +1737,12 @@ gd_status gd_dock_stream(gd_job *j, const gd_mc_param *mc, gd_record_fn fn, void
 
 gd_status gd_job_replicas(gd_job *j, gd_replica_out *out) {
   if (!j || !out) return GD_ERR_ARG;
-  return gdr::read_out(j, out);
+  OutStage res;
+  gd_status st = out_launch(&j, &out, 1, nullptr, j->stream, res);
+  const hipError_t e = hipStreamSynchronize(j->stream);
+  if (st == GD_OK && e != hipSuccess) st = hip_fail(e, "results");
+  if (st == GD_OK) out_copy(&j, &out, 1, res);
+  return st;
 }
 
 gd_status gd_dock_records(gd_job *j, int cap, float *rec, int *count) {
