@@ -33,6 +33,14 @@ struct ChainList {
 };
 }  // namespace gdr
 
+namespace gdr {
+struct EvalLanes {
+  GdJob *job;
+  int *ligi, *prti;
+  float *prop;
+};
+}  // namespace gdr
+
 struct gd_job {
   GdJob h{};                 // host mirror of the device struct
   GdJob *d_job = nullptr;    // device copy
@@ -63,6 +71,11 @@ struct gd_job {
   int n_streams = 2;         // streams the plain path steps on (1 .. kMaxParts)
   hipStream_t part_stream[kMaxParts] = {};
   gdr::ChainList chain;      // the stepping kernel's list, its queue and its counters
+  // buffers of energy evaluations: a part of the arena for the lanes of up to Rp
+  // poses (their other buffers are the job's own), and a workspace for more
+  gdr::EvalLanes ev{};
+  void *d_eval = nullptr;
+  size_t eval_bytes = 0;
   void *d_chain = nullptr;
   size_t chain_bytes = 0;
   // protein points in source order, laid out on the device per tile count
@@ -105,6 +118,11 @@ struct HostBuf {
   void release();
 };
 void host_pool_users(int change);
+// Host words for gd_energy_eval_noalloc, one buffer per device, made with the
+// device's first job and held until the process ends (null if there was no memory).
+constexpr size_t kNoallocHostBytes = 512 << 10;
+void noalloc_host_make();
+float *noalloc_host();
 // Results of jobs whose runs are done in stream order: out_launch queues the
 // kernel that gathers them (and the word *d_fail, if given), out_copy hands them
 // over once the stream was waited for.  out[k] may be null.
@@ -117,10 +135,24 @@ gd_status out_launch(gd_job *const *jobs, gd_replica_out *const *out, int n, con
                      OutStage &o);
 void out_copy(gd_job *const *jobs, gd_replica_out *const *out, int n, const OutStage &o);
 float far_r2_threshold(double pmf0, double el1);
-gd_status launch_pair(int lc, const GdJob *d_jobs, const GdItem *d_items, int n_items, hipStream_t s);
+// nb, nb_list: see gd_pair_kernel.
+gd_status launch_pair(int lc, const GdJob *d_jobs, const GdItem *d_items, int n_items, hipStream_t s, int nb = 0,
+                      int nb_list = 0);
 gd_status launch_finish(const GdJob *d_jobs, const GdBlock *d_blocks, int n_blocks, int mode,
                         int step, hipStream_t s);
-gd_status launch_transform(const GdJob *d_jobs, const GdBlock *d_blocks, int n_blocks, hipStream_t s);
+// Device buffers of one evaluation pass over nb 64-lane blocks.
+struct EvalBufs {
+  GdJob *job;
+  int *ligi, *prti;
+  float *prop, *coords, *plin, *phpc, *pmcs, *fin;
+};
+// The buffers laid out from base on; returns their bytes (base may be null).
+size_t eval_carve(const GdJob &g, int nb, char *base, EvalBufs *b);
+constexpr size_t kEvalHostWords = 2 + 6 + 10 + 9;  // host words of a pose: inputs, results
+// One pass over cnt poses on the job's stream, waited for: setup, pair, reduce
+// and finish kernels.  host: kEvalHostWords words a pose that kernels read and write.
+gd_status eval_pass(gd_job *j, const EvalBufs &b, int cnt, const int *conf, const float *pose, float *terms,
+                    float *raw, float *host);
 gd_status launch_exchange(const GdJob *d_jobs, int round, hipStream_t s);  // of one job
 size_t chain_sync_bytes(int n_blocks);
 // Steps that one launch may take (0: this list is stepped by launches).

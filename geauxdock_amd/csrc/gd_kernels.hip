@@ -17,7 +17,7 @@
 //                    test, and proposes + transforms the next move
 //                    (Philox4x32-10, counter-based).
 // plus gd_start_kernel (replica table and ligands of a run's start),
-// gd_transform_kernel (pose -> ligand coordinates, for energy evaluation),
+// gd_eval_setup_kernel (the poses of an energy evaluation as lanes),
 // gd_pack_kernel (results to the host), gd_exchange_kernel (temperature swaps) and
 // the pose-swap kernels gd_swap_propose_kernel / gd_swap_accept_kernel.
 //
@@ -553,22 +553,32 @@ __device__ __forceinline__ void gd_pair_item(const GdJob *__restrict__ jobs, con
   if constexpr (!AG) __syncthreads();
 }
 
-// One work group of GD_GROUP waves per item (grid = items).
+// One work group of GD_GROUP waves per item (grid = items).  nb > 0: the list holds
+// the items of one job, for each (chunk, tile group) those of its nb_list blocks
+// from block 0 on, and the launch covers blocks 0 .. nb-1 (any nb).
 template <int LC>
 __global__ __launch_bounds__(64 * GD_GROUP) __attribute__((amdgpu_waves_per_eu(LC == 4 ? 8 : 1))) void gd_pair_kernel(const GdJob *__restrict__ jobs,
                                                        const GdItem *__restrict__ items,
-                                                       int n_items) {
+                                                       int n_items, int nb, int nb_list) {
   __shared__ float red[GD_GROUP][GD_NLIN + LC][64];
   const int iid = gd_uniform((int)blockIdx.x);
   if (iid >= n_items) return;  // whole group: no wave waits at the barriers
-  gd_pair_item<LC>(jobs, gd_c(items)[iid], threadIdx.x & 63, gd_uniform((int)(threadIdx.x >> 6)), red);
+  GdItem it;
+  if (nb > 0) {
+    const int k = gd_uniform(iid / nb);
+    it = gd_c(items)[(size_t)k * nb_list];
+    it.rb = 64 * (iid - k * nb);
+  } else {
+    it = gd_c(items)[iid];
+  }
+  gd_pair_item<LC>(jobs, it, threadIdx.x & 63, gd_uniform((int)(threadIdx.x >> 6)), red);
 }
 
 // Persistent form: a fixed grid sized to the machine; every group pulls item
 // indices from a device counter until the list is exhausted, which balances
 // items of uneven cost (complexes of different sizes in one launch).  The
 // counter is zeroed by the kernel that runs before each launch (finish or
-// transform kernel); every group exits once the counter passes n_items.
+// start kernel); every group exits once the counter passes n_items.
 template <int LC>
 __global__ __launch_bounds__(64 * GD_GROUP) __attribute__((amdgpu_waves_per_eu(LC == 4 ? 8 : 1))) void gd_pair_kernel_wq(const GdJob *__restrict__ jobs,
                                                           const GdItem *__restrict__ items,
@@ -587,9 +597,9 @@ __global__ __launch_bounds__(64 * GD_GROUP) __attribute__((amdgpu_waves_per_eu(L
   }
 }
 
-template __global__ void gd_pair_kernel<4>(const GdJob *, const GdItem *, int);
-template __global__ void gd_pair_kernel<8>(const GdJob *, const GdItem *, int);
-template __global__ void gd_pair_kernel<16>(const GdJob *, const GdItem *, int);
+template __global__ void gd_pair_kernel<4>(const GdJob *, const GdItem *, int, int, int);
+template __global__ void gd_pair_kernel<8>(const GdJob *, const GdItem *, int, int, int);
+template __global__ void gd_pair_kernel<16>(const GdJob *, const GdItem *, int, int, int);
 template __global__ void gd_pair_kernel_wq<4>(const GdJob *, const GdItem *, int, int *);
 template __global__ void gd_pair_kernel_wq<8>(const GdJob *, const GdItem *, int, int *);
 template __global__ void gd_pair_kernel_wq<16>(const GdJob *, const GdItem *, int, int *);
@@ -647,22 +657,41 @@ __device__ __forceinline__ void gd_transform_atoms(GdJobC &J, int r, const float
   gd_transform_lig(J, r, gd_g(J.ligi)[r], R, t, wave, nwave);
 }
 
-// Transform the current proposal (prop) of every replica in the block.
-__global__ __launch_bounds__(256) void gd_transform_kernel(const GdJob *__restrict__ jobs,
-                                                            const GdBlock *__restrict__ blocks,
-                                                            int *__restrict__ wq) {
-  if (wq && blockIdx.x == 0 && threadIdx.x == 0) *wq = 0;  // next pair launch's queue
-  const GdBlock bk = gd_c(blocks)[blockIdx.x];
-  GdJobC &J = gd_c(jobs)[bk.job];
+// ---------------------------------------------------------------------------
+// Energy evaluation: the poses of a call become lanes.  conf [cnt][2] (ligand,
+// protein conformer) and pose [cnt][6] are host memory, read over the link once
+// and in order; the job struct of the evaluation comes with the launch and the
+// first group stores it for the kernels that follow.  Padding lanes: conformer 0
+// at the zero pose.  One group of four waves per 64 lanes.
+__global__ __launch_bounds__(256) void gd_eval_setup_kernel(const GdJob job, GdJob *__restrict__ d_job,
+                                                             const int *__restrict__ conf,
+                                                             const float *__restrict__ pose, int cnt) {
+  (void)job;
+  __shared__ int s_conf[2 * 64];
+  __shared__ float s_pose[6 * 64];
+  GdJobC &J = *(GdJobC *)__builtin_amdgcn_kernarg_segment_ptr();
+  const int rb = 64 * (int)blockIdx.x, n = min(64, cnt - rb);
+  for (int k = threadIdx.x; k < 6 * 64; k += 256) {
+    s_pose[k] = k < 6 * n ? pose[(size_t)6 * rb + k] : 0.0f;
+    if (k < 2 * 64) s_conf[k] = k < 2 * n ? conf[(size_t)2 * rb + k] : 0;
+  }
+  if (blockIdx.x == 0)
+    for (int k = threadIdx.x; k < (int)(sizeof(GdJob) / 4); k += 256)
+      ((unsigned *)d_job)[k] = ((const GD_AS_CONST unsigned *)&J)[k];
+  __syncthreads();
   const int lane = threadIdx.x & 63, wave = gd_uniform((int)(threadIdx.x >> 6));
-  const int r = bk.rb + lane;
-  const GD_AS_GLOBAL float *prop = gd_g(J.prop);
+  const int r = rb + lane, lig = s_conf[2 * lane];
   float m[6];
-  for (int i = 0; i < 6; ++i) m[i] = prop[(size_t)i * J.Rp + r];
+  for (int i = 0; i < 6; ++i) m[i] = s_pose[6 * lane + i];
+  if (wave == 0) {
+    gd_g(J.ligi)[r] = lig;
+    gd_g(J.prti)[r] = s_conf[2 * lane + 1];
+    for (int i = 0; i < 6; ++i) gd_g(J.prop)[(size_t)i * J.Rp + r] = m[i];
+  }
   float R[9];
   gd_rotation(m, R);
   const float t[3] = {m[0] + J.center[0], m[1] + J.center[1], m[2] + J.center[2]};
-  gd_transform_atoms(J, r, R, t, wave, 4);
+  gd_transform_lig(J, r, lig, R, t, wave, 4);
 }
 
 // ---------------------------------------------------------------------------
@@ -930,11 +959,13 @@ __device__ __forceinline__ void gd_reduce_wave(GdJobC &J, const int r, const int
 
 // Reduce kernel: GD_RK work groups (4 waves, one slice) per block; one group per
 // block kept too few loads in flight.
+// (Reduce and finish without a block list: blocks 0, 1, ... of job 0.)
 __global__ __launch_bounds__(256) void gd_reduce_kernel(const GdJob *__restrict__ jobs,
                                                          const GdBlock *__restrict__ blocks) {
   __shared__ float red[4][8][64];
   const int bi = blockIdx.x / GD_RK, k = blockIdx.x % GD_RK;
-  const GdBlock bk = gd_c(blocks)[bi];
+  GdBlock bk = {0, 64 * bi};
+  if (blocks) bk = gd_c(blocks)[bi];
   GdJobC &J = gd_c(jobs)[bk.job];
   const int lane = threadIdx.x & 63, wave = gd_uniform((int)(threadIdx.x >> 6));
   float acc[8];
@@ -1095,11 +1126,11 @@ __device__ __forceinline__ void gd_finish_post(GdJobC &J, const int rb, const in
     e[9] = tot;
 
     if (!move) {
-      if (live) {
-        GD_AS_GLOBAL float *evt = gd_g(J.ev_terms), *evr = gd_g(J.ev_raw);
-        for (int i = 0; i < 10; ++i) evt[(size_t)r * 10 + i] = e[i];
-        for (int i = 0; i < 9; ++i) evr[(size_t)r * 9 + i] = raw[i];
-      }
+      float *o = &sh.xf[0][0][0];
+#pragma unroll
+      for (int i = 0; i < 10; ++i) o[10 * lane + i] = e[i];
+#pragma unroll
+      for (int i = 0; i < 9; ++i) o[10 * 64 + 9 * lane + i] = raw[i];
     } else {
       // Metropolis (:382-392); the initial pass draws u = 0
       const float u = sh.u_s[lane];
@@ -1108,8 +1139,16 @@ __device__ __forceinline__ void gd_finish_post(GdJobC &J, const int rb, const in
       sh.acc_s[lane] = a;  // padding lanes keep their pose
     }
   }
-  if (!move) return;
   __syncthreads();
+  if (!move) {
+    // rows of the block's live lanes, in order: the buffers may be host memory
+    const float *o = &sh.xf[0][0][0];
+    const int n = min(64, J.R - rb);
+    GD_AS_GLOBAL float *evt = gd_g(J.ev_terms) + (size_t)10 * rb, *evr = gd_g(J.ev_raw) + (size_t)9 * rb;
+    for (int k = 64 * wave + lane; k < 10 * n; k += 64 * FW) evt[k] = o[k];
+    for (int k = 64 * wave + lane; k < 9 * n; k += 64 * FW) evr[k] = o[10 * 64 + k];
+    return;
+  }
   {
     const int c = sh.acc_s[lane] ? 0 : 1;
     float R[9], t[3];
@@ -1169,7 +1208,8 @@ __global__ __launch_bounds__(64 * GD_FW) void gd_finish_kernel(const GdJob *__re
   if (wq && blockIdx.x == 0 && threadIdx.x == 0) *wq = 0;  // next pair launch's queue
   if (step_base) launch_step += *step_base;  // graph replays: base step in device memory
   __shared__ GdFinLds sh;
-  const GdBlock bk = gd_c(blocks)[blockIdx.x];
+  GdBlock bk = {0, 64 * (int)blockIdx.x};
+  if (blocks) bk = gd_c(blocks)[blockIdx.x];
   GdJobC &J = gd_c(jobs)[bk.job];
   const int lane = threadIdx.x & 63, wave = gd_uniform((int)(threadIdx.x >> 6));
   const int step = launch_step - J.step0;  // this job's MC step

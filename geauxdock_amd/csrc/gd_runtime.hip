@@ -30,8 +30,8 @@
 
 // kernels (gd_kernels.hip)
 template <int LC>
-__global__ void gd_pair_kernel(const GdJob *, const GdItem *, int);
-__global__ void gd_transform_kernel(const GdJob *, const GdBlock *, int *);
+__global__ void gd_pair_kernel(const GdJob *, const GdItem *, int, int, int);
+__global__ void gd_eval_setup_kernel(const GdJob, GdJob *, const int *, const float *, int);
 __global__ void gd_reduce_kernel(const GdJob *, const GdBlock *);
 __global__ void gd_finish_kernel(const GdJob *, const GdBlock *, int, int, const int *, int *);
 template <int LC>
@@ -688,6 +688,10 @@ static gd_status pack_job(const gd_job_desc *d, gd_job *j) {
   a.add(&g.ev_terms, (size_t)10 * Rp);
   a.add(&g.ev_raw, (size_t)9 * Rp);
   a.add(&g.wq, 64);
+  a.add(&j->ev.job, 1);
+  a.add(&j->ev.ligi, (size_t)Rp);
+  a.add(&j->ev.prti, (size_t)Rp);
+  a.add(&j->ev.prop, (size_t)6 * Rp);
   gd_status st = a.commit(&j->d_base);
   if (st != GD_OK) return st;
   j->bytes = a.off;
@@ -730,7 +734,8 @@ size_t footprint(const gd_job_desc *d, bool shared) {
              a(std::max<size_t>(1, M) * 8) + a(nt * 4);
   b += a(6 * Rp * 4) * 2 + a(10 * Rp * 4) + a(Rp * 4) * 6 + a(2 * Rp * 4) + a(Rp * 4) +
        a(Rp * 4) + a(nl * np * nt * 4) +
-       a(3 * L * Rp * 4) + a(2 * Rp * 4) + a(10 * Rp * 4) + a(9 * Rp * 4) + a(64 * 4);
+       a(3 * L * Rp * 4) + a(2 * Rp * 4) + a(10 * Rp * 4) + a(9 * Rp * 4) + a(64 * 4) + a(sizeof(GdJob)) +
+       a(Rp * 4) * 2 + a(6 * Rp * 4);
   int lc, ptile;
   if (shared) {
     lc = 4;
@@ -836,18 +841,18 @@ gd_status sync_job_struct(gd_job *j) {
 
 // ---- launches ---------------------------------------------------------------
 gd_status launch_pair(int lc, const GdJob *d_jobs, const GdItem *d_items, int n_items,
-                      hipStream_t s) {
+                      hipStream_t s, int nb, int nb_list) {
   if (n_items <= 0) return GD_OK;
   const dim3 grid(n_items), block(64 * GD_GROUP);  // one group per item
   switch (lc) {
     case 4:
-      hipLaunchKernelGGL(gd_pair_kernel<4>, grid, block, 0, s, d_jobs, d_items, n_items);
+      hipLaunchKernelGGL(gd_pair_kernel<4>, grid, block, 0, s, d_jobs, d_items, n_items, nb, nb_list);
       break;
     case 8:
-      hipLaunchKernelGGL(gd_pair_kernel<8>, grid, block, 0, s, d_jobs, d_items, n_items);
+      hipLaunchKernelGGL(gd_pair_kernel<8>, grid, block, 0, s, d_jobs, d_items, n_items, nb, nb_list);
       break;
     case 16:
-      hipLaunchKernelGGL(gd_pair_kernel<16>, grid, block, 0, s, d_jobs, d_items, n_items);
+      hipLaunchKernelGGL(gd_pair_kernel<16>, grid, block, 0, s, d_jobs, d_items, n_items, nb, nb_list);
       break;
     default:
       return GD_ERR_ARG;
@@ -864,15 +869,6 @@ gd_status launch_finish(const GdJob *d_jobs, const GdBlock *d_blocks, int n_bloc
                      (const int *)nullptr, (int *)nullptr);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? GD_OK : hip_fail(e, "finish kernel launch");
-}
-
-gd_status launch_transform(const GdJob *d_jobs, const GdBlock *d_blocks, int n_blocks,
-                           hipStream_t s) {
-  if (n_blocks <= 0) return GD_OK;
-  hipLaunchKernelGGL(gd_transform_kernel, dim3(n_blocks), dim3(256), 0, s, d_jobs, d_blocks,
-                     (int *)nullptr);
-  hipError_t e = hipGetLastError();
-  return e == hipSuccess ? GD_OK : hip_fail(e, "transform kernel launch");
 }
 
 gd_status launch_exchange(const GdJob *d_jobs, int round, hipStream_t s) {
@@ -1026,6 +1022,21 @@ void host_pool_users(int change) {
   for (auto &b : gone) hipHostFree(b.first);
 }
 
+static std::atomic<float *> g_noalloc_host[64];
+void noalloc_host_make() {
+  static std::mutex mu;
+  if (g_device < 0 || g_device >= 64 || g_noalloc_host[g_device].load()) return;
+  std::lock_guard<std::mutex> lk(mu);
+  if (g_noalloc_host[g_device].load()) return;
+  void *p = nullptr;
+  if (hipHostMalloc(&p, kNoallocHostBytes, hipHostMallocPortable) != hipSuccess) {
+    (void)hipGetLastError();
+    return;
+  }
+  g_noalloc_host[g_device].store((float *)p);
+}
+float *noalloc_host() { return g_device < 0 || g_device >= 64 ? nullptr : g_noalloc_host[g_device].load(); }
+
 gd_status HostBuf::acquire(size_t n) {
   release();
   size_t want = 64 << 10;
@@ -1103,6 +1114,63 @@ gd_status out_launch(gd_job *const *jobs, gd_replica_out *const *out, int n, con
     if (list.n == GD_PACK_JOBS && (st = send()) != GD_OK) return st;
   }
   return list.n > 0 || list.fail ? send() : GD_OK;
+}
+
+// ---- energy evaluation --------------------------------------------------------
+constexpr size_t kEvalWorkspace = 64 << 20;
+
+size_t eval_carve(const GdJob &g, int nb, char *base, EvalBufs *b) {
+  const size_t Rp = (size_t)nb * 64;
+  size_t o = 0;
+  const auto take = [&](size_t bytes) {
+    char *at = base ? base + o : nullptr;
+    o += (bytes + 255) / 256 * 256;
+    return at;
+  };
+  EvalBufs c;
+  c.job = (GdJob *)take(sizeof(GdJob));
+  c.ligi = (int *)take(Rp * sizeof(int));
+  c.prti = (int *)take(Rp * sizeof(int));
+  c.prop = (float *)take(6 * Rp * sizeof(float));
+  c.coords = (float *)take((size_t)3 * g.L * Rp * sizeof(float));
+  c.plin = (float *)take((size_t)GD_NLIN * g.nL * g.nG * Rp * sizeof(float));
+  c.phpc = (float *)take((size_t)g.L * g.nG * Rp * sizeof(float));
+  c.pmcs = (float *)take((size_t)std::max(1, g.M) * g.nL * Rp * sizeof(float));
+  c.fin = (float *)take((size_t)nb * GD_RK * 8 * 64 * sizeof(float));
+  if (b) *b = c;
+  return o;
+}
+
+gd_status eval_pass(gd_job *j, const EvalBufs &b, int cnt, const int *conf, const float *pose, float *terms,
+                    float *raw, float *host) {
+  const int nb = (cnt + 63) / 64;
+  hipStream_t s = j->stream;
+  GdJob x = j->h;  // the job's tables, the evaluation's lanes and buffers
+  x.R = cnt;
+  x.Rp = nb * 64;
+  x.ligi = b.ligi, x.prti = b.prti, x.prop = b.prop, x.coords = b.coords;
+  x.part_lin = b.plin, x.part_hpc = b.phpc, x.part_mcs = b.pmcs, x.fin_part = b.fin;
+  int *h_conf = (int *)host;
+  float *h_pose = host + 2 * (size_t)cnt;
+  x.ev_terms = host + 8 * (size_t)cnt;  // written over the link by the finish kernel
+  x.ev_raw = host + 18 * (size_t)cnt;
+  x.rec = nullptr;
+  x.rec_cap = 0;
+  x.record = 0;
+  std::memcpy(h_conf, conf, (size_t)cnt * 2 * sizeof(int));
+  std::memcpy(h_pose, pose, (size_t)cnt * 6 * sizeof(float));
+  hipLaunchKernelGGL(gd_eval_setup_kernel, dim3(nb), dim3(256), 0, s, x, b.job, (const int *)h_conf,
+                     (const float *)h_pose, cnt);
+  hipError_t e = hipGetLastError();
+  gd_status st = e == hipSuccess ? GD_OK : hip_fail(e, "eval setup kernel launch");
+  if (st == GD_OK) st = launch_pair(x.lc, b.job, j->d_items, x.nL * x.nG * nb, s, nb, j->h.Rp / 64);
+  if (st == GD_OK) st = launch_finish(b.job, nullptr, nb, GD_MODE_EVAL, 0, s);
+  e = hipStreamSynchronize(s);
+  if (st == GD_OK && e != hipSuccess) st = hip_fail(e, "energy evaluation");
+  if (st != GD_OK) return st;
+  std::memcpy(terms, x.ev_terms, (size_t)cnt * 10 * sizeof(float));
+  if (raw) std::memcpy(raw, x.ev_raw, (size_t)cnt * 9 * sizeof(float));
+  return GD_OK;
 }
 
 void out_copy(gd_job *const *jobs, gd_replica_out *const *out, int n, const OutStage &o) {
@@ -1201,6 +1269,7 @@ gd_status gd_job_create(const gd_job_desc *desc, gd_job **out) {
   if (st != GD_OK) return st;
   gd_job *j = new gd_job();
   gdr::host_pool_users(1);
+  gdr::noalloc_host_make();
   hipError_t e = hipStreamCreateWithFlags(&j->stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
     gdr::host_pool_users(-1);
@@ -1233,6 +1302,7 @@ gd_status gd_job_destroy(gd_job *j) {
   if (j->d_job) hipFree(j->d_job);
   if (j->d_lists) hipFree(j->d_lists);
   gdr::chain_drop(j);
+  if (j->d_eval) hipFree(j->d_eval);
   if (j->d_rec) hipFree(j->d_rec);
   if (j->h_rec) hipHostFree(j->h_rec);
   if (j->copy_stream) hipStreamDestroy(j->copy_stream);
@@ -1260,7 +1330,7 @@ size_t gd_job_footprint(const gd_job_desc *d) { return footprint(d, false); }
 // lists, the record ring (when a run recorded) and the device job struct.
 size_t gd_job_device_bytes(const gd_job *j) {
   if (!j) return 0;
-  return j->bytes + j->part_bytes + j->lists_bytes + j->chain_bytes + j->rec_bytes + sizeof(GdJob);
+  return j->bytes + j->part_bytes + j->lists_bytes + j->chain_bytes + j->eval_bytes + j->rec_bytes + sizeof(GdJob);
 }
 
 gd_status gd_tiling_get(const gd_job *j, gd_tiling *t) {
@@ -1309,65 +1379,48 @@ gd_status gd_energy_eval(gd_job *j, int n, const int *conf, const float *pose, f
     if (conf[2 * i] < 0 || conf[2 * i] >= g.n_lig || conf[2 * i + 1] < 0 || conf[2 * i + 1] >= g.n_prt)
       return GD_ERR_ARG;
   const int Rp = g.Rp, L = g.L;
-  hipStream_t s = j->stream;
-  // save the replica conformer maps, restore at the end
-  std::vector<int> ligi_save(Rp), prti_save(Rp);
-  std::vector<float> prop_save((size_t)6 * Rp);
-  hipError_t e;
-  if ((e = hipStreamSynchronize(s)) != hipSuccess ||
-      (e = hipMemcpy(ligi_save.data(), g.ligi, Rp * sizeof(int), hipMemcpyDeviceToHost)) != hipSuccess ||
-      (e = hipMemcpy(prti_save.data(), g.prti, Rp * sizeof(int), hipMemcpyDeviceToHost)) != hipSuccess ||
-      (e = hipMemcpy(prop_save.data(), g.prop, (size_t)6 * Rp * sizeof(float), hipMemcpyDeviceToHost)) != hipSuccess)
-    return hip_fail(e, "hipMemcpy save");
-  std::vector<int> li(Rp), pi(Rp);
-  std::vector<float> pp((size_t)6 * Rp), ot((size_t)10 * Rp), orw((size_t)9 * Rp),
-      oc((size_t)3 * L * Rp);
-  const int saveR = g.R;
-  for (int base = 0; base < n && st == GD_OK; base += Rp) {
-    const int cnt = std::min(Rp, n - base);
-    std::fill(li.begin(), li.end(), 0);
-    std::fill(pi.begin(), pi.end(), 0);
-    std::fill(pp.begin(), pp.end(), 0.0f);
-    for (int i = 0; i < cnt; ++i) {
-      li[i] = conf[2 * (base + i)];
-      pi[i] = conf[2 * (base + i) + 1];
-      for (int k = 0; k < 6; ++k) pp[(size_t)k * Rp + i] = pose[6 * (size_t)(base + i) + k];
-    }
-    g.R = cnt;
-    if ((e = hipMemcpyAsync(j->d_job, &g, sizeof(GdJob), hipMemcpyHostToDevice, s)) != hipSuccess ||
-        (e = hipMemcpyAsync(g.ligi, li.data(), Rp * sizeof(int), hipMemcpyHostToDevice, s)) != hipSuccess ||
-        (e = hipMemcpyAsync(g.prti, pi.data(), Rp * sizeof(int), hipMemcpyHostToDevice, s)) != hipSuccess ||
-        (e = hipMemcpyAsync(g.prop, pp.data(), (size_t)6 * Rp * sizeof(float), hipMemcpyHostToDevice, s)) != hipSuccess) {
-      st = hip_fail(e, "hipMemcpyAsync eval");
-      break;
-    }
-    if ((st = launch_transform(j->d_job, j->d_blocks, j->n_blocks, s)) != GD_OK) break;
-    if ((st = launch_pair(g.lc, j->d_job, j->d_items, j->n_items, s)) != GD_OK) break;
-    if ((st = launch_finish(j->d_job, j->d_blocks, j->n_blocks, GD_MODE_EVAL, 0, s)) != GD_OK) break;
-    if ((e = hipMemcpyAsync(ot.data(), g.ev_terms, (size_t)10 * Rp * sizeof(float), hipMemcpyDeviceToHost, s)) != hipSuccess ||
-        (e = hipMemcpyAsync(orw.data(), g.ev_raw, (size_t)9 * Rp * sizeof(float), hipMemcpyDeviceToHost, s)) != hipSuccess ||
-        (coords && (e = hipMemcpyAsync(oc.data(), g.coords, (size_t)3 * L * Rp * sizeof(float), hipMemcpyDeviceToHost, s)) != hipSuccess) ||
-        (e = hipStreamSynchronize(s)) != hipSuccess) {
-      st = hip_fail(e, "eval readback");
-      break;
-    }
-    for (int i = 0; i < cnt; ++i) {
-      for (int k = 0; k < 10; ++k) terms[(size_t)(base + i) * 10 + k] = ot[(size_t)i * 10 + k];
-      if (raw)
-        for (int k = 0; k < 9; ++k) raw[(size_t)(base + i) * 9 + k] = orw[(size_t)i * 9 + k];
-      if (coords)
-        for (int l = 0; l < L; ++l)
-          for (int d = 0; d < 3; ++d)
-            coords[((size_t)(base + i) * L + l) * 3 + d] = oc[(size_t)(3 * l + d) * Rp + i];
+  // Poses of a pass: the job's lanes where they suffice or fill the device (1,024
+  // or more); smaller jobs with more poses take a workspace for up to 2,048, so
+  // that a pass of theirs fills it too (500 poses of a 25-replica complex: one
+  // pass in place of eight; 880 poses of a 220-replica one: one in place of four).
+  EvalBufs b = {j->ev.job, j->ev.ligi, j->ev.prti, j->ev.prop, g.coords, g.part_lin, g.part_hpc, g.part_mcs,
+                g.fin_part};
+  int lanes = Rp;
+  if (n > Rp && Rp < 1024) {
+    int nb = std::min((n + 63) / 64, 2048 / 64);
+    while (nb > Rp / 64 && eval_carve(g, nb, nullptr, nullptr) > kEvalWorkspace) --nb;
+    const size_t need = eval_carve(g, nb, nullptr, nullptr);
+    if (nb > Rp / 64) {
+      if (need > j->eval_bytes) {
+        if (j->d_eval) hipFree(j->d_eval);
+        j->d_eval = nullptr;
+        j->eval_bytes = 0;
+        if (hipMalloc(&j->d_eval, need) == hipSuccess) j->eval_bytes = need;
+        else j->d_eval = nullptr, (void)hipGetLastError();
+      }
+      if (j->d_eval) {
+        eval_carve(g, nb, (char *)j->d_eval, &b);
+        lanes = nb * 64;
+      }
     }
   }
-  g.R = saveR;
-  hipMemcpyAsync(g.ligi, ligi_save.data(), Rp * sizeof(int), hipMemcpyHostToDevice, s);
-  hipMemcpyAsync(g.prti, prti_save.data(), Rp * sizeof(int), hipMemcpyHostToDevice, s);
-  hipMemcpyAsync(g.prop, prop_save.data(), (size_t)6 * Rp * sizeof(float), hipMemcpyHostToDevice, s);
-  hipMemcpyAsync(j->d_job, &g, sizeof(GdJob), hipMemcpyHostToDevice, s);
-  e = hipStreamSynchronize(s);
-  if (st == GD_OK && e != hipSuccess) st = hip_fail(e, "eval restore");
+  HostBuf host;
+  if ((st = host.acquire((size_t)std::min(n, lanes) * kEvalHostWords * sizeof(float))) != GD_OK) return st;
+  std::vector<float> oc;
+  for (int base = 0; base < n && st == GD_OK; base += lanes) {
+    const int cnt = std::min(lanes, n - base);
+    st = eval_pass(j, b, cnt, conf + 2 * (size_t)base, pose + 6 * (size_t)base, terms + 10 * (size_t)base,
+                   raw ? raw + 9 * (size_t)base : nullptr, (float *)host.p);
+    if (st != GD_OK || !coords) continue;
+    const int W = (cnt + 63) / 64 * 64;  // lanes of the pass
+    oc.resize((size_t)3 * L * W);
+    const hipError_t e = hipMemcpy(oc.data(), b.coords, oc.size() * sizeof(float), hipMemcpyDeviceToHost);
+    if (e != hipSuccess) return hip_fail(e, "eval coordinates");
+    for (int i = 0; i < cnt; ++i)
+      for (int l = 0; l < L; ++l)
+        for (int d = 0; d < 3; ++d)
+          coords[((size_t)(base + i) * L + l) * 3 + d] = oc[(size_t)(3 * l + d) * W + i];
+  }
   return st;
 }
 

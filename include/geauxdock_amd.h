@@ -199,14 +199,15 @@ gd_status gd_energy_eval(gd_job *job, int n_pose, const int *conf, const float *
 /* gd_energy_eval that allocates nothing: no hipMalloc, hipFree or other
  * allocating call, for callers that cannot allocate (code under HIP graph
  * capture, tight serving loops, harnesses that forbid it).  No counterpart in
- * the reference.  The kernels' scratch (partial sums, staged poses, work
- * items, results) lives in one static device array of
- * GD_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends; poses run in
- * chunks of 64-pose blocks that fit it, and a job whose single block needs
- * more returns GD_ERR_SIZE.  Same results, bit for bit, as gd_energy_eval
- * (terms[n][10], raw[n][9] optional; no coordinates).  The job's replica
- * state is not touched.  Calls that overlap on one GPU share the array and
- * race; the array keeps the last call's contents. */
+ * the reference.  The kernels' scratch (partial sums, poses, transformed ligands)
+ * lives in one static device array of GD_NOALLOC_SCRATCH_BYTES per GPU, and
+ * inputs and results pass through one host buffer per GPU, made with its first
+ * job; both are held until the process ends.  Poses run in passes of 64-pose
+ * blocks that fit them, and a job whose single block needs more scratch returns
+ * GD_ERR_SIZE.  Same results, bit for bit, as gd_energy_eval (terms[n][10],
+ * raw[n][9] optional; no coordinates).  The job's replica state is not touched.
+ * Calls that overlap on one GPU share the buffers and race; the scratch keeps
+ * the last call's contents. */
 #define GD_NOALLOC_SCRATCH_BYTES (64 << 20)
 gd_status gd_energy_eval_noalloc(gd_job *job, int n_pose, const int *conf, const float *pose,
                                  float *terms, float *raw);
