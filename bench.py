@@ -406,9 +406,9 @@ def batched(kind, n_jobs, mc_steps, batch_size=0, plain_sample=0, roofline_steps
             "ratio_vs_plain_reference_shape": (n_jobs / tb) / ref_jps,
             "target_10x_met": (n_jobs / tb) / ref_jps >= 10.0,
             "best_energy_bitwise_equal_to_plain": same,
-            "roofline": roofline(flops, pair_ms, "gd_pair_kernel_wq<4>", launches_timed=st.n_pair_launch,
+            "roofline": roofline(flops, pair_ms, "gd_chain_kernel<4>", launches_timed=st.n_pair_launch,
                                  prt_pairs_per_launch=pairs,
-                                 measured="%d MC steps of the first %d jobs, every 16th pair launch "
+                                 measured="%d MC steps of the first %d jobs, the stepping kernel "
                                           "event-timed" % (roofline_steps, nb))}
     if cpu:
         rs, ms = oracle_rate(hosts[0], 20, cpu_threads())

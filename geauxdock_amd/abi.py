@@ -137,6 +137,7 @@ PROTOTYPES = {
     "gd_tiling_get": (C.c_int, [_vp, C.POINTER(gd_tiling)]),
     "gd_job_set_streams": (C.c_int, [_vp, C.c_int]),
     "gd_job_set_step_wait": (C.c_int, [_vp, C.c_double]),
+    "gd_server_set_step_wait": (C.c_int, [_vp, C.c_double]),
     "gd_tiling_set": (C.c_int, [_vp, C.POINTER(gd_tiling)]),
     "gd_autotune": (C.c_int, [_vp, C.c_int, C.POINTER(gd_tiling), C.POINTER(C.c_double)]),
     "gd_autotune_shared": (C.c_int, [C.POINTER(_vp), C.c_int, C.c_int, C.POINTER(gd_tiling),

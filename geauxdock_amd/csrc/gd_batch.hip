@@ -67,14 +67,56 @@ struct BatchLists {
   std::vector<int> axes;     // [n_jobs] GD_EXCH_* bits that can act (axis bit and > 1 entries)
   int n_items = 0, n_blocks = 0, n_jobs = 0, ex_cap = 0;
   void *mem = nullptr;
+  ChainList chain;           // the same jobs for the stepping kernel
+  int chain_max = 0;         // steps of one of its launches (0: step by launches)
+  double wait_s = GD_CHAIN_WAIT_S;  // bound of its waits (or a job's, if shorter)
+  bool failed = false;       // it failed on lists that were rebuilt since
+  void *qmem = nullptr;      // its counters, then its queue; grows only
+  size_t sync_bytes = 0, queue_bytes = 0;
+  BatchLists() = default;
+  BatchLists(const BatchLists &) = delete;
+  BatchLists &operator=(const BatchLists &) = delete;
   ~BatchLists() {
     if (mem) (void)hipFree(mem);
+    if (qmem) (void)hipFree(qmem);
   }
+  // Counters and queue for the lists of `chain`.  The queue
+  // keeps its contents: entries of earlier launches hold earlier epochs.
+  gd_status chain_memory(hipStream_t s) {
+    if (qmem && chain.epoch > 0) {
+      unsigned f = 0;
+      hipError_t e = hipStreamSynchronize(s);
+      if (e == hipSuccess) e = hipMemcpy(&f, (unsigned *)qmem + GD_SY_FAILED, sizeof f, hipMemcpyDeviceToHost);
+      if (e != hipSuccess) return hip_fail(e, "stepping kernel status");
+      failed = failed || f != 0;
+    }
+    const size_t bs = (chain_sync_bytes(chain.n_blocks) + 255) / 256 * 256, bq = chain.queue_bytes();
+    hipError_t e = hipSuccess;
+    if (bs > sync_bytes || bq > queue_bytes) {
+      if (qmem) (void)hipFree(qmem);
+      qmem = nullptr;
+      sync_bytes = std::max(sync_bytes, bs), queue_bytes = std::max(queue_bytes, bq);
+      if ((e = hipMalloc(&qmem, sync_bytes + queue_bytes)) != hipSuccess) {
+        sync_bytes = queue_bytes = 0;
+        return hip_fail(e, "hipMalloc stepping queue");
+      }
+      e = hipMemsetAsync(qmem, 0, sync_bytes + queue_bytes, s);
+    } else {
+      e = hipMemsetAsync(qmem, 0, sync_bytes, s);
+    }
+    chain.steps = 0;
+    chain.d_sync = (unsigned *)qmem;
+    chain.d_queue = (unsigned long long *)((char *)qmem + sync_bytes);
+    return e == hipSuccess ? GD_OK : hip_fail(e, "stepping queue");
+  }
+  // stepping: with the lists of the stepping kernel.
   gd_status build(const std::vector<gd_job *> &jobs, const std::vector<int> &which,
-                  hipStream_t s) {
+                  hipStream_t s, bool stepping) {
     std::vector<GdJob> js;
     std::vector<GdItem> items;
     std::vector<GdBlock> blocks;
+    std::vector<GdItem> citems;
+    std::vector<GdChainBlock> cblocks;
     axes.clear();
     for (int k = 0; k < (int)which.size(); ++k) {
       gd_job *j = jobs[which[k]];
@@ -85,8 +127,15 @@ struct BatchLists {
                      ((h.xaxes & GD_EXCH_PRT) && h.n_prt > 1 ? GD_EXCH_PRT : 0));
       // job-local items in the job's order (chunks by decreasing KDE work, then
       // tile groups, then replica blocks)
-      for (const GdItem &it : j->items) items.push_back({k, it.rb, it.a, it.b});
-      for (int rb = 0; rb < j->h.Rp; rb += 64) blocks.push_back({k, rb});
+      const int item0 = (int)citems.size();
+      for (const GdItem &it : j->items) {
+        items.push_back({k, it.rb, it.a, it.b});
+        if (it.rb == 0) citems.push_back({k, 0, it.a, it.b});
+      }
+      for (int rb = 0; rb < j->h.Rp; rb += 64) {
+        blocks.push_back({k, rb});
+        cblocks.push_back({k, rb, item0, (int)citems.size() - item0});
+      }
     }
     // longest items first: the persistent queue then ends with small items
     std::stable_sort(items.begin(), items.end(), [&](const GdItem &a, const GdItem &b) {
@@ -102,9 +151,11 @@ struct BatchLists {
     const size_t bb = (blocks.size() * sizeof(GdBlock) + 255) / 256 * 256;
     const size_t be = ((size_t)ex_cap * sizeof(GdExch) + 255) / 256 * 256;
     const size_t bs = ((size_t)ex_cap * sizeof(int) + 255) / 256 * 256;
+    const size_t bt = (citems.size() * sizeof(GdItem) + 255) / 256 * 256;
+    const size_t bc = (cblocks.size() * sizeof(GdChainBlock) + 255) / 256 * 256;
     if (mem) (void)hipFree(mem);
     mem = nullptr;
-    hipError_t e = hipMalloc(&mem, bj + bi + bb + be + bs + 512);
+    hipError_t e = hipMalloc(&mem, bj + bi + bb + be + bs + 512 + bt + bc);
     if (e != hipSuccess) return hip_fail(e, "hipMalloc batch");
     char *p = (char *)mem;
     d_jobs = (GdJob *)p;
@@ -114,6 +165,23 @@ struct BatchLists {
     d_swr = (int *)(p + bj + bi + bb + be);
     d_wq = (int *)(p + bj + bi + bb + be + bs);
     d_base = d_wq + 64;
+    char *pc = p + bj + bi + bb + be + bs + 512;
+    chain.d_items = (GdItem *)pc;
+    chain.d_blocks = (GdChainBlock *)(pc + bt);
+    std::vector<const GdJob *> hs;
+    for (const GdJob &h : js) hs.push_back(&h);
+    chain.shape(hs);
+    chain.wait_s = wait_s;
+    for (int k : which) chain.wait_s = std::min(chain.wait_s, jobs[k]->chain.wait_s);
+    chain_max = stepping ? chain_max_steps(chain) : 0;
+    if (chain_max > 0 && chain_memory(s) != GD_OK) {  // no memory for it
+      (void)hipGetLastError();
+      chain_max = 0;
+    }
+    if (chain_max > 0 &&
+        ((e = hipMemcpyAsync(pc, citems.data(), citems.size() * sizeof(GdItem), hipMemcpyHostToDevice, s)) != hipSuccess ||
+         (e = hipMemcpyAsync(pc + bt, cblocks.data(), cblocks.size() * sizeof(GdChainBlock), hipMemcpyHostToDevice, s)) != hipSuccess))
+      return hip_fail(e, "batch upload");
     if ((e = hipMemcpyAsync(d_jobs, js.data(), js.size() * sizeof(GdJob), hipMemcpyHostToDevice, s)) != hipSuccess ||
         (e = hipMemcpyAsync(d_items, items.data(), items.size() * sizeof(GdItem), hipMemcpyHostToDevice, s)) != hipSuccess ||
         (e = hipMemcpyAsync(d_blocks, blocks.data(), blocks.size() * sizeof(GdBlock), hipMemcpyHostToDevice, s)) != hipSuccess ||
@@ -220,11 +288,18 @@ gd_status batch_step(const BatchLists &B, int lc, int grid, int launch_step, con
   return GD_OK;
 }
 
-// Start state and initial-energy pass of every job in the lists.
-gd_status batch_init(const BatchLists &B, int lc, int grid, hipStream_t s) {
+// Start state of every job in the lists.
+gd_status batch_start(const BatchLists &B, hipStream_t s) {
   hipLaunchKernelGGL(gd_start_kernel, dim3(B.n_blocks), dim3(256), 0, s, B.d_jobs, B.d_blocks, B.d_wq);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return hip_fail(e, "start kernel launch");
+  return e == hipSuccess ? GD_OK : hip_fail(e, "start kernel launch");
+}
+
+// Start state and initial-energy pass of every job in the lists.
+gd_status batch_init(const BatchLists &B, int lc, int grid, hipStream_t s) {
+  gd_status st = batch_start(B, s);
+  if (st != GD_OK) return st;
+  hipError_t e;
   if ((e = launch_pair_wq(lc, B.d_jobs, B.d_items, B.n_items, B.d_wq, grid, s)) != hipSuccess)
     return hip_fail(e, "pair kernel (queue) launch");
   hipLaunchKernelGGL(gd_reduce_kernel, dim3(B.n_blocks * GD_RK), dim3(256), 0, s, B.d_jobs, B.d_blocks);
@@ -235,9 +310,11 @@ gd_status batch_init(const BatchLists &B, int lc, int grid, hipStream_t s) {
 }
 
 // Batched docking (gd_batch_dock); the overrides (> 0) replace the shared
-// tile size and the persistent grid's waves per CU (autotuner sweeps).
-gd_status batch_dock_impl(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, gd_replica_out *out,
-                          gd_stats *stats, int ptile_override, int waves_override) {
+// tile size and the persistent grid's waves per CU (autotuner sweeps).  step_ok:
+// the stepping kernel may be used; *again: one of its waits ran out of time and
+// the batch is to be repeated without it.
+gd_status batch_run(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, gd_replica_out *out,
+                    gd_stats *stats, int ptile_override, int waves_override, bool step_ok, bool *again) {
   if (!jobs_in || n_jobs <= 0 || !mc) return GD_ERR_ARG;
   gd_status st = ensure_device();
   if (st != GD_OK) return st;
@@ -261,11 +338,17 @@ gd_status batch_dock_impl(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, g
   std::vector<int> active(n_jobs);
   for (int k = 0; k < n_jobs; ++k) active[k] = k;
   BatchLists B;
-  if ((st = B.build(jobs, active, s)) != GD_OK) return st;
+  if ((st = B.build(jobs, active, s, step_ok)) != GD_OK) return st;
   const int grid = pair_grid(waves_override > 0 ? waves_override : pair_waves_per_cu(lc));
   KTimer tp;
   const auto t0 = std::chrono::steady_clock::now();
-  if ((st = batch_init(B, lc, grid, s)) != GD_OK) return st;
+  // the stepping kernel takes the steps up to the next exchange point or end of
+  // any job in one launch (256 jobs of 25 replicas and a screen of large ones are
+  // in the figures of gd_chain_kernel); the initial pass goes with the first
+  bool init = step_ok && B.chain_max > 0;
+  int chain_steps = 0;
+  if ((st = init ? batch_start(B, s) : batch_init(B, lc, grid, s)) != GD_OK) return st;
+  if (init && steps_max == 0) st = launch_chain(B.chain, B.d_jobs, 0, 1, true, s);
 
   // Segments of identical shape are captured once into a HIP graph and
   // replayed with the base step in device memory (no memset nodes).
@@ -288,7 +371,7 @@ gd_status batch_dock_impl(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, g
   std::vector<int> round;
   while (step < steps_max && st == GD_OK) {
     // graph path: whole segment, every job active, exchange point at its end
-    if (uniform && seg > 1 && step + seg <= steps_max && !stats) {
+    if (!(step_ok && B.chain_max > 0) && uniform && seg > 1 && step + seg <= steps_max && !stats) {
       hipError_t e = hipMemcpyAsync(B.d_base, &step, sizeof(int), hipMemcpyHostToDevice, s);
       if (e != hipSuccess) {
         st = hip_fail(e, "hipMemcpyAsync base");
@@ -336,7 +419,23 @@ gd_status batch_dock_impl(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, g
       if (step < mc[k].steps_total) act.push_back(k);
     if (act.size() != (size_t)B.n_jobs) {
       // shrink the lists to the jobs still running; their step0 stays 0
-      if ((st = B.build(jobs, act, s)) != GD_OK) break;
+      if ((st = B.build(jobs, act, s, step_ok)) != GD_OK) break;
+    }
+    int n = 1;
+    const bool chain = step_ok && B.chain_max > 0;
+    if (chain) {
+      n = B.chain_max - (init ? 1 : 0);
+      for (int k : act) {
+        const int spe = mc[k].steps_per_exchange;
+        n = std::min(n, mc[k].steps_total - step);
+        if (spe > 0) n = std::min(n, spe - step % spe);
+      }
+      if (stats && (st = tp.begin(s)) != GD_OK) break;
+      if ((st = launch_chain(B.chain, B.d_jobs, step, n + (init ? 1 : 0), init, s)) != GD_OK) break;
+      if (stats && (st = tp.end(s)) != GD_OK) break;
+      chain_steps += n + (init ? 1 : 0);
+      init = false;
+      step += n - 1;  // the last of them
     }
     round.assign(act.size(), -1);
     for (int q = 0; q < (int)act.size(); ++q) {
@@ -344,7 +443,9 @@ gd_status batch_dock_impl(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, g
       if (spe > 0 && (step + 1) % spe == 0) round[q] = (step + 1) / spe - 1;
     }
     xp.set(B, round);
-    st = batch_step(B, lc, grid, step, nullptr, &xp, s, stats ? &tp : nullptr);
+    if (!chain) st = batch_step(B, lc, grid, step, nullptr, &xp, s, stats ? &tp : nullptr);
+    else if (!xp.empty() && (st = exchange_upload(B, xp, s)) == GD_OK)
+      st = exchange_launch(B, lc, grid, (int)xp.ex.size(), xp.axes, step, nullptr, s);
     if (st != GD_OK) break;
     if (!xp.empty() || (stats && (step + 1) % 64 == 0)) {
       hipError_t e = hipStreamSynchronize(s);  // exchange tables are rewritten next time
@@ -359,14 +460,17 @@ gd_status batch_dock_impl(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, g
   OutStage res;
   std::vector<gd_replica_out *> outs(n_jobs, nullptr);
   for (int k = 0; k < n_jobs && out; ++k) outs[k] = &out[k];
-  if (st == GD_OK) st = out_launch(jobs.data(), outs.data(), n_jobs, nullptr, s, res);
+  if (st == GD_OK)
+    st = out_launch(jobs.data(), outs.data(), n_jobs, B.qmem ? (const unsigned *)B.qmem + GD_SY_FAILED : nullptr, s,
+                    res);
   hipError_t e = hipStreamSynchronize(s);
   if (st == GD_OK && e != hipSuccess) st = hip_fail(e, "hipStreamSynchronize");
+  *again = st == GD_OK && (B.failed || (res.fail && *res.fail));
   if (st == GD_OK && stats) st = tp.collect();
   const auto t1 = std::chrono::steady_clock::now();
   if (gexec) (void)hipGraphExecDestroy(gexec);
   if (graph) (void)hipGraphDestroy(graph);
-  if (st != GD_OK) return st;
+  if (st != GD_OK || *again) return st;
   if (stats) {
     stats->ms_total = std::chrono::duration<double, std::milli>(t1 - t0).count();
     stats->ms_pair_kernel = tp.ms;
@@ -377,9 +481,26 @@ gd_status batch_dock_impl(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, g
     // the batch's timed runs synchronise every 64 steps: the period on the host clock
     stats->ms_step_period = steps_max > 0 ? stats->ms_total / steps_max : 0.0;
     stats->ms_pair_span = tp.n ? tp.ms / tp.n : 0.0;
+    if (chain_steps > 0) stats->n_pair_launch = chain_steps, stats->ms_pair_span = tp.ms / chain_steps;
   }
   out_copy(jobs.data(), outs.data(), n_jobs, res);
   return GD_OK;
+}
+
+gd_status batch_dock_impl(gd_job **jobs, int n_jobs, const gd_mc_param *mc, gd_replica_out *out,
+                          gd_stats *stats, int ptile_override, int waves_override) {
+  bool again = false;
+  gd_status st;
+  {
+    // a sweep over persistent grids runs by launches
+    Stepping turn(waves_override <= 0);
+    st = batch_run(jobs, n_jobs, mc, out, stats, ptile_override, waves_override, turn.mine, &again);
+  }
+  if (st == GD_OK && again) {
+    again = false;
+    st = batch_run(jobs, n_jobs, mc, out, stats, ptile_override, waves_override, false, &again);
+  }
+  return st;
 }
 
 }  // namespace
@@ -584,10 +705,13 @@ struct gd_server {
   // guards active, lists, dirty, launch_step (never held by submit or results)
   std::mutex smu;
   std::vector<ServJob *> active;
+  std::vector<ServJob *> restart;  // to begin again at the next step
   int launch_step = 0;
   hipStream_t stream = nullptr;
   BatchLists lists;
   bool dirty = true;
+  bool lists_stepping = false;   // the lists were built with the stepping kernel's
+  bool by_launches = false;      // a wait of the stepping kernel ran out of time
   int lc = kSharedLc;
   std::chrono::steady_clock::time_point t0;
   // host input pipeline: file requests parsed by a loader thread
@@ -687,6 +811,7 @@ extern "C" gd_status gd_server_destroy(gd_server *s) {
   for (FileReq *r : s->files) delete r;
   for (auto &kv : s->held) delete kv.second;
   (void)hipStreamSynchronize(s->stream);
+  for (ServJob *j : s->restart) s->active.push_back(j);
   for (ServJob *j : s->active) {
     gd_job_destroy(j->job);
     delete j;
@@ -695,6 +820,14 @@ extern "C" gd_status gd_server_destroy(gd_server *s) {
   (void)hipStreamDestroy(s->stream);
   delete s;
   gdr::host_pool_users(-1);
+  return GD_OK;
+}
+
+extern "C" gd_status gd_server_set_step_wait(gd_server *s, double seconds) {
+  if (!s || !(seconds >= 0.0) || seconds > 60.0) return GD_ERR_ARG;
+  std::lock_guard<std::mutex> ls(s->smu);
+  s->lists.wait_s = seconds;
+  s->dirty = true;
   return GD_OK;
 }
 
@@ -822,20 +955,21 @@ extern "C" gd_status gd_server_cancel(gd_server *s, int64_t ticket) {
   }
   // an active job: wait for a running sweep
   std::lock_guard<std::mutex> ls(s->smu);
-  for (auto it = s->active.begin(); it != s->active.end(); ++it)
-    if ((*it)->ticket == ticket) {
-      (void)hipStreamSynchronize(s->stream);
-      ServJob *j = *it;
-      s->active.erase(it);
-      s->dirty = true;
-      std::lock_guard<std::mutex> lk(s->mu);
-      fail_request(s, ticket, GD_ERR_STATE, j->t_submit, j->t_admit);
-      s->results.back().replica_steps = (double)j->job->h.R * j->done_steps;
-      s->used -= j->foot;
-      gd_job_destroy(j->job);
-      delete j;
-      return GD_OK;
-    }
+  for (std::vector<ServJob *> *list : {&s->active, &s->restart})
+    for (auto it = list->begin(); it != list->end(); ++it)
+      if ((*it)->ticket == ticket) {
+        (void)hipStreamSynchronize(s->stream);
+        ServJob *j = *it;
+        list->erase(it);
+        s->dirty = true;
+        std::lock_guard<std::mutex> lk(s->mu);
+        fail_request(s, ticket, GD_ERR_STATE, j->t_submit, j->t_admit);
+        s->results.back().replica_steps = (double)j->job->h.R * j->done_steps;
+        s->used -= j->foot;
+        gd_job_destroy(j->job);
+        delete j;
+        return GD_OK;
+      }
   return GD_ERR_ARG;
 }
 
@@ -885,6 +1019,8 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
   // (1) admission: FIFO while the estimated footprint fits and a slot is free;
   // an admitted job is then charged its actual device bytes
   std::vector<ServJob *> admitted;
+  admitted.swap(s->restart);  // those of a sweep that failed, from their first step
+  for (ServJob *j : admitted) j->job->h.step0 = j->step0 = s->launch_step;
   for (;;) {
     ServJob *j = nullptr;
     {
@@ -926,7 +1062,7 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
       nj.push_back(j->job);
     }
     BatchLists B;
-    st = B.build(nj, idx, hs);
+    st = B.build(nj, idx, hs, false);
     if (st == GD_OK) st = batch_init(B, s->lc, pair_grid(pair_waves_per_cu(s->lc)), hs);
     if (st == GD_OK) {
       hipError_t e = hipStreamSynchronize(hs);
@@ -947,6 +1083,7 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
   }
   // (3) advance every active job by up to sweep_steps (no lock held but smu:
   // submits and result queries proceed meanwhile)
+  Stepping turn(!s->by_launches);
   for (int k = 0; k < s->cfg.sweep_steps && st == GD_OK; ++k) {
     std::vector<int> act;
     std::vector<gd_job *> jobs;
@@ -955,23 +1092,41 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
       if (s->active[q]->done_steps < s->active[q]->mc.steps_total && !s->active[q]->converged)
         act.push_back(q);
     if (act.empty()) break;
-    if (s->dirty || (int)act.size() != s->lists.n_jobs) {
+    if (s->dirty || (int)act.size() != s->lists.n_jobs || s->lists_stepping != turn.mine) {
       for (int q : act) jobs[q]->h.step0 = s->active[q]->step0;
-      if ((st = s->lists.build(jobs, act, hs)) != GD_OK) return st;
+      if ((st = s->lists.build(jobs, act, hs, turn.mine)) != GD_OK) return st;
+      s->lists_stepping = turn.mine;
       s->dirty = false;
+    }
+    // by the stepping kernel up to the next exchange point or end of any job
+    const bool chain = turn.mine && s->lists.chain_max > 0;
+    int n = 1;
+    if (chain) {
+      n = std::min(s->lists.chain_max, s->cfg.sweep_steps - k);
+      for (int q : act) {
+        const ServJob *j = s->active[q];
+        const int spe = j->mc.steps_per_exchange;
+        n = std::min(n, j->mc.steps_total - j->done_steps);
+        if (spe > 0) n = std::min(n, spe - j->done_steps % spe);
+      }
+      st = launch_chain(s->lists.chain, s->lists.d_jobs, s->launch_step, n, false, hs);
     }
     std::vector<int> round(act.size(), -1);
     for (int q = 0; q < (int)act.size(); ++q) {
       ServJob *j = s->active[act[q]];
       const int spe = j->mc.steps_per_exchange;
-      if (spe > 0 && (j->done_steps + 1) % spe == 0) round[q] = (j->done_steps + 1) / spe - 1;
+      if (spe > 0 && (j->done_steps + n) % spe == 0) round[q] = (j->done_steps + n) / spe - 1;
     }
     ExchPoint xp;
     xp.set(s->lists, round);
-    st = batch_step(s->lists, s->lc, pair_grid(pair_waves_per_cu(s->lc)), s->launch_step, nullptr, &xp, hs, nullptr);
+    const int grid = pair_grid(pair_waves_per_cu(s->lc)), last = s->launch_step + n - 1;
+    if (!chain) st = batch_step(s->lists, s->lc, grid, last, nullptr, &xp, hs, nullptr);
+    else if (st == GD_OK && !xp.empty() && (st = exchange_upload(s->lists, xp, hs)) == GD_OK)
+      st = exchange_launch(s->lists, s->lc, grid, (int)xp.ex.size(), xp.axes, last, nullptr, hs);
     if (!xp.empty()) (void)hipStreamSynchronize(hs);  // exchange tables are reused next step
-    ++s->launch_step;
-    for (int q : act) s->active[q]->done_steps += 1;
+    s->launch_step += n;
+    k += n - 1;
+    for (int q : act) s->active[q]->done_steps += n;
     // jobs whose step counts end here leave the lists at the next step
     bool any_done = false;
     for (int q : act)
@@ -981,6 +1136,23 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
   hipError_t e = hipStreamSynchronize(hs);
   if (st == GD_OK && e != hipSuccess) st = hip_fail(e, "sweep");
   if (st != GD_OK) return st;
+  if (turn.mine && s->lists.qmem) {
+    unsigned f = 0;
+    e = hipMemcpy(&f, (unsigned *)s->lists.qmem + GD_SY_FAILED, sizeof f, hipMemcpyDeviceToHost);
+    if (e != hipSuccess) return hip_fail(e, "stepping kernel status");
+    if (f || s->lists.failed) {
+      // a wait ran out of time: the jobs begin again, by launches (the same bits:
+      // a job's draws are a function of its own steps)
+      s->by_launches = s->dirty = true;
+      for (ServJob *j : s->active) {
+        j->done_steps = 0;
+        j->converged = false;
+        j->best_hist.clear();
+        s->restart.push_back(j);
+      }
+      s->active.clear();
+    }
+  }
   // (4) convergence: a job's sweep ends every sweep_steps of its own steps
   if (s->cfg.converge_sweeps > 0) {
     for (ServJob *j : s->active) {
@@ -1024,7 +1196,7 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
     s->used -= j->foot;
     delete j;
   }
-  if (n_active) *n_active = (int)s->active.size();
+  if (n_active) *n_active = (int)(s->active.size() + s->restart.size());
   std::lock_guard<std::mutex> lk(s->mu);
   if (n_done) *n_done = (int)s->results.size();
   return GD_OK;

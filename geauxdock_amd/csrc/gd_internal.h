@@ -157,6 +157,15 @@ gd_status launch_exchange(const GdJob *d_jobs, int round, hipStream_t s);  // of
 size_t chain_sync_bytes(int n_blocks);
 // Steps that one launch may take (0: this list is stepped by launches).
 int chain_max_steps(const ChainList &c);
+// The right to launch the stepping kernel, for as long as the object lives: one
+// run of the process at a time has it (see dock_impl).
+struct Stepping {
+  bool mine;
+  explicit Stepping(bool wanted);
+  ~Stepping();
+  Stepping(const Stepping &) = delete;
+  Stepping &operator=(const Stepping &) = delete;
+};
 gd_status launch_chain(ChainList &c, const GdJob *d_jobs, int step0, int n_steps, bool init,
                        hipStream_t s);
 // One conformer swap sub-step along `axis` (0 ligand, 1 protein) for the jobs

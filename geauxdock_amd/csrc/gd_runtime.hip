@@ -935,6 +935,16 @@ int chain_max_steps(const ChainList &c) {
   return n >= 2 ? n : 0;  // the first launch takes the initial pass and a step
 }
 
+// One run at a time uses the stepping kernel: groups of two such launches that
+// wait for each other's slots could fill the device between them.  Runs that
+// overlap it step by launches, as does a run repeated because a wait ran out of
+// time (another process's launch can hold slots too): the same bits either way.
+static std::atomic<int> g_stepping{0};
+Stepping::Stepping(bool wanted) : mine(wanted && g_stepping.exchange(1) == 0) {}
+Stepping::~Stepping() {
+  if (mine) g_stepping.store(0);
+}
+
 gd_status launch_chain(ChainList &c, const GdJob *d_jobs, int step0, int n_steps, bool init,
                        hipStream_t s) {
   if (n_steps <= 0) return GD_OK;
@@ -1758,18 +1768,15 @@ static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
   return GD_OK;
 }
 
-// One run at a time uses the stepping kernel: groups of two such launches that
-// wait for each other's slots could fill the device between them.  Runs that
-// overlap it step by launches, as does a run repeated because a wait ran out of
-// time (another process's launch can hold slots too): the same bits either way.
-static std::atomic<int> g_stepping{0};
 static gd_status dock_impl(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
                            gd_replica_out *out, gd_stats *stats) {
   int handed = 0;
   bool again = false;
-  const bool chain = g_stepping.exchange(1) == 0;
-  gd_status st = dock_run(j, mc, sink, out, stats, chain, &handed, &again);
-  if (chain) g_stepping.store(0);
+  gd_status st;
+  {
+    Stepping turn(true);
+    st = dock_run(j, mc, sink, out, stats, turn.mine, &handed, &again);
+  }
   if (st == GD_OK && again) {
     again = false;
     st = dock_run(j, mc, sink, out, stats, false, &handed, &again);

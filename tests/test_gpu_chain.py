@@ -101,6 +101,82 @@ def test_threads_dock_side_by_side(ene):
             _same(want[k], out)
 
 
+# lists of jobs: one block (launches), many small ones, jobs of unlike sizes whose
+# lengths and exchange intervals differ, more blocks than finishers
+LISTS = {
+    "one block": [(300, 9, 3, 2, 1)],
+    "small": [(500 + 7 * k, 8 + k, 5, 5, 1) for k in range(12)],
+    "unlike": [(37, 2, 1, 1, 1), (3000, 40, 10, 11, 4), (700, 30, 13, 5, 1), (1200, 24, 5, 5, 2)],
+    "blocks": [(150, 6, 16, 8, 5) for _ in range(7)],
+}
+
+
+def _batch(devs, mcs, stats=False):
+    import ctypes as C
+    from geauxdock_amd import abi
+    outs = [g.host.ReplicaOut(d.n_rep) for d in devs]
+    arr = (C.c_void_p * len(devs))(*[d.h for d in devs])
+    oc = (abi.gd_replica_out * len(devs))(*[o.c for o in outs])
+    st = abi.gd_stats()
+    g.check(g.lib().gd_batch_dock(arr, len(devs), (abi.gd_mc_param * len(devs))(*mcs), oc,
+                                  C.byref(st) if stats else None), "gd_batch_dock")
+    return outs, st
+
+
+@pytest.mark.parametrize("name", list(LISTS))
+@pytest.mark.parametrize("steps,spe", [(0, 0), (11, 4), (30, 0)])
+def test_batch_chain_matches_launches(ene, name, steps, spe):
+    """A wait bound of 0 has the batch repeated by launches."""
+    jobs = [g.synth_complex(*s, seed=k + 1, ene=ene) for k, s in enumerate(LISTS[name])]
+    devs = [g.DeviceJob(j) for j in jobs]
+    ragged = name == "unlike"
+    mcs = [g.make_mc(steps + (3 * k if ragged and steps else 0), steps_per_exchange=spe + (k if ragged and spe else 0),
+                     seed=3, job_id=k, move_mode="gaussian", axes=("temp", "lig", "prt")) for k in range(len(jobs))]
+    a, st = _batch(devs, mcs, stats=True)
+    b, _ = _batch(devs, mcs)
+    devs[-1].set_step_wait(0.0)
+    c, _ = _batch(devs, mcs)
+    devs[-1].set_step_wait(2.0)
+    d, _ = _batch(devs, mcs)
+    for k in range(len(jobs)):
+        for o in (b, c, d):
+            _same(a[k], o[k])
+    assert steps == 0 or st.n_pair_launch > 0
+    for x in devs:
+        x.close()
+
+
+def test_server_chain_matches_launches(ene):
+    import ctypes as C
+    from geauxdock_amd import abi
+    jobs = [g.synth_complex(*s, seed=k + 1, ene=ene) for k, s in enumerate(LISTS["unlike"])]
+    mcs = [g.make_mc(20 + 9 * k, steps_per_exchange=4 + k, seed=3, job_id=k, axes=("temp", "lig")) for k in range(4)]
+    got = []
+    for wait in (2.0, 0.0):
+        s = C.c_void_p()
+        cfg = abi.gd_server_config(hbm_budget=64 << 30, max_active=3, sweep_steps=13)
+        g.check(g.lib().gd_server_create(C.byref(cfg), C.byref(s)), "create")
+        g.check(g.lib().gd_server_set_step_wait(s, wait), "wait")
+        outs = [g.host.ReplicaOut(j.n_rep) for j in jobs]
+        for j, mc, o in zip(jobs, mcs, outs):
+            t = C.c_int64()
+            g.check(g.lib().gd_server_submit(s, C.byref(j.desc), C.byref(mc), C.byref(o.c), C.byref(t)), "submit")
+        done = 0
+        for _ in range(60):
+            na, nd, n, res = C.c_int(), C.c_int(), C.c_int(), (abi.gd_job_result * 8)()
+            g.check(g.lib().gd_server_step(s, C.byref(na), C.byref(nd)), "step")
+            g.lib().gd_server_results(s, res, 8, C.byref(n))
+            assert all(res[i].status == 0 for i in range(n.value))
+            done += n.value
+            if done == 4:
+                break
+        assert done == 4
+        g.lib().gd_server_destroy(s)
+        got.append(outs)
+    for a, b in zip(*got):
+        _same(a, b)
+
+
 @pytest.mark.parametrize("bad", [-1.0, 61.0, float("nan")])
 def test_bad_wait(ene, bad):
     dev = g.DeviceJob(g.synth_complex(40, 4, 2, 2, 1, seed=1, ene=ene))
