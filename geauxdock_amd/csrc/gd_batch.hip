@@ -1032,8 +1032,8 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
       s->pending.pop_front();
       s->used += j->foot;  // held while the job is created
     }
-    st = gd_job_create(&j->desc, &j->job);
-    if (st == GD_OK) st = shared_tiling(j->job, 0);  // serving tiling: a function of the complex only
+    // the tiling of shared launches (a function of the complex only), on the server's stream
+    st = job_create(&j->desc, hs, &j->job);
     if (st == GD_OK) {
       set_mc(j->job->h, &j->mc);
       j->job->h.record = 0;

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <functional>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -34,6 +35,26 @@ struct ChainList {
 }  // namespace gdr
 
 namespace gdr {
+// Host memory that kernels read and write directly, from a pool shared by all
+// threads: it keeps at most kHostPoolBytes of unused buffers, and none once the
+// last job and server are gone (host_pool_users).  A buffer is given back only
+// when no kernel uses it any more.
+constexpr size_t kHostPoolBytes = 16u << 20;
+struct HostBuf {
+  void *p = nullptr;
+  size_t bytes = 0;
+  bool pinned = true;
+  HostBuf() = default;
+  HostBuf(const HostBuf &) = delete;
+  HostBuf &operator=(const HostBuf &) = delete;
+  ~HostBuf() { release(); }
+  // copies_only: no kernel will use it, so large buffers may be ordinary memory
+  gd_status acquire(size_t n, bool copies_only = false);
+  void release();
+
+ private:
+  gd_status plain(size_t n);
+};
 struct EvalLanes {
   GdJob *job;
   int *ligi, *prti;
@@ -83,10 +104,12 @@ struct gd_job {
   std::vector<float4> src_pattr;   // [P]
   std::vector<float> src_pspv;     // [n_types + 1][P]
   std::vector<int> src_key;        // [P] class * GD_PTAB_PT + point type
-  std::vector<int> src_spread;     // [P] order inside a (class, type) group
+  std::vector<int> src_order;      // [P] points by class, type and spread
   std::vector<int> atom_kde;       // [L] KDE anchors of each device atom (item order)
   int laid_nP = 0;                 // tile count of the device order (0: none yet)
   hipStream_t stream = nullptr;
+  bool own_stream = true;
+  std::vector<std::unique_ptr<gdr::HostBuf>> staged;  // uploads in flight on stream
 };
 
 namespace gdr {
@@ -101,22 +124,8 @@ int pair_waves_per_cu(int lc);       // persistent pair kernel residency
 int lg2_floor(int x);
 gd_status apply_tiling(gd_job *j, int lc, int ptile);
 gd_status sync_job_struct(gd_job *j);
+gd_status job_create(const gd_job_desc *desc, hipStream_t shared, gd_job **out);
 void set_mc(GdJob &g, const gd_mc_param *mc);
-// Host memory that kernels read and write directly, from a pool shared by all
-// threads: it keeps at most kHostPoolBytes of unused buffers, and none once the
-// last job and server are gone (host_pool_users).  A buffer is given back only
-// when no kernel uses it any more.
-constexpr size_t kHostPoolBytes = 16u << 20;
-struct HostBuf {
-  void *p = nullptr;
-  size_t bytes = 0;
-  HostBuf() = default;
-  HostBuf(const HostBuf &) = delete;
-  HostBuf &operator=(const HostBuf &) = delete;
-  ~HostBuf() { release(); }
-  gd_status acquire(size_t n);
-  void release();
-};
 void host_pool_users(int change);
 // Host words for gd_energy_eval_noalloc, one buffer per device, made with the
 // device's first job and held until the process ends (null if there was no memory).

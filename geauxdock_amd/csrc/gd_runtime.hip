@@ -17,6 +17,7 @@
 #include <cmath>
 #include <limits>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -349,6 +350,17 @@ static gd_status alloc_partials(gd_job *j, GdJob &g, int cap_rp) {
   return st;
 }
 
+// Staging memory for an upload on the job's stream, held until sync_job_struct
+// has waited for it.
+static gd_status stage(gd_job *j, size_t bytes, HostBuf **out) {
+  std::unique_ptr<HostBuf> b(new HostBuf);
+  const gd_status st = b->acquire(bytes, true);
+  if (st != GD_OK) return st;
+  *out = b.get();
+  j->staged.push_back(std::move(b));
+  return GD_OK;
+}
+
 // Device order of the protein points for the job's tile count: class by
 // class, tile b of nP reads points pcls[c] + b, + nP, ... (strided, see the
 // pair kernel).  The class's points sorted by (type, spread) are dealt out so
@@ -359,12 +371,8 @@ static gd_status alloc_partials(gd_job *j, GdJob &g, int cap_rp) {
 static gd_status layout_points(gd_job *j) {
   GdJob &g = j->h;
   const int P = g.P, nP = g.nP, np = g.n_prt;
-  std::vector<int> ord(P), porder(P);
-  for (int p = 0; p < P; ++p) ord[p] = p;
-  std::stable_sort(ord.begin(), ord.end(), [&](int x, int y) {
-    return j->src_key[x] != j->src_key[y] ? j->src_key[x] < j->src_key[y]
-                                          : j->src_spread[x] < j->src_spread[y];
-  });
+  const std::vector<int> &ord = j->src_order;
+  std::vector<int> porder(P);
   for (int c = 0; c < 4; ++c) {
     const int lo = g.pcls[c], n = g.pcls[c + 1] - lo, q = n / nP, r = n % nP;
     for (int i = 0; i < n; ++i) {
@@ -379,22 +387,24 @@ static gd_status layout_points(gd_job *j) {
     }
   }
   const size_t nty1 = j->src_pspv.size() / (size_t)P;
-  std::vector<float4> pco((size_t)np * P), pattr(P);
-  std::vector<float> pspv(j->src_pspv.size());
+  // gathered into staging memory in the device's layout (pcoord, pattr and pspv
+  // follow each other) and sent in one copy; sync_job_struct waits for it
+  HostBuf *buf;
+  gd_status st = stage(j, (size_t)((const char *)g.pspv - (const char *)g.pcoord) + j->src_pspv.size() * sizeof(float),
+                       &buf);
+  if (st != GD_OK) return st;
+  char *h = (char *)buf->p;
+  float4 *pco = (float4 *)h, *pattr = (float4 *)(h + ((const char *)g.pattr - (const char *)g.pcoord));
+  float *pspv = (float *)(h + ((const char *)g.pspv - (const char *)g.pcoord));
   for (int i = 0; i < np; ++i)
     for (int q2 = 0; q2 < P; ++q2) pco[(size_t)i * P + q2] = j->src_pco[(size_t)i * P + porder[q2]];
   for (int q2 = 0; q2 < P; ++q2) pattr[q2] = j->src_pattr[porder[q2]];
   for (size_t t = 0; t < nty1; ++t)
     for (int q2 = 0; q2 < P; ++q2) pspv[t * P + q2] = j->src_pspv[t * P + porder[q2]];
+  const size_t bytes = (size_t)((const char *)(g.pspv + j->src_pspv.size()) - (const char *)g.pcoord);
   hipError_t e;
   if ((e = hipStreamSynchronize(j->stream)) != hipSuccess ||
-      (e = hipMemcpyAsync((void *)g.pcoord, pco.data(), pco.size() * sizeof(float4),
-                          hipMemcpyHostToDevice, j->stream)) != hipSuccess ||
-      (e = hipMemcpyAsync((void *)g.pattr, pattr.data(), pattr.size() * sizeof(float4),
-                          hipMemcpyHostToDevice, j->stream)) != hipSuccess ||
-      (e = hipMemcpyAsync((void *)g.pspv, pspv.data(), pspv.size() * sizeof(float),
-                          hipMemcpyHostToDevice, j->stream)) != hipSuccess ||
-      (e = hipStreamSynchronize(j->stream)) != hipSuccess)
+      (e = hipMemcpyAsync((void *)g.pcoord, h, bytes, hipMemcpyHostToDevice, j->stream)) != hipSuccess)
     return hip_fail(e, "point layout upload");
   j->laid_nP = nP;
   return GD_OK;
@@ -437,6 +447,34 @@ gd_status apply_tiling(gd_job *j, int lc, int ptile) {
 }
 
 // ---------------------------------------------------------------------------
+// pmf1 summed over every (atom, point) pair, atom by atom, in double.  By the
+// counts of the types where that is the same number: if the magnitudes sum to
+// less than 2^53 units in the last place of the smallest value, every partial sum
+// in any order is exact.
+static double pmf_sum(const gd_job_desc *d) {
+  const gd_enepara *e = d->ene;
+  std::vector<int> nl(GD_NLT, 0), np(GD_NPT, 0);
+  for (int l = 0; l < d->lig_natom; ++l) ++nl[d->lig_t[l]];
+  for (int p = 0; p < d->prt_npoint; ++p) ++np[d->prt_t[p]];
+  double sum = 0.0, mag = 0.0, ulp = INFINITY;
+  for (int a = 0; a < GD_NLT; ++a)
+    for (int b = 0; b < GD_NPT; ++b) {
+      const float v = e->pmf1[a][b];
+      const double n = (double)nl[a] * np[b];
+      if (n == 0.0 || v == 0.0f) continue;
+      int ex;
+      std::frexp(v, &ex);
+      ulp = std::min(ulp, std::ldexp(1.0, ex - 24));
+      mag += std::fabs((double)v) * n;
+      sum += v * n;
+    }
+  if (mag < 4503599627370496.0 * ulp) return sum;  // 2^52: one bit to spare for mag's own rounding
+  double sp = 0.0;
+  for (int l = 0; l < d->lig_natom; ++l)
+    for (int p = 0; p < d->prt_npoint; ++p) sp += e->pmf1[d->lig_t[l]][d->prt_t[p]];
+  return sp;
+}
+
 // Pack a complex into the device layout.
 static gd_status pack_job(const gd_job_desc *d, gd_job *j) {
   const int L = d->lig_natom, P = d->prt_npoint, K = d->kde_npoint, M = d->mcs_nrow;
@@ -535,30 +573,42 @@ static gd_status pack_job(const gd_job_desc *d, gd_job *j) {
     for (int c = 0; c < 4; ++c) g.pcls[c + 1] = g.pcls[c] + nc[c];
     j->src_key.resize(P);
     for (int p = 0; p < P; ++p) j->src_key[p] = cls(p) * GD_PTAB_PT + d->prt_t[p];
-    // within a (class, type) group: the bit-reversed rank of the distance to the
+    // within a (class, type) group: by the bit-reversed rank of the distance to the
     // pocket centre (protein conformer 0), a low-discrepancy order in which any
     // run of consecutive points spans near and far points evenly
-    std::vector<float> dist(P);
+    std::vector<uint64_t> rec(P), tmp(P);  // distance bits, point
     for (int p = 0; p < P; ++p) {
       const float dx = d->prt_x[p] - d->pocket_center[0], dy = d->prt_y[p] - d->pocket_center[1],
                   dz = d->prt_z[p] - d->pocket_center[2];
-      dist[p] = dx * dx + dy * dy + dz * dz;
+      const float dist = dx * dx + dy * dy + dz * dz;  // >= 0: ordered as its bits
+      uint32_t u;
+      std::memcpy(&u, &dist, 4);
+      rec[p] = (uint64_t)u << 32 | (uint32_t)p;
     }
+    // stable radix passes over the distance, then the key
+    const auto pass = [&](const auto &digit, int n) {
+      std::vector<int> at(n + 1, 0);
+      for (int p = 0; p < P; ++p) ++at[digit(rec[p]) + 1];
+      for (int k = 0; k < n; ++k) at[k + 1] += at[k];
+      for (int p = 0; p < P; ++p) tmp[at[digit(rec[p])]++] = rec[p];
+      rec.swap(tmp);
+    };
+    for (int sh = 32; sh < 64; sh += 11) pass([&](uint64_t v) { return (int)(v >> sh & 2047); }, 2048);
+    pass([&](uint64_t v) { return j->src_key[(uint32_t)v]; }, 4 * GD_PTAB_PT);
     std::vector<int> ord(P);
-    for (int p = 0; p < P; ++p) ord[p] = p;
-    std::stable_sort(ord.begin(), ord.end(), [&](int x, int y) {
-      return j->src_key[x] != j->src_key[y] ? j->src_key[x] < j->src_key[y] : dist[x] < dist[y];
-    });
-    j->src_spread.resize(P);
+    for (int p = 0; p < P; ++p) ord[p] = (int)(uint32_t)rec[p];
+    j->src_order.resize(P);
     for (int i = 0; i < P;) {
       int e = i;
       while (e < P && j->src_key[ord[e]] == j->src_key[ord[i]]) ++e;
       int bits = 0;
       while ((1 << bits) < e - i) ++bits;
-      for (int k = i; k < e; ++k) {
-        unsigned v = (unsigned)(k - i), rv = 0;
-        for (int t = 0; t < bits; ++t) rv |= ((v >> t) & 1u) << (bits - 1 - t);
-        j->src_spread[ord[k]] = (int)rv;
+      // in the order of the bit-reversed rank
+      int o = i;
+      for (unsigned rv = 0; rv < (1u << bits); ++rv) {
+        unsigned v = 0;
+        for (int t = 0; t < bits; ++t) v |= ((rv >> t) & 1u) << (bits - 1 - t);
+        if ((int)v < e - i) j->src_order[o++] = ord[i + (int)v];
       }
       i = e;
     }
@@ -600,10 +650,8 @@ static gd_status pack_job(const gd_job_desc *d, gd_job *j) {
     GdAtom &a = atoms[l];
     a.tidx = trow[lt];
     a.q = d->lig_c[l];
-    int b = 0;
-    while (b < K && d->kde_t[b] < lt) ++b;
-    int en = b;
-    while (en < K && d->kde_t[en] == lt) ++en;
+    const int b = K ? (int)(std::lower_bound(d->kde_t, d->kde_t + K, lt) - d->kde_t) : 0;
+    const int en = K ? (int)(std::upper_bound(d->kde_t, d->kde_t + K, lt) - d->kde_t) : 0;
     a.kde_b = b;
     a.kde_e = en;
     j->atom_kde[l] = en - b;
@@ -636,10 +684,7 @@ static gd_status pack_job(const gd_job_desc *d, gd_job *j) {
   // pmf1 summed over every (atom, point) pair: the PMF term of a pose is this
   // constant minus the pair kernel's corrections
   {
-    double sp = 0.0;
-    for (int l = 0; l < L; ++l)
-      for (int p = 0; p < P; ++p) sp += e->pmf1[d->lig_t[l]][d->prt_t[p]];
-    g.pmf_all = (float)sp;
+    g.pmf_all = (float)pmf_sum(d);
   }
   // scalars
   g.lj0 = e->lj0, g.lj1 = e->lj1, g.el0 = e->el0, g.el1 = e->el1, g.a1 = e->a1, g.b1 = e->b1;
@@ -660,16 +705,16 @@ static gd_status pack_job(const gd_job_desc *d, gd_job *j) {
   GdAtom *d_atoms;
   float *d_ptab, *d_pspv, *d_mb;
   float2 *d_mcsrow;
-  a.add(&d_lig0, lig0.size());
+  a.add(&d_lig0, lig0.size());  // the tables, to d_mb: one upload
   a.add(&d_atoms, atoms.size());
-  a.add(&d_pco, j->src_pco.size());
-  a.add(&d_pattr, j->src_pattr.size());
   a.add(&d_ptab, ptab.size());
-  a.add(&d_pspv, j->src_pspv.size());
   a.add(&d_kde, kde.size());
   a.add(&d_mcs, mcs.size());
   a.add(&d_mcsrow, mcsrow.size());
   a.add(&d_mb, (size_t)nt);
+  a.add(&d_pco, j->src_pco.size());  // the points: another (layout_points)
+  a.add(&d_pattr, j->src_pattr.size());
+  a.add(&d_pspv, j->src_pspv.size());
   a.add(&g.mm, (size_t)6 * Rp);
   a.add(&g.prop, (size_t)6 * Rp);
   a.add(&g.en, (size_t)10 * Rp);
@@ -697,17 +742,21 @@ static gd_status pack_job(const gd_job_desc *d, gd_job *j) {
   j->bytes = a.off;
   g.lig0 = d_lig0, g.atoms = d_atoms, g.pcoord = d_pco, g.pattr = d_pattr, g.ptab = d_ptab;
   g.pspv = d_pspv, g.kde = d_kde, g.mcs = d_mcs, g.mcsrow = d_mcsrow, g.minus_beta = d_mb;
-  auto up = [&](void *dst, const void *src, size_t n) -> gd_status {
-    hipError_t e2 = hipMemcpy(dst, src, n, hipMemcpyHostToDevice);
-    return e2 == hipSuccess ? GD_OK : hip_fail(e2, "hipMemcpy H2D");
+  const size_t bytes = (size_t)((char *)(d_mb + nt) - (char *)d_lig0);
+  HostBuf *buf;
+  if ((st = stage(j, bytes, &buf)) != GD_OK) return st;
+  const auto put = [&](const void *dst, const void *src, size_t n) {
+    std::memcpy((char *)buf->p + ((const char *)dst - (const char *)d_lig0), src, n);
   };
-  if ((st = up(d_lig0, lig0.data(), lig0.size() * sizeof(float4))) != GD_OK) return st;
-  if ((st = up(d_atoms, atoms.data(), atoms.size() * sizeof(GdAtom))) != GD_OK) return st;
-  if ((st = up(d_ptab, ptab.data(), ptab.size() * sizeof(float))) != GD_OK) return st;
-  if ((st = up(d_kde, kde.data(), kde.size() * sizeof(float4))) != GD_OK) return st;
-  if ((st = up(d_mcs, mcs.data(), mcs.size() * sizeof(float4))) != GD_OK) return st;
-  if ((st = up(d_mcsrow, mcsrow.data(), mcsrow.size() * sizeof(float2))) != GD_OK) return st;
-  if ((st = up(d_mb, d->minus_beta, (size_t)nt * sizeof(float))) != GD_OK) return st;
+  put(d_lig0, lig0.data(), lig0.size() * sizeof(float4));
+  put(d_atoms, atoms.data(), atoms.size() * sizeof(GdAtom));
+  put(d_ptab, ptab.data(), ptab.size() * sizeof(float));
+  put(d_kde, kde.data(), kde.size() * sizeof(float4));
+  put(d_mcs, mcs.data(), mcs.size() * sizeof(float4));
+  put(d_mcsrow, mcsrow.data(), mcsrow.size() * sizeof(float2));
+  put(d_mb, d->minus_beta, (size_t)nt * sizeof(float));
+  const hipError_t e2 = hipMemcpyAsync(d_lig0, buf->p, bytes, hipMemcpyHostToDevice, j->stream);
+  if (e2 != hipSuccess) return hip_fail(e2, "table upload");
   j->h = g;
   return GD_OK;
 }
@@ -791,8 +840,6 @@ static gd_status chain_make(gd_job *j) {
 }
 
 gd_status sync_job_struct(gd_job *j) {
-  hipError_t e = hipMemcpyAsync(j->d_job, &j->h, sizeof(GdJob), hipMemcpyHostToDevice, j->stream);
-  if (e != hipSuccess) return hip_fail(e, "hipMemcpyAsync job");
   std::vector<GdBlock> blocks;
   for (int rb = 0; rb < j->h.Rp; rb += 64) blocks.push_back({0, rb});
   j->n_blocks = (int)blocks.size();
@@ -821,22 +868,24 @@ gd_status sync_job_struct(gd_job *j) {
   const size_t bi = (size_t)j->n_items * sizeof(GdItem), bb = (size_t)j->n_blocks * sizeof(GdBlock),
                bh = part_items.size() * sizeof(GdItem);
   j->lists_bytes = 0;
-  e = hipMalloc(&j->d_lists, up(bi) + up(bb) + up(bh) + 256);
+  hipError_t e = hipMalloc(&j->d_lists, up(bi) + up(bb) + up(bh) + 256);
   if (e != hipSuccess) return hip_fail(e, "hipMalloc lists");
   j->lists_bytes = up(bi) + up(bb) + up(bh) + 256;
   j->d_items = (GdItem *)j->d_lists;
   j->d_blocks = (GdBlock *)((char *)j->d_lists + up(bi));
   j->d_items_part[0] = (GdItem *)((char *)j->d_lists + up(bi) + up(bb));
   for (int k = 1; k < np; ++k) j->d_items_part[k] = j->d_items_part[k - 1] + j->n_items_part[k - 1];
-  if ((e = hipMemcpyAsync(j->d_items, j->items.data(), bi, hipMemcpyHostToDevice, j->stream)) != hipSuccess)
-    return hip_fail(e, "hipMemcpyAsync items");
-  if ((e = hipMemcpyAsync(j->d_blocks, blocks.data(), bb, hipMemcpyHostToDevice, j->stream)) != hipSuccess)
-    return hip_fail(e, "hipMemcpyAsync blocks");
-  if (bh && (e = hipMemcpyAsync(j->d_items_part[0], part_items.data(), bh, hipMemcpyHostToDevice,
-                                j->stream)) != hipSuccess)
-    return hip_fail(e, "hipMemcpyAsync part items");
-  e = hipStreamSynchronize(j->stream);
-  return e == hipSuccess ? GD_OK : hip_fail(e, "hipStreamSynchronize");
+  HostBuf *buf;
+  const gd_status st = stage(j, up(bi) + up(bb) + bh, &buf);
+  if (st != GD_OK) return st;
+  std::memcpy(buf->p, j->items.data(), bi);
+  std::memcpy((char *)buf->p + up(bi), blocks.data(), bb);
+  if (bh) std::memcpy((char *)buf->p + up(bi) + up(bb), part_items.data(), bh);
+  e = hipMemcpyAsync(j->d_lists, buf->p, up(bi) + up(bb) + bh, hipMemcpyHostToDevice, j->stream);
+  const hipError_t e2 = hipStreamSynchronize(j->stream);
+  j->staged.clear();
+  if (e == hipSuccess) e = e2;
+  return e == hipSuccess ? GD_OK : hip_fail(e, "list upload");
 }
 
 // ---- launches ---------------------------------------------------------------
@@ -1047,8 +1096,9 @@ void noalloc_host_make() {
 }
 float *noalloc_host() { return g_device < 0 || g_device >= 64 ? nullptr : g_noalloc_host[g_device].load(); }
 
-gd_status HostBuf::acquire(size_t n) {
+gd_status HostBuf::acquire(size_t n, bool copies_only) {
   release();
+  if (copies_only && n > kHostPoolBytes) return plain(n);  // not worth pinning for one copy
   size_t want = 64 << 10;
   while (want < n) want *= 2;
   Pool &P = pool();
@@ -1067,14 +1117,34 @@ gd_status HostBuf::acquire(size_t n) {
   const hipError_t e = hipHostMalloc(&p, want, hipHostMallocPortable);
   if (e != hipSuccess) {
     p = nullptr;
+    if (copies_only) {
+      (void)hipGetLastError();
+      return plain(n);
+    }
     return hip_fail(e, "hipHostMalloc");
   }
   bytes = want;
   return GD_OK;
 }
 
+gd_status HostBuf::plain(size_t n) {
+  p = std::malloc(n);
+  if (!p) {
+    set_error("out of host memory");
+    return GD_ERR_HIP;
+  }
+  pinned = false;
+  bytes = n;
+  return GD_OK;
+}
+
 void HostBuf::release() {
   if (!p) return;
+  if (!pinned) {
+    std::free(p);
+    p = nullptr, bytes = 0, pinned = true;
+    return;
+  }
   Pool &P = pool();
   {
     std::lock_guard<std::mutex> lk(P.mu);
@@ -1204,6 +1274,47 @@ void out_copy(gd_job *const *jobs, gd_replica_out *const *out, int n, const OutS
   }
 }
 
+// A job of its own (plain tiling, its own stream), or, with a stream, one that
+// runs in shared launches on that stream.
+gd_status job_create(const gd_job_desc *desc, hipStream_t shared, gd_job **out) {
+  if (!desc || !out) return GD_ERR_ARG;
+  *out = nullptr;
+  gd_status st = ensure_device();
+  if (st != GD_OK) return st;
+  gd_job *j = new gd_job();
+  host_pool_users(1);
+  noalloc_host_make();
+  hipError_t e = hipSuccess;
+  j->own_stream = shared == nullptr;
+  j->stream = shared;
+  if (!shared) e = hipStreamCreateWithFlags(&j->stream, hipStreamNonBlocking);
+  if (e != hipSuccess) {
+    host_pool_users(-1);
+    delete j;
+    return hip_fail(e, "hipStreamCreate");
+  }
+  st = pack_job(desc, j);
+  if (st == GD_OK) {
+    e = hipMalloc(&j->d_job, sizeof(GdJob));
+    if (e != hipSuccess) st = hip_fail(e, "hipMalloc job");
+  }
+  if (st == GD_OK) {
+    int lc = 4, ptile;
+    if (shared)
+      ptile = shared_ptile(j->h.L, j->h.P);
+    else
+      default_tiling(j->h.L, j->h.P, j->h.R, lc, ptile);
+    st = apply_tiling(j, lc, ptile);
+  }
+  if (st == GD_OK) st = sync_job_struct(j);
+  if (st != GD_OK) {
+    gd_job_destroy(j);
+    return st;
+  }
+  *out = j;
+  return GD_OK;
+}
+
 }  // namespace gdr
 
 using namespace gdr;
@@ -1272,41 +1383,14 @@ void gd_philox(const uint32_t ctr[4], const uint32_t key[2], int rounds, uint32_
   for (int i = 0; i < 4; ++i) out[i] = r.v[i];
 }
 
-gd_status gd_job_create(const gd_job_desc *desc, gd_job **out) {
-  if (!desc || !out) return GD_ERR_ARG;
-  *out = nullptr;
-  gd_status st = ensure_device();
-  if (st != GD_OK) return st;
-  gd_job *j = new gd_job();
-  gdr::host_pool_users(1);
-  gdr::noalloc_host_make();
-  hipError_t e = hipStreamCreateWithFlags(&j->stream, hipStreamNonBlocking);
-  if (e != hipSuccess) {
-    gdr::host_pool_users(-1);
-    delete j;
-    return hip_fail(e, "hipStreamCreate");
-  }
-  st = pack_job(desc, j);
-  if (st == GD_OK) {
-    e = hipMalloc(&j->d_job, sizeof(GdJob));
-    if (e != hipSuccess) st = hip_fail(e, "hipMalloc job");
-  }
-  if (st == GD_OK) {
-    int lc, ptile;
-    default_tiling(j->h.L, j->h.P, j->h.R, lc, ptile);
-    st = apply_tiling(j, lc, ptile);
-  }
-  if (st == GD_OK) st = sync_job_struct(j);
-  if (st != GD_OK) {
-    gd_job_destroy(j);
-    return st;
-  }
-  *out = j;
-  return GD_OK;
-}
+gd_status gd_job_create(const gd_job_desc *desc, gd_job **out) { return gdr::job_create(desc, nullptr, out); }
 
 gd_status gd_job_destroy(gd_job *j) {
   if (!j) return GD_OK;
+  if (!j->staged.empty()) {  // uploads of a creation that failed
+    hipStreamSynchronize(j->stream);
+    j->staged.clear();
+  }
   if (j->d_base) hipFree(j->d_base);
   if (j->d_part) hipFree(j->d_part);
   if (j->d_job) hipFree(j->d_job);
@@ -1318,7 +1402,7 @@ gd_status gd_job_destroy(gd_job *j) {
   if (j->copy_stream) hipStreamDestroy(j->copy_stream);
   for (hipStream_t ps : j->part_stream)
     if (ps) hipStreamDestroy(ps);
-  if (j->stream) hipStreamDestroy(j->stream);
+  if (j->stream && j->own_stream) hipStreamDestroy(j->stream);
   delete j;
   gdr::host_pool_users(-1);
   return GD_OK;
@@ -1374,10 +1458,8 @@ gd_status gd_tiling_set(gd_job *j, const gd_tiling *t) {
   return sync_job_struct(j);
 }
 
-// Energies of arbitrary poses through the same pair/finish kernels: the poses
-// are loaded as a temporary replica set (chunks of at most the job's padded
-// replica count), transformed, evaluated in EVAL mode, and the job's own
-// replica state is restored afterwards.
+// Energies of arbitrary poses through the same pair/finish kernels, on lanes of
+// their own (eval_pass); the job's replica state is not touched.
 gd_status gd_energy_eval(gd_job *j, int n, const int *conf, const float *pose, float *terms,
                          float *raw, float *coords) {
   if (!j || n < 0 || (n > 0 && (!conf || !pose || !terms))) return GD_ERR_ARG;
