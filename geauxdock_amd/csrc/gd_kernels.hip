@@ -152,8 +152,13 @@ struct GdPairConst {
 // ligand atom of the lane against one protein point, with the force-field row
 // rw of (atom type, point type) in scalar registers.  CLS: bit 0 = cdc point
 // (hydrophobic term), bit 1 = class-2 point (psp term); the caller dispatches
-// on the point's flags once, so the pairs carry no per-pair class tests.
-template <int CLS>
+// on the point's flags once, so the pairs carry no per-pair class tests.  TERMS:
+// GD_T_LJ, GD_T_REST or both.
+#define GD_T_LJ 1
+#define GD_T_REST 2
+#define GD_T_ALL 3
+#define GD_T_KDE 4  // no pair terms: KDE and MCS shares (gd_pair_kernel_split)
+template <int CLS, int TERMS = GD_T_ALL>
 __device__ __forceinline__ void gd_pair_one(
     const GdPairConst &k, const float (&rw)[GD_ROW], const GD_AS_CONST float *__restrict__ pspv,
     const int P, const int p, const unsigned prow, const float4 c, const float pele, const float phpp,
@@ -173,7 +178,7 @@ __device__ __forceinline__ void gd_pair_one(
     // p1 = p1a / r^9, p2 = p2a / r^6, multiplied through by r^9 / p1a:
     // (1 - q r^3) / (lj0 (1 + lj1 r^2) + w r^9), q = p2a / p1a, w = 1 / p1a
     // (rows with p1a = p2a = 0 carry w = inf: the term is 0)
-    {
+    if constexpr (TERMS & GD_T_LJ) {
       const float r3 = r2 * rr;
       const float r9 = (r3 * r3) * r3;
       const float num = __builtin_fmaf(nq, r3, 1.0f);
@@ -183,6 +188,7 @@ __device__ __forceinline__ void gd_pair_one(
       // the iteration stayed live to its end (registers)
       asm volatile("" : "+v"(evdw));
     }
+    if constexpr (!(TERMS & GD_T_REST)) return;
     // Contact PMF (:88-91): pmf1 / (1 + exp2(x)), x = (6 - r/2)(r - pmf0) log2(e).
     // It is summed as pmf1 - pmf1 / (1 + exp2(-x)): the pmf1 of every pair of
     // the job is one constant added once per replica, and epmf collects only the
@@ -283,7 +289,7 @@ __device__ __forceinline__ void gd_load_rows(const GD_AS_CONST char *__restrict_
 
 // The LC chunk atoms against one point, rows given (held across the points of
 // one point type).
-template <int LC, int CLS>
+template <int LC, int CLS, int TERMS>
 __device__ __forceinline__ void gd_pair_atoms_rows(
     const GdPairConst &k, const float (&rw)[LC][GD_ROW], const GD_AS_CONST float *__restrict__ pspv,
     const int P, const int p, const float4 c, const float pele, const float phpp, const float pmf_a,
@@ -291,7 +297,7 @@ __device__ __forceinline__ void gd_pair_atoms_rows(
     float (&ele)[LC], float (&hpc)[LC], float &evdw, float &epmf, float &epsp, float &ehdb) {
 #pragma unroll
   for (int j = 0; j < LC; ++j) {
-    gd_pair_one<CLS>(k, rw[j], pspv, P, p, trow[j], c, pele, phpp, pmf_a, lx[j], ly[j], lz[j], ele[j],
+    gd_pair_one<CLS, TERMS>(k, rw[j], pspv, P, p, trow[j], c, pele, phpp, pmf_a, lx[j], ly[j], lz[j], ele[j],
                      hpc[j], evdw, epmf, epsp, ehdb);
     // one atom at a time: interleaving atoms raises register use for no gain
     // in issue rate
@@ -346,7 +352,7 @@ __device__ __forceinline__ void gd_pair_atoms_load(
 // type does and stay in scalar registers across the run; within a type the
 // order spreads the distances to the pocket evenly over the tiles, so every
 // tile holds the same mix of near and far points and waves cost the same.
-template <int LC, int CLS>
+template <int LC, int CLS, int TERMS>
 __device__ __forceinline__ void gd_pair_class(
     const GD_AS_CONST GdJob &J0, const int b, const unsigned pcoff, const GdPairConst &k, const float pmf_a,
     const float (&lx)[LC], const float (&ly)[LC], const float (&lz)[LC], const unsigned (&trow)[LC],
@@ -388,7 +394,7 @@ __device__ __forceinline__ void gd_pair_class(
         ty_cur = ty;
         gd_load_rows<LC>(ptab, trow, poff, *reinterpret_cast<float(*)[LC][GD_ROW]>(&rw));
       }
-      gd_pair_atoms_rows<LC, CLS>(k, *reinterpret_cast<float(*)[LC][GD_ROW]>(&rw), pspv, P, q, c,
+      gd_pair_atoms_rows<LC, CLS, TERMS>(k, *reinterpret_cast<float(*)[LC][GD_ROW]>(&rw), pspv, P, q, c,
                                   pa.x, pa.y, pmf_a, lx, ly, lz, trow, ele, hpc, evdw, epmf, epsp,
                                   ehdb);
     } else {
@@ -414,7 +420,7 @@ __device__ __forceinline__ void gd_pair_class(
 
 // The point loop of one item, class by class (padding atoms of a partial
 // chunk contribute exactly zero).
-template <int LC>
+template <int LC, int TERMS = GD_T_ALL>
 __device__ __forceinline__ void gd_pair_points(
     const GD_AS_CONST GdJob &J, const int b, const unsigned pc,
     const GdPairConst &k, const float (&lx)[LC], const float (&ly)[LC], const float (&lz)[LC],
@@ -423,10 +429,10 @@ __device__ __forceinline__ void gd_pair_points(
   // log2(e)/2 held in a VGPR: a VALU op reads at most one SGPR or literal
   float pmf_a;
   asm("v_mov_b32 %0, 0x3f38aa3b" : "=v"(pmf_a));  // log2(e) / 2
-  gd_pair_class<LC, 0>(J, b, pc, k, pmf_a, lx, ly, lz, trow, ele, hpc, evdw, epmf, epsp, ehdb);
-  gd_pair_class<LC, 1>(J, b, pc, k, pmf_a, lx, ly, lz, trow, ele, hpc, evdw, epmf, epsp, ehdb);
-  gd_pair_class<LC, 2>(J, b, pc, k, pmf_a, lx, ly, lz, trow, ele, hpc, evdw, epmf, epsp, ehdb);
-  gd_pair_class<LC, 3>(J, b, pc, k, pmf_a, lx, ly, lz, trow, ele, hpc, evdw, epmf, epsp, ehdb);
+  gd_pair_class<LC, 0, TERMS>(J, b, pc, k, pmf_a, lx, ly, lz, trow, ele, hpc, evdw, epmf, epsp, ehdb);
+  gd_pair_class<LC, 1, TERMS>(J, b, pc, k, pmf_a, lx, ly, lz, trow, ele, hpc, evdw, epmf, epsp, ehdb);
+  gd_pair_class<LC, 2, TERMS>(J, b, pc, k, pmf_a, lx, ly, lz, trow, ele, hpc, evdw, epmf, epsp, ehdb);
+  gd_pair_class<LC, 3, TERMS>(J, b, pc, k, pmf_a, lx, ly, lz, trow, ele, hpc, evdw, epmf, epsp, ehdb);
 }
 
 template <int LC, bool AG = false>
@@ -603,6 +609,157 @@ template __global__ void gd_pair_kernel<16>(const GdJob *, const GdItem *, int, 
 template __global__ void gd_pair_kernel_wq<4>(const GdJob *, const GdItem *, int, int *);
 template __global__ void gd_pair_kernel_wq<8>(const GdJob *, const GdItem *, int, int *);
 template __global__ void gd_pair_kernel_wq<16>(const GdJob *, const GdItem *, int, int *);
+
+// ---------------------------------------------------------------------------
+// Pair kernel for launches that leave most of the chip idle: the sums of
+// gd_pair_item<4> in its order (the results are the same bits), with an item on
+// three CUs.  Three groups of GD_GROUP waves per item: one takes the tiles' KDE and
+// MCS shares, one the pairs' Lennard-Jones terms and one their other terms.  In one
+// group they run after each other on the SIMDs of one CU, bound by their issue,
+// while other CUs have nothing to do (one pose, 344 points, 34 atoms, 27 items: 8.4
+// us of pairs, 9.6 of anchors and 1 of MCS rows in 20.6 us of a group; in three the
+// longest takes 10.6.  25 replicas, 1,200 points, 24 atoms, 90 items: 21.1 -> 19.1
+// us a step).  Measured and not taken: 16 waves in one group (10% less than here),
+// four anchors or atoms side by side in one wave and rows or anchors held across the
+// lanes (v_readlane; slower than gd_pair_kernel): what is short here is issue, not
+// independent work.
+template <int ROLE>
+__device__ __forceinline__ void gd_pair_item_split(const GdJob *__restrict__ jobs, const GdItem it, const int lane,
+                                                   const int wave, float (*__restrict__ red)[GD_NLIN + 4][64]) {
+  const GD_AS_CONST GdJob &J = gd_c(jobs)[it.job];
+  const int Rp = J.Rp, L = J.L, nP = J.nP;
+  const int b = it.b * GD_GROUP + wave, r = it.rb + lane;
+  const int l0 = it.a * 4, nl = min(4, L - l0);
+  const GD_AS_CONST GdAtom *__restrict__ atoms = gd_c(J.atoms);
+  const GD_AS_GLOBAL float *__restrict__ coords = gd_g((const float *)J.coords);
+  float lx[4], ly[4], lz[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int l = l0 + min(j, nl - 1);
+    lx[j] = coords[(size_t)(3 * l + 0) * Rp + r];
+    ly[j] = coords[(size_t)(3 * l + 1) * Rp + r];
+    lz[j] = coords[(size_t)(3 * l + 2) * Rp + r];
+  }
+  const int nG = J.nG;
+  const size_t nS = (size_t)J.nL * nG;
+  const int slot = it.a * nG + it.b;
+  GD_AS_GLOBAL float *__restrict__ pl = gd_g(J.part_lin);
+  if constexpr (ROLE != GD_T_KDE) {
+    float ele[4], hpc[4];
+    unsigned trow[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      trow[j] = (unsigned)atoms[l0 + j].tidx;
+      ele[j] = hpc[j] = 0.0f;
+    }
+    const unsigned pc = (unsigned)gd_g(J.prti)[r] * (unsigned)J.P * 16u;
+    GdPairConst k;
+    k.lj0 = J.lj0;
+    k.lj01 = J.lj0 * J.lj1;
+    const float el1 = J.el1;
+    k.e0 = J.el0 * el1;
+    k.e2 = J.a1 * el1 * el1 * el1;
+    k.e3 = J.b1 * el1 * el1 * el1 * el1;
+    k.inv_el1 = J.inv_el1;
+    float evdw = 0.0f, epmf = 0.0f, epsp = 0.0f, ehdb = 0.0f;
+    gd_pair_points<4, ROLE>(J, b, pc, k, lx, ly, lz, trow, ele, hpc, evdw, epmf, epsp, ehdb);
+    if constexpr (ROLE == GD_T_LJ) {
+      red[wave][0][lane] = evdw;
+    } else {
+      float eele = 0.0f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) eele = __builtin_fmaf(atoms[l0 + j].q, ele[j], eele);
+      eele *= k.inv_el1;
+      red[wave][1][lane] = eele;
+      red[wave][2][lane] = epmf;
+      red[wave][3][lane] = epsp;
+      red[wave][4][lane] = ehdb;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) red[wave][GD_NLIN + j][lane] = hpc[j];
+    }
+  } else {
+    // the shares of gd_pair_item
+    const GD_AS_CONST float4 *__restrict__ kde = gd_c(J.kde);
+    const float inv_np = 1.0f / (float)nP, kde2l = J.kde2l;
+    auto gauss = [&](const float4 kp, int j) {
+      const float dx = lx[j] - kp.x, dy = ly[j] - kp.y, dz = lz[j] - kp.z;
+      const float d2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
+      return gd_exp2(kde2l * d2);
+    };
+    float ekde = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const GdAtom at = atoms[l0 + j];
+      const int nb = at.kde_e - at.kde_b;
+      const int k0 = at.kde_b + gd_uniform((int)((float)(nb * b) * inv_np));
+      const int k1 = b + 1 == nP ? at.kde_e : at.kde_b + gd_uniform((int)((float)(nb * (b + 1)) * inv_np));
+      float s = 0.0f;
+      int i = k0;
+#pragma unroll 1
+      for (; i + 4 <= k1; i += 4) {  // four anchors to a load, added in order
+        const float4 a0 = kde[i], a1 = kde[i + 1], a2 = kde[i + 2], a3 = kde[i + 3];
+        const float e0 = gauss(a0, j), e1 = gauss(a1, j), e2 = gauss(a2, j), e3 = gauss(a3, j);
+        s = (((s + e0) + e1) + e2) + e3;
+      }
+#pragma unroll 1
+      for (; i < k1; ++i) s += gauss(kde[i], j);
+      ekde = __builtin_fmaf(s, at.kde_inv_n, ekde);
+    }
+    red[wave][5][lane] = ekde;
+    const int M = J.M, nL = J.nL;
+    const GD_AS_CONST float4 *__restrict__ mcs = gd_c(J.mcs);
+    GD_AS_GLOBAL float *__restrict__ pm = gd_g(J.part_mcs);
+    for (int m = b; m < M; m += nP) {
+      float d = 0.0f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float4 t = mcs[(size_t)m * J.Ls + l0 + j];
+        if (t.w != 0.0f) {
+          const float dx = lx[j] - t.x, dy = ly[j] - t.y, dz = lz[j] - t.z;
+          d += __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
+        }
+      }
+      pm[((size_t)m * nL + it.a) * Rp + r] = d;
+    }
+  }
+  __syncthreads();
+  // the group's sums over its tiles, a value to a wave: ele, pmf, psp, H-bond and
+  // the atoms' hpc, or the one of the other roles
+  GD_AS_GLOBAL float *__restrict__ ph = gd_g(J.part_hpc);
+  const int q = ROLE == GD_T_LJ ? 0 : ROLE == GD_T_KDE ? 5 : wave < 4 ? 1 + wave : GD_NLIN + wave - 4;
+  if (ROLE != GD_T_REST && wave != 0) return;
+  float v = red[0][q][lane];
+#pragma unroll
+  for (int w = 1; w < GD_GROUP; ++w) v += red[w][q][lane];
+  if (q < GD_NLIN)
+    pl[((size_t)q * nS + slot) * Rp + r] = v;
+  else if (q - GD_NLIN < nl)
+    ph[((size_t)(l0 + q - GD_NLIN) * nG + it.b) * Rp + r] = v;
+}
+
+// gd_pair_kernel's arguments, three groups to an item.
+__global__ __launch_bounds__(64 * GD_GROUP) void gd_pair_kernel_split(const GdJob *__restrict__ jobs,
+                                                                       const GdItem *__restrict__ items,
+                                                                       int n_items, int nb, int nb_list) {
+  __shared__ float red[GD_GROUP][GD_NLIN + 4][64];
+  const int role = gd_uniform((int)blockIdx.y), iid = gd_uniform((int)blockIdx.x);
+  if (iid >= n_items) return;
+  GdItem it;
+  if (nb > 0) {
+    const int k = gd_uniform(iid / nb);
+    it = gd_c(items)[(size_t)k * nb_list];
+    it.rb = 64 * (iid - k * nb);
+  } else {
+    it = gd_c(items)[iid];
+  }
+  const int lane = threadIdx.x & 63, wave = gd_uniform((int)(threadIdx.x >> 6));
+  if (role == 0)
+    gd_pair_item_split<GD_T_KDE>(jobs, it, lane, wave, red);
+  else if (role == 1)
+    gd_pair_item_split<GD_T_REST>(jobs, it, lane, wave, red);
+  else
+    gd_pair_item_split<GD_T_LJ>(jobs, it, lane, wave, red);
+}
 
 // ---------------------------------------------------------------------------
 // Ligand transform of one replica's proposal (kernel_cpp_montecarlo_soa.C:

@@ -32,6 +32,7 @@
 // kernels (gd_kernels.hip)
 template <int LC>
 __global__ void gd_pair_kernel(const GdJob *, const GdItem *, int, int, int);
+__global__ void gd_pair_kernel_split(const GdJob *, const GdItem *, int, int, int);
 __global__ void gd_eval_setup_kernel(const GdJob, GdJob *, const int *, const float *, int);
 __global__ void gd_reduce_kernel(const GdJob *, const GdBlock *);
 __global__ void gd_finish_kernel(const GdJob *, const GdBlock *, int, int, const int *, int *);
@@ -893,6 +894,17 @@ gd_status launch_pair(int lc, const GdJob *d_jobs, const GdItem *d_items, int n_
                       hipStream_t s, int nb, int nb_list) {
   if (n_items <= 0) return GD_OK;
   const dim3 grid(n_items), block(64 * GD_GROUP);  // one group per item
+  // At most an item to a CU: three groups to an item (gd_pair_kernel_split), which
+  // run beside each other.  From about 1.3 items a CU on its repeated work costs more
+  // than it gains.  An evaluation of poses with the split kernel / with one group an
+  // item: 27 items 46.7 / 59.4 us, 90 items 40.0 / 42.0, 180 items 43.9 / 45.4, 240
+  // items 49.0 / 49.3, 280 items 74.6 / 77.1, 420 items 99.4 / 83.3, 540 items 55.8 /
+  // 53.1 (points and anchors per item differ).
+  if (lc == 4 && n_items <= n_cu()) {
+    hipLaunchKernelGGL(gd_pair_kernel_split, dim3(n_items, 3), block, 0, s, d_jobs, d_items, n_items, nb, nb_list);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? GD_OK : hip_fail(e, "pair kernel launch");
+  }
   switch (lc) {
     case 4:
       hipLaunchKernelGGL(gd_pair_kernel<4>, grid, block, 0, s, d_jobs, d_items, n_items, nb, nb_list);
