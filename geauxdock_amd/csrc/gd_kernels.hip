@@ -767,12 +767,9 @@ __global__ __launch_bounds__(64 * GD_GROUP) void gd_pair_kernel_split(const GdJo
 // Every product of the rotation is rounded on its own (no contraction), and
 // the transform below is one explicit FMA chain, so that every kernel that
 // transforms a pose (transform, finish, swap) gives the same bits for it.
-__device__ __forceinline__ void gd_rotation(const float m[6], float R[9]) {
+__device__ __forceinline__ void gd_rotation_of(const float s[3], const float c[3], float R[9]) {
 #pragma clang fp contract(off)
-  float s1, c1, s2, c2, s3, c3;
-  sincosf(m[3], &s1, &c1);
-  sincosf(m[4], &s2, &c2);
-  sincosf(m[5], &s3, &c3);
+  const float s1 = s[0], c1 = c[0], s2 = s[1], c2 = c[1], s3 = s[2], c3 = c[2];
   R[0] = c1 * c2;
   R[1] = c1 * s2 * s3 - c3 * s1;
   R[2] = s1 * s3 + c1 * c3 * s2;
@@ -782,6 +779,12 @@ __device__ __forceinline__ void gd_rotation(const float m[6], float R[9]) {
   R[6] = -s2;
   R[7] = c2 * s3;
   R[8] = c2 * c3;
+}
+__device__ __forceinline__ void gd_rotation(const float m[6], float R[9]) {
+  float s[3], c[3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) sincosf(m[3 + i], &s[i], &c[i]);
+  gd_rotation_of(s, c, R);
 }
 
 // The finish, transform and move code reads the job struct through the
@@ -819,36 +822,58 @@ __device__ __forceinline__ void gd_transform_atoms(GdJobC &J, int r, const float
 // protein conformer) and pose [cnt][6] are host memory, read over the link once
 // and in order; the job struct of the evaluation comes with the launch and the
 // first group stores it for the kernels that follow.  Padding lanes: conformer 0
-// at the zero pose.  One group of four waves per 64 lanes.
-__global__ __launch_bounds__(256) void gd_eval_setup_kernel(const GdJob job, GdJob *__restrict__ d_job,
-                                                             const int *__restrict__ conf,
-                                                             const float *__restrict__ pose, int cnt) {
+// at the zero pose.  One group of GD_SW waves per 64 lanes.  Its time is a chain of
+// latencies -- the poses over the link, their sines, the conformers' atoms, the
+// coordinates out -- so each link of it is taken once: an input word to a thread, an
+// angle to a wave, and up to GD_SA atoms of a wave loaded before the first is used
+// (with four waves that took the atoms one after the other 12.3 us for 880 poses of
+// 80 atoms, 8.6 for 1,760 of 40).
+#define GD_SW 16
+#define GD_SA 5
+__global__ __launch_bounds__(64 * GD_SW) void gd_eval_setup_kernel(const GdJob job, GdJob *__restrict__ d_job,
+                                                                   const int *__restrict__ conf,
+                                                                   const float *__restrict__ pose, int cnt) {
   (void)job;
   __shared__ int s_conf[2 * 64];
-  __shared__ float s_pose[6 * 64];
+  __shared__ float s_pose[6 * 64], s_sin[3][64], s_cos[3][64];
   GdJobC &J = *(GdJobC *)__builtin_amdgcn_kernarg_segment_ptr();
-  const int rb = 64 * (int)blockIdx.x, n = min(64, cnt - rb);
-  for (int k = threadIdx.x; k < 6 * 64; k += 256) {
+  const int rb = 64 * (int)blockIdx.x, n = min(64, cnt - rb), k = threadIdx.x;
+  if (k < 6 * 64)
     s_pose[k] = k < 6 * n ? pose[(size_t)6 * rb + k] : 0.0f;
-    if (k < 2 * 64) s_conf[k] = k < 2 * n ? conf[(size_t)2 * rb + k] : 0;
-  }
-  if (blockIdx.x == 0)
-    for (int k = threadIdx.x; k < (int)(sizeof(GdJob) / 4); k += 256)
-      ((unsigned *)d_job)[k] = ((const GD_AS_CONST unsigned *)&J)[k];
+  else if (k < 8 * 64)
+    s_conf[k - 6 * 64] = k - 6 * 64 < 2 * n ? conf[(size_t)2 * rb + k - 6 * 64] : 0;
+  else if (blockIdx.x == 0)
+    for (int q = k - 8 * 64; q < (int)(sizeof(GdJob) / 4); q += 64 * GD_SW - 8 * 64)
+      ((unsigned *)d_job)[q] = ((const GD_AS_CONST unsigned *)&J)[q];
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = gd_uniform((int)(threadIdx.x >> 6));
-  const int r = rb + lane, lig = s_conf[2 * lane];
-  float m[6];
-  for (int i = 0; i < 6; ++i) m[i] = s_pose[6 * lane + i];
-  if (wave == 0) {
+  const int r = rb + lane, lig = s_conf[2 * lane], L = J.L, Rp = J.Rp;
+  const GD_AS_GLOBAL float4 *lc = gd_g(J.lig0) + (size_t)lig * L;
+  float4 a[GD_SA];
+#pragma unroll
+  for (int q = 0; q < GD_SA; ++q) a[q] = lc[min(wave + q * GD_SW, L - 1)];
+  if (wave < 3) {
+    float sn, cs;
+    sincosf(s_pose[6 * lane + 3 + wave], &sn, &cs);
+    s_sin[wave][lane] = sn;
+    s_cos[wave][lane] = cs;
+  } else if (wave == 3) {
     gd_g(J.ligi)[r] = lig;
     gd_g(J.prti)[r] = s_conf[2 * lane + 1];
-    for (int i = 0; i < 6; ++i) gd_g(J.prop)[(size_t)i * J.Rp + r] = m[i];
+    for (int i = 0; i < 6; ++i) gd_g(J.prop)[(size_t)i * Rp + r] = s_pose[6 * lane + i];
   }
+  __syncthreads();
+  const float sn[3] = {s_sin[0][lane], s_sin[1][lane], s_sin[2][lane]};
+  const float cs[3] = {s_cos[0][lane], s_cos[1][lane], s_cos[2][lane]};
   float R[9];
-  gd_rotation(m, R);
-  const float t[3] = {m[0] + J.center[0], m[1] + J.center[1], m[2] + J.center[2]};
-  gd_transform_lig(J, r, lig, R, t, wave, 4);
+  gd_rotation_of(sn, cs, R);
+  const float t[3] = {s_pose[6 * lane] + J.center[0], s_pose[6 * lane + 1] + J.center[1],
+                      s_pose[6 * lane + 2] + J.center[2]};
+  GD_AS_GLOBAL float *co = gd_g(J.coords);
+#pragma unroll
+  for (int q = 0; q < GD_SA; ++q)
+    if (wave + q * GD_SW < L) gd_put_atom(co, Rp, r, wave + q * GD_SW, R, t, a[q]);
+  for (int l = wave + GD_SA * GD_SW; l < L; l += GD_SW) gd_put_atom(co, Rp, r, l, R, t, lc[l]);
 }
 
 // ---------------------------------------------------------------------------

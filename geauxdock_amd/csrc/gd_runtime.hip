@@ -1251,7 +1251,7 @@ gd_status eval_pass(gd_job *j, const EvalBufs &b, int cnt, const int *conf, cons
   x.record = 0;
   std::memcpy(h_conf, conf, (size_t)cnt * 2 * sizeof(int));
   std::memcpy(h_pose, pose, (size_t)cnt * 6 * sizeof(float));
-  hipLaunchKernelGGL(gd_eval_setup_kernel, dim3(nb), dim3(256), 0, s, x, b.job, (const int *)h_conf,
+  hipLaunchKernelGGL(gd_eval_setup_kernel, dim3(nb), dim3(1024), 0, s, x, b.job, (const int *)h_conf,
                      (const float *)h_pose, cnt);
   hipError_t e = hipGetLastError();
   gd_status st = e == hipSuccess ? GD_OK : hip_fail(e, "eval setup kernel launch");
