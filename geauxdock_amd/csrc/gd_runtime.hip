@@ -983,17 +983,29 @@ void ChainList::shape(const std::vector<const GdJob *> &jobs) {
 // most): jobs whose single step is a sizeable part of that (10^11 pairs, 50 ms)
 // gain nothing from it and are stepped by launches.  So are jobs of one block,
 // where a step is one chain of latencies and the launches are the shorter one
-// (25 replicas, 24 atoms, 1,200 points: 19.9 us a step against 21.6; 40 atoms,
-// 3,000 points: 25.8 against 29.2), and of two blocks with many items, which the
-// 8 finishers of a block read more slowly than the reduce launch's 16 groups (105
-// replicas, 80 atoms, 9,000 points, 2,840 items: 91 against 111; with 1,480: 82
-// by launches, 76 here).
+// (25 replicas, 24 atoms, 1,200 points: 19.1 us a step against 21.6), and of two
+// blocks with many items, which the 8 finishers of a block read more slowly than
+// the reduce launch's 16 groups (105 replicas, 80 atoms, 9,000 points, 2,840 items:
+// 91 against 111).
 int chain_max_steps(const ChainList &c) {
   if (c.n_blocks < 2 || (c.n_blocks == 2 && c.n_items > 2048) || c.step_pairs > 1e11) return 0;
   const double by_time = 1e12 / std::max(1.0, c.step_pairs);
   const double by_count = (double)(1 << 22) / ((double)c.n_entries * c.per_entry);
   const int n = (int)std::min({(double)c.cap_steps, by_time, by_count});
   return n >= 2 ? n : 0;  // the first launch takes the initial pass and a step
+}
+
+// A plain run of few items is stepped by launches on one stream: a stream of its own
+// for each half of the blocks leaves too little in a launch, and where the process's
+// streams share a hardware queue costs twice the launches.  The line lies where the
+// stepping kernel becomes the shorter (us a step, one stream / stepping kernel): two
+// blocks 19.3 / 24.4 (120 items), 29.9 / 35.2 (480), 46.3 / 55.4 (1,110), 53.4 / 64.1
+// (1,650); four blocks 23.7 / 27.4 (96), 24.1 / 24.8 (360), 30.0 / 31.5 (512), 34.4 /
+// 34.3 (720); seven blocks 20.9 / 24.5 (224), 30.5 / 29.1 (420).  An item is the
+// pairs of 64 replicas, 4 atoms and 8 tiles of 10 to 60 points here.
+static bool step_by_one_stream(const ChainList &c) {
+  const int cu = g_cu > 0 ? g_cu : 256;
+  return c.n_items <= (c.n_blocks <= 2 ? 8 * cu : c.n_blocks <= 4 ? 2 * cu : cu);
 }
 
 // One run at a time uses the stepping kernel: groups of two such launches that
@@ -1635,12 +1647,14 @@ static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
     return launch_pair(g.lc, j->d_job, j->d_items, j->n_items, s);
   };
   // the stepping kernel takes the steps between exchange points and dump ends
-  // in one launch; a job whose streams were set, or with wide ligand chunks, is
-  // stepped by launches
+  // in one launch; a job whose streams were set, with wide ligand chunks, or of few
+  // items is stepped by launches
   int chain_max = 0;
-  if (chain && !j->by_launches && g.lc == 4) {
+  bool few = false;
+  if (!j->by_launches && g.lc == 4) {
     j->chain.shape({&g});
-    chain_max = chain_max_steps(j->chain);
+    few = step_by_one_stream(j->chain);
+    chain_max = chain && !few ? chain_max_steps(j->chain) : 0;
     if (chain_max > 0 && chain_make(j) != GD_OK) {  // no memory for its lists
       (void)hipGetLastError();
       chain_max = 0;
@@ -1665,7 +1679,7 @@ static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
   // parts' pair work.  Between exchange points the parts share nothing; they
   // join for every exchange point (which spans the whole job) and at dump ends.
   const int np = j->n_parts;
-  bool multi = chain_max == 0 && np >= 2;
+  bool multi = chain_max == 0 && np >= 2 && !few;
   for (int k = 0; k < np; ++k) multi = multi && j->nb_part[k] > 0;
   hipStream_t ps[gd_job::kMaxParts] = {s};
   hipEvent_t ev_fork = nullptr, ev_join[gd_job::kMaxParts] = {};

@@ -276,8 +276,9 @@ typedef struct {
 gd_status gd_tiling_get(const gd_job *job, gd_tiling *t);
 /* By default gd_dock takes the steps of a job of two or more 64-replica blocks
  * in launches of the stepping kernel, which run from one exchange point or dump
- * end to the next; other jobs, and runs that overlap another run's stepping
- * kernel, take a pair, a reduce and a finish launch for each step.
+ * end to the next; jobs of one block or of few work items a step, and runs that
+ * overlap another run's stepping kernel, take a pair, a reduce and a finish launch
+ * for each step.
  * gd_job_set_streams has the job stepped by those launches from then on, on 1
  * to 4 streams (default 2): with n, each steps one of n contiguous parts of the
  * replica blocks between exchange points, so one part's reduce and finish
