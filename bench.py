@@ -244,7 +244,7 @@ def c1_extra():
             "reference_shape": {"jobs_per_s": 1.0 / t_ref, "replica_steps_per_s": job.n_rep * 3000 / t_ref,
                                 "shape": "steps_per_dump 200, blocking record copy after each dump; "
                                          "timed from the host complex to results"},
-            "roofline": roofline(flops, pair_ms, "gd_pair_kernel<%d>" % lc,
+            "roofline": roofline(flops, pair_ms, "gd_pair_kernel_split" if lc == 4 else "gd_pair_kernel<%d>" % lc,
                                  launches_timed=st.n_pair_launch, prt_pairs_per_launch=pairs,
                                  note="25 replicas are one 64-lane block: the launch fills a "
                                       "few CUs of 256"),

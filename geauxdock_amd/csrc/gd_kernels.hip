@@ -9,6 +9,8 @@
 //                    attributes, force-field rows, KDE anchors and MCS targets
 //                    are wave-uniform scalar loads and the inner loop is pure
 //                    FP32 VALU on ligand coordinates held in VGPRs.
+//                    (gd_pair_kernel_split: three groups per item where the
+//                    items are few.)
 //   gd_reduce_kernel 16 work groups per 64-replica block: sum the partial
 //                    sums and apply the non-linear per-atom (hpc) and per-row
 //                    (MCS) terms; one slice of 8 values per group.
