@@ -343,12 +343,13 @@ gd_status batch_run(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, gd_repl
   KTimer tp;
   const auto t0 = std::chrono::steady_clock::now();
   // the stepping kernel takes the steps up to the next exchange point or end of
-  // any job in one launch (256 jobs of 25 replicas and a screen of large ones are
-  // in the figures of gd_chain_kernel); the initial pass goes with the first
+  // any job in one launch.  The initial pass goes with the first, which takes every
+  // job of the list; with a job of no steps among them, which leaves the lists before
+  // it, the pass is launches of its own
   bool init = step_ok && B.chain_max > 0;
+  for (int k = 0; k < n_jobs; ++k) init = init && mc[k].steps_total > 0;
   int chain_steps = 0;
   if ((st = init ? batch_start(B, s) : batch_init(B, lc, grid, s)) != GD_OK) return st;
-  if (init && steps_max == 0) st = launch_chain(B.chain, B.d_jobs, 0, 1, true, s);
 
   // Segments of identical shape are captured once into a HIP graph and
   // replayed with the base step in device memory (no memset nodes).
