@@ -135,6 +135,8 @@ PROTOTYPES = {
     "gd_batch_dock": (C.c_int, [C.POINTER(_vp), C.c_int, C.POINTER(gd_mc_param),
                                 C.POINTER(gd_replica_out), C.POINTER(gd_stats)]),
     "gd_tiling_get": (C.c_int, [_vp, C.POINTER(gd_tiling)]),
+    "gd_stepping_shape": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int),
+                                    C.POINTER(C.c_int)]),
     "gd_job_set_streams": (C.c_int, [_vp, C.c_int]),
     "gd_job_set_step_wait": (C.c_int, [_vp, C.c_double]),
     "gd_server_set_step_wait": (C.c_int, [_vp, C.c_double]),

@@ -124,6 +124,7 @@ struct GdItem {           // one 4-wave work group of the pair kernel
 #define GD_SY_HEAD 96
 #define GD_SY_BLOCK 64
 #define GD_CHAIN_WAIT_S 2.0  // seconds until one wait of the stepping kernel gives up
+#define GD_CHAIN_LDS (27 << 10)  // LDS of a group, at most (gd_chain_kernel)
 
 struct GdChainBlock {     // one 64-replica block of the stepping kernel
   int job;

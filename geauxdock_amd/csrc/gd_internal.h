@@ -28,8 +28,10 @@ struct ChainList {
   int lds = 0;                          // LDS added to a group's, which bounds the groups of a CU
   double wait_s = GD_CHAIN_WAIT_S;      // bound of one wait in the kernel
   double step_pairs = 0;                // (atom, point) pairs of one step
-  // The host lists (items of each job, blocks) and the launch shape.
-  void shape(const std::vector<const GdJob *> &jobs);
+  // The host lists (items of each job, blocks) and the launch shape on a device of
+  // `cu` CUs (0: this one).
+  void shape(const std::vector<const GdJob *> &jobs, int cu = 0);
+  int slots = 0;                        // groups that such a device holds at a time
   size_t queue_bytes() const { return (size_t)n_entries * stride * cap_steps * sizeof(unsigned long long); }
 };
 }  // namespace gdr

@@ -1468,6 +1468,8 @@ union GdChainLds {
   };
 };
 
+static_assert(sizeof(GdChainLds<4>) + 64 <= GD_CHAIN_LDS, "ChainList::shape counts a CU's groups by it");
+
 typedef const GD_AS_CONST GdChain GdChainC;
 
 // The counters of block b of the launch's list.

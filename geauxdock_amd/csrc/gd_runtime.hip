@@ -948,17 +948,21 @@ size_t chain_sync_bytes(int n_blocks) {
 // leave slots free (220 replicas, 46 atoms, 4,001 points: 39.0 us a step, with 1
 // group 54.8, with 8 42.2; 1,760 replicas, 24 atoms, 1,200 points: 39.5, with 1
 // 49.2), then one, whose time the other blocks' items cover (1,760 replicas, 40
-// atoms, 3,000 points: 104.8 us, with 4 groups 108.2).  At most 64 finishers, each
-// then with several blocks.
+// atoms, 3,000 points: 104.8 us, with 4 groups 108.2).  At most 64 teams, each then
+// with several blocks.  Finishers hold their slots for a whole launch, and while some
+// of them wait for one no worker of the launch runs: they are at most a quarter of
+// what the device holds (256 of 1,024 groups on 256 CUs), so that the finishers of
+// three processes leave room for workers.
 // Groups of a CU: where the items of a step are fewer than the slots, added LDS
 // keeps a CU from taking four groups while others have none, and keeps groups
 // that only wait from being resident: 128 replicas, 40 atoms, 9,000 points (400
 // items): 50.2 us a step with one group to a CU, 62.9 with four; 440 replicas, 20
-// atoms, 9,000 points (420): 65.9 with two, 70.4 with four.
+// atoms, 9,000 points (420): 65.9 with two, 70.4 with four.  Less is added where
+// the finishers would be over their quarter.
 // Queue entries: blocks of one job are eight entries each, on lines of their own
 // where there are few blocks (waiting workers then poll different lines); in
 // longer lists an entry is 8 items.  The queue holds up to 1 MB of them.
-void ChainList::shape(const std::vector<const GdJob *> &jobs) {
+void ChainList::shape(const std::vector<const GdJob *> &jobs, int cu) {
   n_blocks = n_items = n_entries = 0;
   step_pairs = 0.0;
   int most = 1;
@@ -973,10 +977,19 @@ void ChainList::shape(const std::vector<const GdJob *> &jobs) {
   stride = n_blocks <= 8 ? 16 : 1;
   cap_steps = (int)std::max(2.0, std::min(1024.0, (double)(1 << 17) / ((double)n_entries * stride)));
   n_teams = std::min(n_blocks, 64);
-  const int cu = g_cu > 0 ? g_cu : 256;
+  if (cu <= 0) cu = g_cu > 0 ? g_cu : 256;
   team = n_blocks <= 2 ? 8 : n_blocks <= 8 || n_items <= 6 * cu ? 4 : 1;
   const int groups = n_items + 2 * n_teams * team;
-  lds = groups <= 7 * cu / 4 ? 60 << 10 : groups <= 4 * cu ? 28 << 10 : groups <= 6 * cu ? 14 << 10 : 0;
+  static const int added[] = {60 << 10, 28 << 10, 14 << 10, 0};  // 1, 2, 3 and 4 groups to a CU
+  int k = groups <= 7 * cu / 4 ? 0 : groups <= 4 * cu ? 1 : groups <= 6 * cu ? 2 : 3;
+  while (k < 3 && 4 * n_teams * team > (k + 1) * cu) ++k;
+  lds = added[k];
+  slots = (k + 1) * cu;
+  static_assert((160 << 10) / (GD_CHAIN_LDS + (60 << 10)) == 1 && (160 << 10) / (GD_CHAIN_LDS + (28 << 10)) == 2 &&
+                    (160 << 10) / (GD_CHAIN_LDS + (14 << 10)) == 3 && (160 << 10) / GD_CHAIN_LDS >= 4,
+                "groups of a CU");
+  team = std::min(team, std::max(1, slots / 4 / n_teams));
+  n_teams = std::min(n_teams, std::max(1, slots / 4));
 }
 
 // One launch stays under about a second and 2^22 groups (2^32 work items is the
@@ -1449,6 +1462,21 @@ size_t gd_job_footprint(const gd_job_desc *d) { return footprint(d, false); }
 size_t gd_job_device_bytes(const gd_job *j) {
   if (!j) return 0;
   return j->bytes + j->part_bytes + j->lists_bytes + j->chain_bytes + j->eval_bytes + j->rec_bytes + sizeof(GdJob);
+}
+
+gd_status gd_stepping_shape(int n_cu, int n_jobs, int n_rep, int lig_chunks, int tile_groups, int *finishers,
+                            int *slots) {
+  if (n_cu < 1 || n_jobs < 1 || n_rep < 1 || lig_chunks < 1 || tile_groups < 1 || !finishers || !slots)
+    return GD_ERR_ARG;
+  GdJob g;
+  std::memset(&g, 0, sizeof g);
+  g.Rp = (n_rep + 63) / 64 * 64;
+  g.nL = lig_chunks, g.nG = tile_groups;
+  gdr::ChainList c;
+  c.shape(std::vector<const GdJob *>(n_jobs, &g), n_cu);
+  *finishers = c.n_teams * c.team;
+  *slots = c.slots;
+  return GD_OK;
 }
 
 gd_status gd_tiling_get(const gd_job *j, gd_tiling *t) {

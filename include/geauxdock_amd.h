@@ -415,6 +415,12 @@ gd_status gd_host_job_free(gd_host_job *h);
 float gd_kabsch_rmsd(int n, const float *a_xyz, const float *b_xyz);
 
 /* ---- diagnostics (tests and measurement; no reference counterpart) ------ */
+/* Launch shape of the stepping kernel for n_jobs jobs of n_rep replicas, lig_chunks
+ * ligand chunks and tile_groups protein tile groups on a device of n_cu CUs: the
+ * work groups that stay for the whole launch, and those that the device holds at a
+ * time. */
+gd_status gd_stepping_shape(int n_cu, int n_jobs, int n_rep, int lig_chunks, int tile_groups, int *finishers,
+                            int *slots);
 /* Philox4x32-R of one counter block (known-answer tests). */
 void gd_philox(const uint32_t ctr[4], const uint32_t key[2], int rounds, uint32_t out[4]);
 /* Move increments as gd_dock draws them: inc[s][r][6] for replicas r < n_rep
