@@ -25,6 +25,7 @@ struct ChainList {
   int cap_steps = 0;                    // steps the queue holds
   int n_teams = 0, team = 0;            // finisher teams, groups of a team
   unsigned epoch = 0, steps = 0;        // launches and their steps since the counters were zero
+  bool stale = false;                   // a run did not end well: its counters are zeroed before they are used
   int lds = 0;                          // LDS added to a group's, which bounds the groups of a CU
   double wait_s = GD_CHAIN_WAIT_S;      // bound of one wait in the kernel
   double step_pairs = 0;                // (atom, point) pairs of one step

@@ -830,6 +830,7 @@ static gd_status chain_make(gd_job *j) {
   cl.d_sync = (unsigned *)(base + up(bi) + up(bb));
   cl.d_queue = (unsigned long long *)(base + up(bi) + up(bb) + up(bs));
   cl.epoch = cl.steps = 0;
+  cl.stale = false;
   if ((e = hipMemcpyAsync(base, items.data(), bi, hipMemcpyHostToDevice, j->stream)) != hipSuccess ||
       (e = hipMemcpyAsync(base + up(bi), blocks.data(), bb, hipMemcpyHostToDevice, j->stream)) != hipSuccess ||
       (e = hipMemsetAsync(cl.d_sync, 0, up(bs) + up(bq), j->stream)) != hipSuccess ||
@@ -1045,7 +1046,6 @@ gd_status launch_chain(ChainList &c, const GdJob *d_jobs, int step0, int n_steps
   a.epoch = ++c.epoch;
   a.n_entries = c.n_entries;
   a.steps_before = c.steps;
-  c.steps += (unsigned)n_steps;
   a.n_teams = c.n_teams;
   a.team = c.team;
   a.n_steps = n_steps;
@@ -1057,7 +1057,9 @@ gd_status launch_chain(ChainList &c, const GdJob *d_jobs, int step0, int n_steps
   const int grid = c.n_teams * c.team + c.n_entries * c.per_entry * n_steps;
   hipLaunchKernelGGL(gd_chain_kernel<4>, dim3(grid), dim3(64 * GD_GROUP), c.lds, s, a);
   const hipError_t e = hipGetLastError();
-  return e == hipSuccess ? GD_OK : hip_fail(e, "stepping kernel launch");
+  if (e != hipSuccess) return hip_fail(e, "stepping kernel launch");
+  c.steps += (unsigned)n_steps;  // the counters hold what was launched
+  return GD_OK;
 }
 
 gd_status launch_swap(int axis, const GdJob *d_jobs, const GdBlock *d_blocks, int n_blocks,
@@ -1748,6 +1750,15 @@ static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
     return r == hipSuccess ? GD_OK : hip_fail(r, "stream join");
   };
   const auto t0 = std::chrono::steady_clock::now();
+  if (chain_max > 0) {
+    ChainList &c = j->chain;
+    if (c.stale) {
+      if ((e = hipMemsetAsync(c.d_sync, 0, chain_sync_bytes(c.n_blocks), s)) != hipSuccess)
+        return hip_fail(e, "stepping kernel counters");
+      c.steps = 0;
+    }
+    c.stale = true;  // until this run has ended well
+  }
   // initial energies (MonteCarlo_d with s2max = 1)
   hipLaunchKernelGGL(gd_start_job_kernel, dim3(j->n_blocks), dim3(256), 0, s, g, j->d_job);
   if ((e = hipGetLastError()) != hipSuccess) st = hip_fail(e, "start kernel launch");
@@ -1870,12 +1881,8 @@ static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
     }
   }
   if (st == GD_OK && chain_max > 0) {
-    if (*res.fail) {
-      e = hipMemset(j->chain.d_sync, 0, chain_sync_bytes(j->chain.n_blocks));
-      if (e != hipSuccess) st = hip_fail(e, "stepping kernel counters");
-      j->chain.steps = 0;
-      *again = st == GD_OK;
-    }
+    *again = *res.fail != 0;
+    j->chain.stale = *again;
   }
   if (st == GD_OK && !*again && sink && !sink->blocking && pending >= 0) deliver(pending, pending & 1);
   if (st == GD_OK && timing) st = multi ? tspan.collect(np) : tp.collect();
