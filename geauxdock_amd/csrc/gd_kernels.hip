@@ -32,6 +32,7 @@
 
 #include "gd_device.h"
 #include "gd_rng.h"
+#include "gd_rules.h"
 
 #define GD_LOG2E 1.44269504088896340736f
 // Smallest float x with expf(x) > 0 in IEEE arithmetic with subnormals: the
@@ -1487,7 +1488,7 @@ __device__ __forceinline__ void gd_chain_push(GdChainC &c, const int b) {
                                 __HIP_MEMORY_SCOPE_AGENT) -
          c.steps_before * (unsigned)c.n_entries;
   at = (unsigned)gd_uniform((int)at);
-  if (at + (unsigned)n > (unsigned)(c.n_entries * c.n_steps)) return;  // after a launch that failed
+  if (!gd_queue_room(at, (unsigned)n, (unsigned)(c.n_entries * c.n_steps))) return;  // after a launch that failed
   for (int k = lane; k < n; k += 64)
     gd_st<true>(gd_g(c.queue) + (size_t)(at + k) * c.stride,
                 (unsigned long long)c.epoch << 32 | (unsigned)(b << 8 | k));
