@@ -63,6 +63,7 @@ gd_status hip_fail(hipError_t e, const char *what) {
   char buf[256];
   std::snprintf(buf, sizeof buf, "%s: %s", what, hipGetErrorString(e));
   set_error(buf);
+  (void)hipGetLastError();  // reported here: the runtime keeps it for the next check of a launch
   return GD_ERR_HIP;
 }
 
@@ -1055,8 +1056,11 @@ gd_status launch_chain(ChainList &c, const GdJob *d_jobs, int step0, int n_steps
   a.wait_ticks = (long long)(c.wait_s * 1e3 * g_wall_khz);
   // the finishers, then a worker group for each item of every step
   const int grid = c.n_teams * c.team + c.n_entries * c.per_entry * n_steps;
-  hipLaunchKernelGGL(gd_chain_kernel<4>, dim3(grid), dim3(64 * GD_GROUP), c.lds, s, a);
-  const hipError_t e = hipGetLastError();
+  void *args[] = {&a};
+  // by the launch's own status: an error that some earlier call left would have the
+  // counters miss a launch that runs
+  const hipError_t e =
+      hipLaunchKernel((const void *)gd_chain_kernel<4>, dim3(grid), dim3(64 * GD_GROUP), args, c.lds, s);
   if (e != hipSuccess) return hip_fail(e, "stepping kernel launch");
   c.steps += (unsigned)n_steps;  // the counters hold what was launched
   return GD_OK;
