@@ -1095,6 +1095,7 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
     if (act.empty()) break;
     if (s->dirty || (int)act.size() != s->lists.n_jobs || s->lists_stepping != turn.mine) {
       for (int q : act) jobs[q]->h.step0 = s->active[q]->step0;
+      s->dirty = true;  // until they are whole
       if ((st = s->lists.build(jobs, act, hs, turn.mine)) != GD_OK) return st;
       s->lists_stepping = turn.mine;
       s->dirty = false;
@@ -1110,7 +1111,10 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
         n = std::min(n, j->mc.steps_total - j->done_steps);
         if (spe > 0) n = std::min(n, spe - j->done_steps % spe);
       }
-      st = launch_chain(s->lists.chain, s->lists.d_jobs, s->launch_step, n, false, hs);
+      if ((st = launch_chain(s->lists.chain, s->lists.d_jobs, s->launch_step, n, false, hs)) != GD_OK) {
+        (void)hipStreamSynchronize(hs);
+        return st;  // the steps were not taken: the next call takes them
+      }
     }
     std::vector<int> round(act.size(), -1);
     for (int q = 0; q < (int)act.size(); ++q) {
@@ -1122,7 +1126,7 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
     xp.set(s->lists, round);
     const int grid = pair_grid(pair_waves_per_cu(s->lc)), last = s->launch_step + n - 1;
     if (!chain) st = batch_step(s->lists, s->lc, grid, last, nullptr, &xp, hs, nullptr);
-    else if (st == GD_OK && !xp.empty() && (st = exchange_upload(s->lists, xp, hs)) == GD_OK)
+    else if (!xp.empty() && (st = exchange_upload(s->lists, xp, hs)) == GD_OK)
       st = exchange_launch(s->lists, s->lc, grid, (int)xp.ex.size(), xp.axes, last, nullptr, hs);
     if (!xp.empty()) (void)hipStreamSynchronize(hs);  // exchange tables are reused next step
     s->launch_step += n;

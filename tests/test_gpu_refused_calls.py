@@ -29,3 +29,61 @@ for _ in range(2):
     same(want, out)
     assert st.n_pair_launch == 31, st.n_pair_launch
 """ % after)
+
+
+_SERVE = """
+jobs = [g.synth_complex(700 + 40 * k, 21 + k, 13, 5, 2, floor_temp=0.05, ceiling_temp=0.3, seed=k + 1, ene=ene)
+        for k in range(3)]
+mcs = [g.make_mc(40 + 9 * k, steps_per_exchange=7 + k, seed=3, job_id=k, axes=("temp", "lig")) for k in range(3)]
+
+def serve(refuse):
+    s = C.c_void_p()
+    cfg = abi.gd_server_config(hbm_budget=64 << 30, max_active=3, sweep_steps=13)
+    g.check(g.lib().gd_server_create(C.byref(cfg), C.byref(s)), "create")
+    outs = [g.host.ReplicaOut(j.n_rep) for j in jobs]
+    for j, mc, o in zip(jobs, mcs, outs):
+        t = C.c_int64()
+        g.check(g.lib().gd_server_submit(s, C.byref(j.desc), C.byref(mc), C.byref(o.c), C.byref(t)), "submit")
+    done = errors = 0
+    for k in range(40):
+        if k in refuse:
+            refuse[k]()
+        na, nd, n, res = C.c_int(), C.c_int(), C.c_int(), (abi.gd_job_result * 8)()
+        errors += g.lib().gd_server_step(s, C.byref(na), C.byref(nd)) != 0
+        shim.refuse_device_over(NONE)
+        g.lib().gd_server_results(s, res, 8, C.byref(n))
+        assert all(res[i].status == 0 for i in range(n.value))
+        done += n.value
+        if done == 3:
+            break
+    assert done == 3
+    g.lib().gd_server_destroy(s)
+    return outs, errors
+
+want, errors = serve({})
+assert errors == 0
+"""
+
+
+@pytest.mark.parametrize("after", [0, 7])
+def test_refused_sweep(tmp_path, after):
+    """The first or second stepping launch of a sweep (6 launches of an exchange point lie
+    between them) is refused: the call is an error, and the
+    next ones take the steps that it did not."""
+    hip_refuse.run(tmp_path, _SERVE + """
+got, errors = serve({1: lambda: shim.refuse_launch_after(%d)})
+assert errors == 1
+for a, b in zip(want, got):
+    same(a, b)
+""" % after)
+
+
+def test_refused_lists(tmp_path):
+    """No memory for the lists of a sweep whose jobs have changed: an error, and
+    the lists are made by the next call."""
+    hip_refuse.run(tmp_path, _SERVE + """
+got, errors = serve({k: lambda: shim.refuse_device_over(0) for k in range(1, 8)})
+assert errors >= 1
+for a, b in zip(want, got):
+    same(a, b)
+""")
