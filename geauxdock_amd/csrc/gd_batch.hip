@@ -69,6 +69,7 @@ struct BatchLists {
   void *mem = nullptr;
   ChainList chain;           // the same jobs for the stepping kernel
   int chain_max = 0;         // steps of one of its launches (0: step by launches)
+  bool suits = false, with_turn = false;  // the lists suit it; they were made with its turn
   double wait_s = GD_CHAIN_WAIT_S;  // bound of its waits (or a job's, if shorter)
   bool failed = false;       // it failed on lists that were rebuilt since
   void *qmem = nullptr;      // its counters, then its queue; grows only
@@ -109,9 +110,10 @@ struct BatchLists {
     chain.d_queue = (unsigned long long *)((char *)qmem + sync_bytes);
     return e == hipSuccess ? GD_OK : hip_fail(e, "stepping queue");
   }
-  // stepping: with the lists of the stepping kernel.
+  // turn: with the lists of the stepping kernel where they suit it and the turn is
+  // to be had (null: without).
   gd_status build(const std::vector<gd_job *> &jobs, const std::vector<int> &which,
-                  hipStream_t s, bool stepping) {
+                  hipStream_t s, Stepping *turn) {
     std::vector<GdJob> js;
     std::vector<GdItem> items;
     std::vector<GdBlock> blocks;
@@ -173,7 +175,10 @@ struct BatchLists {
     chain.shape(hs);
     chain.wait_s = wait_s;
     for (int k : which) chain.wait_s = std::min(chain.wait_s, jobs[k]->chain.wait_s);
-    chain_max = stepping ? chain_max_steps(chain) : 0;
+    chain_max = chain_max_steps(chain);
+    suits = chain_max > 0;
+    with_turn = suits && turn && turn->take();
+    if (!with_turn) chain_max = 0;
     if (chain_max > 0 && chain_memory(s) != GD_OK) {  // no memory for it
       (void)hipGetLastError();
       chain_max = 0;
@@ -337,8 +342,10 @@ gd_status batch_run(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, gd_repl
   // jobs run from launch step 0; a job whose steps are done leaves the lists
   std::vector<int> active(n_jobs);
   for (int k = 0; k < n_jobs; ++k) active[k] = k;
+  Stepping turn;
+  Stepping *const stepping = step_ok ? &turn : nullptr;
   BatchLists B;
-  if ((st = B.build(jobs, active, s, step_ok)) != GD_OK) return st;
+  if ((st = B.build(jobs, active, s, stepping)) != GD_OK) return st;
   const int grid = pair_grid(waves_override > 0 ? waves_override : pair_waves_per_cu(lc));
   KTimer tp;
   const auto t0 = std::chrono::steady_clock::now();
@@ -346,7 +353,7 @@ gd_status batch_run(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, gd_repl
   // any job in one launch.  The initial pass goes with the first, which takes every
   // job of the list; with a job of no steps among them, which leaves the lists before
   // it, the pass is launches of its own
-  bool init = step_ok && B.chain_max > 0;
+  bool init = B.chain_max > 0;
   for (int k = 0; k < n_jobs; ++k) init = init && mc[k].steps_total > 0;
   int chain_steps = 0;
   if ((st = init ? batch_start(B, s) : batch_init(B, lc, grid, s)) != GD_OK) return st;
@@ -372,7 +379,7 @@ gd_status batch_run(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, gd_repl
   std::vector<int> round;
   while (step < steps_max && st == GD_OK) {
     // graph path: whole segment, every job active, exchange point at its end
-    if (!(step_ok && B.chain_max > 0) && uniform && seg > 1 && step + seg <= steps_max && !stats) {
+    if (B.chain_max == 0 && uniform && seg > 1 && step + seg <= steps_max && !stats) {
       hipError_t e = hipMemcpyAsync(B.d_base, &step, sizeof(int), hipMemcpyHostToDevice, s);
       if (e != hipSuccess) {
         st = hip_fail(e, "hipMemcpyAsync base");
@@ -420,10 +427,10 @@ gd_status batch_run(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, gd_repl
       if (step < mc[k].steps_total) act.push_back(k);
     if (act.size() != (size_t)B.n_jobs) {
       // shrink the lists to the jobs still running; their step0 stays 0
-      if ((st = B.build(jobs, act, s, step_ok)) != GD_OK) break;
+      if ((st = B.build(jobs, act, s, stepping)) != GD_OK) break;
     }
     int n = 1;
-    const bool chain = step_ok && B.chain_max > 0;
+    const bool chain = B.chain_max > 0;
     if (chain) {
       n = B.chain_max - (init ? 1 : 0);
       for (int k : act) {
@@ -491,12 +498,8 @@ gd_status batch_run(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, gd_repl
 gd_status batch_dock_impl(gd_job **jobs, int n_jobs, const gd_mc_param *mc, gd_replica_out *out,
                           gd_stats *stats, int ptile_override, int waves_override) {
   bool again = false;
-  gd_status st;
-  {
-    // a sweep over persistent grids runs by launches
-    Stepping turn(waves_override <= 0);
-    st = batch_run(jobs, n_jobs, mc, out, stats, ptile_override, waves_override, turn.mine, &again);
-  }
+  // a sweep over persistent grids runs by launches
+  gd_status st = batch_run(jobs, n_jobs, mc, out, stats, ptile_override, waves_override, waves_override <= 0, &again);
   if (st == GD_OK && again) {
     again = false;
     st = batch_run(jobs, n_jobs, mc, out, stats, ptile_override, waves_override, false, &again);
@@ -711,7 +714,6 @@ struct gd_server {
   hipStream_t stream = nullptr;
   BatchLists lists;
   bool dirty = true;
-  bool lists_stepping = false;   // the lists were built with the stepping kernel's
   bool by_launches = false;      // a wait of the stepping kernel ran out of time
   int lc = kSharedLc;
   std::chrono::steady_clock::time_point t0;
@@ -1063,7 +1065,7 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
       nj.push_back(j->job);
     }
     BatchLists B;
-    st = B.build(nj, idx, hs, false);
+    st = B.build(nj, idx, hs, nullptr);
     if (st == GD_OK) st = batch_init(B, s->lc, pair_grid(pair_waves_per_cu(s->lc)), hs);
     if (st == GD_OK) {
       hipError_t e = hipStreamSynchronize(hs);
@@ -1084,7 +1086,8 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
   }
   // (3) advance every active job by up to sweep_steps (no lock held but smu:
   // submits and result queries proceed meanwhile)
-  Stepping turn(!s->by_launches);
+  Stepping turn;
+  Stepping *const stepping = s->by_launches ? nullptr : &turn;
   for (int k = 0; k < s->cfg.sweep_steps && st == GD_OK; ++k) {
     std::vector<int> act;
     std::vector<gd_job *> jobs;
@@ -1093,11 +1096,12 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
       if (s->active[q]->done_steps < s->active[q]->mc.steps_total && !s->active[q]->converged)
         act.push_back(q);
     if (act.empty()) break;
-    if (s->dirty || (int)act.size() != s->lists.n_jobs || s->lists_stepping != turn.mine) {
+    // made again also where the turn is to be had for lists that were made without it
+    if (s->dirty || (int)act.size() != s->lists.n_jobs ||
+        (stepping && s->lists.suits && turn.take() && !s->lists.with_turn)) {
       for (int q : act) jobs[q]->h.step0 = s->active[q]->step0;
       s->dirty = true;  // until they are whole
-      if ((st = s->lists.build(jobs, act, hs, turn.mine)) != GD_OK) return st;
-      s->lists_stepping = turn.mine;
+      if ((st = s->lists.build(jobs, act, hs, stepping)) != GD_OK) return st;
       s->dirty = false;
     }
     // by the stepping kernel up to the next exchange point or end of any job

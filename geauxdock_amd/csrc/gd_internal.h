@@ -169,12 +169,13 @@ gd_status launch_exchange(const GdJob *d_jobs, int round, hipStream_t s);  // of
 size_t chain_sync_bytes(int n_blocks);
 // Steps that one launch may take (0: this list is stepped by launches).
 int chain_max_steps(const ChainList &c);
-// The right to launch the stepping kernel, for as long as the object lives: one
-// run of the process at a time has it (see dock_impl).
+// The right to launch the stepping kernel, from take() on for as long as the object
+// lives: one run of the process at a time has it.
 struct Stepping {
-  bool mine;
-  explicit Stepping(bool wanted);
+  bool mine = false;
+  Stepping() = default;
   ~Stepping();
+  bool take();  // whether it is this run's
   Stepping(const Stepping &) = delete;
   Stepping &operator=(const Stepping &) = delete;
 };

@@ -1027,8 +1027,13 @@ static bool step_by_one_stream(const ChainList &c) {
 // wait for each other's slots could fill the device between them.  Runs that
 // overlap it step by launches, as does a run repeated because a wait ran out of
 // time (another process's launch can hold slots too): the same bits either way.
+// A run takes the turn once its lists suit the kernel, so that runs which do not use
+// it leave it to the others.
 static std::atomic<int> g_stepping{0};
-Stepping::Stepping(bool wanted) : mine(wanted && g_stepping.exchange(1) == 0) {}
+bool Stepping::take() {
+  if (!mine) mine = g_stepping.exchange(1) == 0;
+  return mine;
+}
 Stepping::~Stepping() {
   if (mine) g_stepping.store(0);
 }
@@ -1685,10 +1690,12 @@ static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
   // items is stepped by launches
   int chain_max = 0;
   bool few = false;
+  Stepping turn;
   if (!j->by_launches && g.lc == 4) {
     j->chain.shape({&g});
     few = step_by_one_stream(j->chain);
     chain_max = chain && !few ? chain_max_steps(j->chain) : 0;
+    if (chain_max > 0 && !turn.take()) chain_max = 0;
     if (chain_max > 0 && chain_make(j) != GD_OK) {  // no memory for its lists
       (void)hipGetLastError();
       chain_max = 0;
@@ -1919,11 +1926,7 @@ static gd_status dock_impl(gd_job *j, const gd_mc_param *mc, const RecSink *sink
                            gd_replica_out *out, gd_stats *stats) {
   int handed = 0;
   bool again = false;
-  gd_status st;
-  {
-    Stepping turn(true);
-    st = dock_run(j, mc, sink, out, stats, turn.mine, &handed, &again);
-  }
+  gd_status st = dock_run(j, mc, sink, out, stats, true, &handed, &again);
   if (st == GD_OK && again) {
     again = false;
     st = dock_run(j, mc, sink, out, stats, false, &handed, &again);
