@@ -87,12 +87,12 @@ struct gd_job {
   // the plain path's stepping parts: n_parts contiguous ranges of the blocks,
   // [b0_part[k], b0_part[k] + nb_part[k]), each with its items (the job's items
   // of those blocks, in the job's order) and a stream (part 0: the job's own)
-  static constexpr int kMaxParts = 4;
+  static constexpr int kMaxParts = 4, kDefaultStreams = 2;
   bool by_launches = false;  // step by launches on n_streams streams (gd_job_set_streams)
   GdItem *d_items_part[kMaxParts] = {};
   int n_items_part[kMaxParts] = {}, nb_part[kMaxParts] = {}, b0_part[kMaxParts] = {};
   int n_parts = 0;
-  int n_streams = 2;         // streams the plain path steps on (1 .. kMaxParts)
+  int n_streams = kDefaultStreams;  // streams the plain path steps on (1 .. kMaxParts)
   hipStream_t part_stream[kMaxParts] = {};
   gdr::ChainList chain;      // the stepping kernel's list, its queue and its counters
   // buffers of energy evaluations: a part of the arena for the lanes of up to Rp

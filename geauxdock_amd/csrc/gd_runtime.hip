@@ -1506,7 +1506,7 @@ gd_status gd_job_set_step_wait(gd_job *j, double seconds) {
 
 gd_status gd_job_set_streams(gd_job *j, int n_streams) {
   if (!j || n_streams < 1 || n_streams > gd_job::kMaxParts) return GD_ERR_ARG;
-  j->by_launches = true;
+  j->by_launches = n_streams != gd_job::kDefaultStreams;
   if (n_streams == j->n_streams) return GD_OK;
   const gd_status st = ensure_device();
   if (st != GD_OK) return st;

@@ -293,7 +293,8 @@ class DeviceJob:
         return t.atoms_per_lane, t.tile_points
 
     def set_streams(self, n):
-        """Step this job by launches, on 1 to 4 streams."""
+        """Streams of this job's runs: 2 (the default) has the library choose how it is
+        stepped; 1, 3 and 4 step it by launches on that many."""
         check(lib().gd_job_set_streams(self.h, n), "gd_job_set_streams")
 
     def set_step_wait(self, seconds):

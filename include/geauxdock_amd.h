@@ -274,13 +274,16 @@ typedef struct {
   int waves_per_cu;         /* persistent grid size per CU */
 } gd_tiling;
 gd_status gd_tiling_get(const gd_job *job, gd_tiling *t);
-/* By default gd_dock takes the steps of a job of two or more 64-replica blocks
+/* By default gd_dock takes the steps of a job of three or more 64-replica blocks
  * in launches of the stepping kernel, which run from one exchange point or dump
- * end to the next; jobs of one block or of few work items a step, and runs that
- * overlap another run's stepping kernel, take a pair, a reduce and a finish launch
- * for each step.
- * gd_job_set_streams has the job stepped by those launches from then on, on 1
- * to 4 streams (default 2): with n, each steps one of n contiguous parts of the
+ * end to the next; jobs of one or two blocks or of few work items a step, and runs
+ * that overlap another run's stepping kernel, take a pair, a reduce and a finish
+ * launch for each step.  (Batches and sweeps of a server use it from two blocks in
+ * all on.)
+ * gd_job_set_streams sets the streams of a job (1 to 4).  With 2, the default,
+ * the job is stepped as above, by launches on two streams where it steps by
+ * launches and has the items for them; with 1, 3 or 4 it is stepped by launches on
+ * that many from then on.  On n streams each steps one of n contiguous parts of the
  * replica blocks between exchange points, so one part's reduce and finish
  * kernels and launch tail overlap the other parts' pair work.  The results are
  * the same bits in all cases.  Waits for the job's stream (the parts' work

@@ -80,3 +80,18 @@ def test_large_runs_side_by_side(ene):
     _together([lambda k=k: run(k) for k in range(3)])
     for d in devs:
         d.close()
+
+
+def test_default_streams(ene):
+    """Two streams are the default: setting them changes nothing, and after another
+    number they bring the default back."""
+    dev = g.DeviceJob(g.synth_complex(4001, 46, 5, 11, 4, seed=2, ene=ene))
+    mc = g.make_mc(24, steps_per_exchange=20, seed=3)
+    want, st = dev.dock(mc)
+    assert st.n_pair_launch == 25
+    for n, launches in ((2, 25), (1, 2), (2, 25), (4, 8), (3, 6), (2, 25)):
+        dev.set_streams(n)
+        out, st = dev.dock(mc)
+        assert np.array_equal(out.energy, want.energy)
+        assert st.n_pair_launch == launches, (n, st.n_pair_launch)
+    dev.close()
