@@ -70,7 +70,7 @@ struct BatchLists {
   ChainList chain;           // the same jobs for the stepping kernel
   int chain_max = 0;         // steps of one of its launches (0: step by launches)
   bool suits = false, with_turn = false;  // the lists suit it; they were made with its turn
-  double wait_s = GD_CHAIN_WAIT_S;  // bound of its waits (or a job's, if shorter)
+  double wait_s = GD_CHAIN_WAIT_S;  // bound of its waits (in a batch a job's, if shorter)
   bool failed = false;       // it failed on lists that were rebuilt since
   void *qmem = nullptr;      // its counters, then its queue; grows only
   size_t sync_bytes = 0, queue_bytes = 0;
@@ -174,7 +174,6 @@ struct BatchLists {
     for (const GdJob &h : js) hs.push_back(&h);
     chain.shape(hs);
     chain.wait_s = wait_s;
-    for (int k : which) chain.wait_s = std::min(chain.wait_s, jobs[k]->chain.wait_s);
     chain_max = chain_max_steps(chain);
     suits = chain_max > 0;
     with_turn = suits && turn && turn->take();
@@ -194,6 +193,34 @@ struct BatchLists {
         (e = hipStreamSynchronize(s)) != hipSuccess)
       return hip_fail(e, "batch upload");
     return GD_OK;
+  }
+};
+
+// Device memory for the state that a batch or a server keeps (launch_keep).
+struct KeepArea {
+  unsigned *mem = nullptr;
+  size_t bytes = 0;
+  KeepArea() = default;
+  KeepArea(const KeepArea &) = delete;
+  KeepArea &operator=(const KeepArea &) = delete;
+  ~KeepArea() {
+    if (mem) (void)hipFree(mem);
+  }
+  // For lists of n_blocks, naming no step where it is new; what it held is gone if it grows.
+  gd_status make(int n_blocks, hipStream_t s) {
+    const size_t want = keep_bytes(n_blocks);
+    if (want <= bytes) return GD_OK;
+    if (mem) (void)hipFree(mem);
+    mem = nullptr;
+    bytes = 0;
+    hipError_t e = hipMalloc(&mem, want);
+    if (e != hipSuccess) {
+      mem = nullptr;
+      return hip_fail(e, "hipMalloc kept state");
+    }
+    bytes = want;
+    e = hipMemsetAsync(mem, 0, GD_KEEP_HEAD * sizeof(unsigned), s);
+    return e == hipSuccess ? GD_OK : hip_fail(e, "kept state");
   }
 };
 
@@ -317,9 +344,11 @@ gd_status batch_init(const BatchLists &B, int lc, int grid, hipStream_t s) {
 // Batched docking (gd_batch_dock); the overrides (> 0) replace the shared
 // tile size and the persistent grid's waves per CU (autotuner sweeps).  step_ok:
 // the stepping kernel may be used; *again: one of its waits ran out of time and
-// the batch is to be repeated without it.
+// the batch is to go on without it from MC step *from, the last one whose state was
+// kept (0: from the start).
 gd_status batch_run(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, gd_replica_out *out,
-                    gd_stats *stats, int ptile_override, int waves_override, bool step_ok, bool *again) {
+                    gd_stats *stats, int ptile_override, int waves_override, bool step_ok, KeepArea &keep,
+                    int *from, bool *again) {
   if (!jobs_in || n_jobs <= 0 || !mc) return GD_ERR_ARG;
   gd_status st = ensure_device();
   if (st != GD_OK) return st;
@@ -340,8 +369,9 @@ gd_status batch_run(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, gd_repl
     steps_max = std::max(steps_max, mc[k].steps_total);
   }
   // jobs run from launch step 0; a job whose steps are done leaves the lists
-  std::vector<int> active(n_jobs);
-  for (int k = 0; k < n_jobs; ++k) active[k] = k;
+  std::vector<int> active;
+  for (int k = 0; k < n_jobs; ++k)
+    if (*from == 0 || mc[k].steps_total > *from) active.push_back(k);
   Stepping turn;
   Stepping *const stepping = step_ok ? &turn : nullptr;
   BatchLists B;
@@ -356,7 +386,12 @@ gd_status batch_run(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, gd_repl
   bool init = B.chain_max > 0;
   for (int k = 0; k < n_jobs; ++k) init = init && mc[k].steps_total > 0;
   int chain_steps = 0;
-  if ((st = init ? batch_start(B, s) : batch_init(B, lc, grid, s)) != GD_OK) return st;
+  double since = 0.0;  // work since the state was kept
+  if (*from > 0)
+    st = launch_keep(true, B.d_jobs, B.d_blocks, B.n_blocks, keep.mem, nullptr, *from, s);
+  else
+    st = init ? batch_start(B, s) : batch_init(B, lc, grid, s);
+  if (st != GD_OK) return st;
 
   // Segments of identical shape are captured once into a HIP graph and
   // replayed with the base step in device memory (no memset nodes).
@@ -374,12 +409,12 @@ gd_status batch_run(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, gd_repl
     pair_evals += (double)g.R * g.L * g.P * (mc[k].steps_total + 1);
     rep_steps += (double)g.R * mc[k].steps_total;
   }
-  int step = 0;
+  int step = *from;
   ExchPoint xp;
   std::vector<int> round;
   while (step < steps_max && st == GD_OK) {
     // graph path: whole segment, every job active, exchange point at its end
-    if (B.chain_max == 0 && uniform && seg > 1 && step + seg <= steps_max && !stats) {
+    if (B.chain_max == 0 && uniform && seg > 1 && step % seg == 0 && step + seg <= steps_max && !stats) {
       hipError_t e = hipMemcpyAsync(B.d_base, &step, sizeof(int), hipMemcpyHostToDevice, s);
       if (e != hipSuccess) {
         st = hip_fail(e, "hipMemcpyAsync base");
@@ -438,6 +473,17 @@ gd_status batch_run(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, gd_repl
         n = std::min(n, mc[k].steps_total - step);
         if (spe > 0) n = std::min(n, spe - step % spe);
       }
+      if (since >= kKeepWork) {
+        since = 0.0;
+        if (keep.make(B.n_blocks, s) == GD_OK &&  // the lists only shrink
+            (st = launch_keep(false, B.d_jobs, B.d_blocks, B.n_blocks, keep.mem,
+                              (const unsigned *)B.qmem + GD_SY_FAILED, step, s)) != GD_OK)
+          break;
+      }
+      since += B.chain.work(n);
+      double wait = B.wait_s;
+      for (int k : act) wait = std::min(wait, jobs[k]->chain.wait_s.load());
+      B.chain.wait_s = wait;
       if (stats && (st = tp.begin(s)) != GD_OK) break;
       if ((st = launch_chain(B.chain, B.d_jobs, step, n + (init ? 1 : 0), init, s)) != GD_OK) break;
       if (stats && (st = tp.end(s)) != GD_OK) break;
@@ -474,6 +520,12 @@ gd_status batch_run(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, gd_repl
   hipError_t e = hipStreamSynchronize(s);
   if (st == GD_OK && e != hipSuccess) st = hip_fail(e, "hipStreamSynchronize");
   *again = st == GD_OK && (B.failed || (res.fail && *res.fail));
+  if (*again && keep.mem) {
+    unsigned kept = 0;
+    if ((e = hipMemcpy(&kept, keep.mem, sizeof kept, hipMemcpyDeviceToHost)) != hipSuccess)
+      st = hip_fail(e, "kept state");
+    *from = (int)kept;
+  }
   if (st == GD_OK && stats) st = tp.collect();
   const auto t1 = std::chrono::steady_clock::now();
   if (gexec) (void)hipGraphExecDestroy(gexec);
@@ -497,12 +549,15 @@ gd_status batch_run(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, gd_repl
 
 gd_status batch_dock_impl(gd_job **jobs, int n_jobs, const gd_mc_param *mc, gd_replica_out *out,
                           gd_stats *stats, int ptile_override, int waves_override) {
+  int from = 0;
   bool again = false;
+  KeepArea keep;
   // a sweep over persistent grids runs by launches
-  gd_status st = batch_run(jobs, n_jobs, mc, out, stats, ptile_override, waves_override, waves_override <= 0, &again);
+  gd_status st = batch_run(jobs, n_jobs, mc, out, stats, ptile_override, waves_override, waves_override <= 0, keep,
+                           &from, &again);
   if (st == GD_OK && again) {
     again = false;
-    st = batch_run(jobs, n_jobs, mc, out, stats, ptile_override, waves_override, false, &again);
+    st = batch_run(jobs, n_jobs, mc, out, stats, ptile_override, waves_override, false, keep, &from, &again);
   }
   return st;
 }
@@ -694,6 +749,8 @@ struct HeldOut {
   }
 };
 
+constexpr int kLaunchSweeps = 256;  // by launches after a wait ran out of time
+
 struct gd_server {
   gd_server_config cfg;
   // mu: pending, results, used, next_ticket, held, cancelled, loading
@@ -709,12 +766,12 @@ struct gd_server {
   // guards active, lists, dirty, launch_step (never held by submit or results)
   std::mutex smu;
   std::vector<ServJob *> active;
-  std::vector<ServJob *> restart;  // to begin again at the next step
   int launch_step = 0;
   hipStream_t stream = nullptr;
   BatchLists lists;
   bool dirty = true;
-  bool by_launches = false;      // a wait of the stepping kernel ran out of time
+  int launch_sweeps = 0;         // sweeps by launches to come, after a wait of the stepping kernel ran out of time
+  KeepArea keep;                 // the active jobs' state at the sweep's first launch of it
   int lc = kSharedLc;
   std::chrono::steady_clock::time_point t0;
   // host input pipeline: file requests parsed by a loader thread
@@ -814,7 +871,6 @@ extern "C" gd_status gd_server_destroy(gd_server *s) {
   for (FileReq *r : s->files) delete r;
   for (auto &kv : s->held) delete kv.second;
   (void)hipStreamSynchronize(s->stream);
-  for (ServJob *j : s->restart) s->active.push_back(j);
   for (ServJob *j : s->active) {
     gd_job_destroy(j->job);
     delete j;
@@ -958,21 +1014,20 @@ extern "C" gd_status gd_server_cancel(gd_server *s, int64_t ticket) {
   }
   // an active job: wait for a running sweep
   std::lock_guard<std::mutex> ls(s->smu);
-  for (std::vector<ServJob *> *list : {&s->active, &s->restart})
-    for (auto it = list->begin(); it != list->end(); ++it)
-      if ((*it)->ticket == ticket) {
-        (void)hipStreamSynchronize(s->stream);
-        ServJob *j = *it;
-        list->erase(it);
-        s->dirty = true;
-        std::lock_guard<std::mutex> lk(s->mu);
-        fail_request(s, ticket, GD_ERR_STATE, j->t_submit, j->t_admit);
-        s->results.back().replica_steps = (double)j->job->h.R * j->done_steps;
-        s->used -= j->foot;
-        gd_job_destroy(j->job);
-        delete j;
-        return GD_OK;
-      }
+  for (auto it = s->active.begin(); it != s->active.end(); ++it)
+    if ((*it)->ticket == ticket) {
+      (void)hipStreamSynchronize(s->stream);
+      ServJob *j = *it;
+      s->active.erase(it);
+      s->dirty = true;
+      std::lock_guard<std::mutex> lk(s->mu);
+      fail_request(s, ticket, GD_ERR_STATE, j->t_submit, j->t_admit);
+      s->results.back().replica_steps = (double)j->job->h.R * j->done_steps;
+      s->used -= j->foot;
+      gd_job_destroy(j->job);
+      delete j;
+      return GD_OK;
+    }
   return GD_ERR_ARG;
 }
 
@@ -1022,8 +1077,6 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
   // (1) admission: FIFO while the estimated footprint fits and a slot is free;
   // an admitted job is then charged its actual device bytes
   std::vector<ServJob *> admitted;
-  admitted.swap(s->restart);  // those of a sweep that failed, from their first step
-  for (ServJob *j : admitted) j->job->h.step0 = j->step0 = s->launch_step;
   for (;;) {
     ServJob *j = nullptr;
     {
@@ -1087,7 +1140,13 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
   // (3) advance every active job by up to sweep_steps (no lock held but smu:
   // submits and result queries proceed meanwhile)
   Stepping turn;
-  Stepping *const stepping = s->by_launches ? nullptr : &turn;
+  Stepping *const stepping = s->launch_sweeps > 0 ? nullptr : &turn;
+  if (s->launch_sweeps > 0) --s->launch_sweeps;
+  // the jobs whose state was kept before the first launch of the stepping kernel,
+  // and the steps they had taken
+  std::vector<ServJob *> kept;
+  std::vector<int> kept_steps;
+  bool no_keep = false;
   for (int k = 0; k < s->cfg.sweep_steps && st == GD_OK; ++k) {
     std::vector<int> act;
     std::vector<gd_job *> jobs;
@@ -1105,7 +1164,16 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
       s->dirty = false;
     }
     // by the stepping kernel up to the next exchange point or end of any job
-    const bool chain = turn.mine && s->lists.chain_max > 0;
+    if (turn.mine && s->lists.chain_max > 0 && kept.empty() && !no_keep) {
+      no_keep = s->keep.make(s->lists.n_blocks, hs) != GD_OK;  // no memory: by launches
+      if (!no_keep) {
+        if ((st = launch_keep(false, s->lists.d_jobs, s->lists.d_blocks, s->lists.n_blocks, s->keep.mem,
+                              (const unsigned *)s->lists.qmem + GD_SY_FAILED, 1, hs)) != GD_OK)
+          break;
+        for (int q : act) kept.push_back(s->active[q]), kept_steps.push_back(s->active[q]->done_steps);
+      }
+    }
+    const bool chain = turn.mine && s->lists.chain_max > 0 && !no_keep;
     int n = 1;
     if (chain) {
       n = std::min(s->lists.chain_max, s->cfg.sweep_steps - k);
@@ -1150,23 +1218,46 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
     e = hipMemcpy(&f, (unsigned *)s->lists.qmem + GD_SY_FAILED, sizeof f, hipMemcpyDeviceToHost);
     if (e != hipSuccess) return hip_fail(e, "stepping kernel status");
     if (f || s->lists.failed) {
-      // a wait ran out of time: the jobs begin again, by launches (the same bits:
-      // a job's draws are a function of its own steps)
-      s->by_launches = s->dirty = true;
-      for (ServJob *j : s->active) {
-        j->done_steps = 0;
-        j->converged = false;
-        j->best_hist.clear();
-        s->restart.push_back(j);
+      // a wait ran out of time: the jobs go on from the state that was kept, by
+      // launches (the same bits: a job's draws are a function of its own steps)
+      s->launch_sweeps = kLaunchSweeps;
+      s->lists.failed = false;
+      std::vector<gd_job *> jobs;
+      std::vector<int> all;
+      for (size_t q = 0; q < kept.size(); ++q) {
+        ServJob *j = kept[q];
+        j->done_steps = kept_steps[q];
+        j->job->h.step0 = j->step0 = s->launch_step - j->done_steps;
+        jobs.push_back(j->job);
+        all.push_back((int)q);
       }
-      s->active.clear();
+      BatchLists B;
+      e = hipMemsetAsync(s->lists.qmem, 0, s->lists.sync_bytes, hs);
+      st = e == hipSuccess ? B.build(jobs, all, hs, nullptr) : hip_fail(e, "stepping kernel counters");
+      if (st == GD_OK) st = launch_keep(true, B.d_jobs, B.d_blocks, B.n_blocks, s->keep.mem, nullptr, 1, hs);
+      e = hipStreamSynchronize(hs);
+      if (st == GD_OK && e != hipSuccess) st = hip_fail(e, "kept state");
+      s->dirty = true;
+      if (st != GD_OK) {
+        // neither steps nor state to go on from: report each
+        std::lock_guard<std::mutex> lk(s->mu);
+        for (ServJob *j : kept) {
+          fail_request(s, j->ticket, st, j->t_submit, j->t_admit);
+          s->used -= j->foot;
+          s->active.erase(std::find(s->active.begin(), s->active.end(), j));
+          gd_job_destroy(j->job);
+          delete j;
+        }
+        return st;
+      }
     }
   }
   // (4) convergence: a job's sweep ends every sweep_steps of its own steps
   if (s->cfg.converge_sweeps > 0) {
     for (ServJob *j : s->active) {
       if (j->converged || j->done_steps >= j->mc.steps_total || j->done_steps == 0 ||
-          j->done_steps % s->cfg.sweep_steps != 0)
+          j->done_steps % s->cfg.sweep_steps != 0 ||
+          (int)j->best_hist.size() >= j->done_steps / s->cfg.sweep_steps)  // a sweep that was taken back
         continue;
       float b;
       if ((st = job_best(j->job, hs, &b)) != GD_OK) return st;
@@ -1205,7 +1296,7 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
     s->used -= j->foot;
     delete j;
   }
-  if (n_active) *n_active = (int)(s->active.size() + s->restart.size());
+  if (n_active) *n_active = (int)s->active.size();
   std::lock_guard<std::mutex> lk(s->mu);
   if (n_done) *n_done = (int)s->results.size();
   return GD_OK;

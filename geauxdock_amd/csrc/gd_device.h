@@ -151,6 +151,11 @@ struct GdChain {          // arguments of one launch of the stepping kernel
   long long wait_ticks;   // bound of one wait, in ticks of the constant-rate counter
 };
 
+// State kept of a 64-replica block (gd_keep_kernel): rows of 64 words.  The area
+// begins with a line that holds the MC step of the state.
+#define GD_KEEP_ROWS 30
+#define GD_KEEP_HEAD 64   // words
+
 struct GdPack {           // one job's results for the host
   const float *mm, *en, *best;
   const int *tmpi, *nacc, *nexc, *acc, *nswp;

@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <functional>
 #include <memory>
 #include <string>
@@ -27,14 +28,27 @@ struct ChainList {
   unsigned epoch = 0, steps = 0;        // launches and their steps since the counters were zero
   bool stale = false;                   // a run did not end well: its counters are zeroed before they are used
   int lds = 0;                          // LDS added to a group's, which bounds the groups of a CU
-  double wait_s = GD_CHAIN_WAIT_S;      // bound of one wait in the kernel
+  std::atomic<double> wait_s{GD_CHAIN_WAIT_S};  // bound of one wait in the kernel
   double step_pairs = 0;                // (atom, point) pairs of one step
   // The host lists (items of each job, blocks) and the launch shape on a device of
   // `cu` CUs (0: this one).
   void shape(const std::vector<const GdJob *> &jobs, int cu = 0);
   int slots = 0;                        // groups that such a device holds at a time
   size_t queue_bytes() const { return (size_t)n_entries * stride * cap_steps * sizeof(unsigned long long); }
+  // Work of n steps on the scale of kKeepWork.
+  double work(int n) const { return n * (step_pairs > 5e7 ? step_pairs : 5e7); }
 };
+
+// A run keeps its state (gd_keep_kernel) once in that many pairs, about 0.2 s; a step of
+// few pairs, whose time is its latency, counts as 25 us of them.
+constexpr double kKeepWork = 4e11;
+inline size_t keep_bytes(int n_blocks) {
+  return (GD_KEEP_HEAD + (size_t)n_blocks * GD_KEEP_ROWS * 64) * sizeof(unsigned);
+}
+// The state of the jobs of a list of blocks, before MC step `step`: kept in `area`
+// unless *failed, or (back) brought back from it.
+gd_status launch_keep(bool back, const GdJob *d_jobs, const GdBlock *d_blocks, int n_blocks, unsigned *area,
+                      const unsigned *failed, int step, hipStream_t s);
 }  // namespace gdr
 
 namespace gdr {
@@ -95,6 +109,8 @@ struct gd_job {
   int n_streams = kDefaultStreams;  // streams the plain path steps on (1 .. kMaxParts)
   hipStream_t part_stream[kMaxParts] = {};
   gdr::ChainList chain;      // the stepping kernel's list, its queue and its counters
+  unsigned *d_keep = nullptr;  // state kept of a run by it
+  bool keep_used = false;      // d_keep names a step of an earlier run
   // buffers of energy evaluations: a part of the arena for the lanes of up to Rp
   // poses (their other buffers are the job's own), and a workspace for more
   gdr::EvalLanes ev{};

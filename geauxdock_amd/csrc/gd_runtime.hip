@@ -38,6 +38,8 @@ __global__ void gd_reduce_kernel(const GdJob *, const GdBlock *);
 __global__ void gd_finish_kernel(const GdJob *, const GdBlock *, int, int, const int *, int *);
 template <int LC>
 __global__ void gd_chain_kernel(const GdChain);
+template <bool BACK>
+__global__ void gd_keep_kernel(const GdJob *, const GdBlock *, unsigned *, const unsigned *, unsigned);
 __global__ void gd_start_job_kernel(const GdJob, GdJob *);
 __global__ void gd_pack_kernel(const GdPackList);
 __global__ void gd_exchange_kernel(const GdJob *, const GdExch *, int);
@@ -820,8 +822,8 @@ static gd_status chain_make(gd_job *j) {
   for (int rb = 0; rb < j->h.Rp; rb += 64) blocks.push_back({0, rb, 0, (int)items.size()});
   auto up = [](size_t b) { return (b + 255) / 256 * 256; };
   const size_t bi = items.size() * sizeof(GdItem), bb = blocks.size() * sizeof(GdChainBlock),
-               bs = chain_sync_bytes(cl.n_blocks), bq = cl.queue_bytes();
-  const size_t all = up(bi) + up(bb) + up(bs) + up(bq);
+               bs = chain_sync_bytes(cl.n_blocks), bq = cl.queue_bytes(), bk = keep_bytes(cl.n_blocks);
+  const size_t all = up(bi) + up(bb) + up(bs) + up(bq) + up(bk);
   hipError_t e = hipMalloc(&j->d_chain, all);
   if (e != hipSuccess) return hip_fail(e, "hipMalloc stepping lists");
   j->chain_bytes = all;
@@ -830,11 +832,13 @@ static gd_status chain_make(gd_job *j) {
   cl.d_blocks = (GdChainBlock *)(base + up(bi));
   cl.d_sync = (unsigned *)(base + up(bi) + up(bb));
   cl.d_queue = (unsigned long long *)(base + up(bi) + up(bb) + up(bs));
+  j->d_keep = (unsigned *)(base + up(bi) + up(bb) + up(bs) + up(bq));
+  j->keep_used = false;
   cl.epoch = cl.steps = 0;
   cl.stale = false;
   if ((e = hipMemcpyAsync(base, items.data(), bi, hipMemcpyHostToDevice, j->stream)) != hipSuccess ||
       (e = hipMemcpyAsync(base + up(bi), blocks.data(), bb, hipMemcpyHostToDevice, j->stream)) != hipSuccess ||
-      (e = hipMemsetAsync(cl.d_sync, 0, up(bs) + up(bq), j->stream)) != hipSuccess ||
+      (e = hipMemsetAsync(cl.d_sync, 0, up(bs) + up(bq) + GD_KEEP_HEAD * sizeof(unsigned), j->stream)) != hipSuccess ||
       (e = hipStreamSynchronize(j->stream)) != hipSuccess) {
     chain_drop(j);
     return hip_fail(e, "stepping list upload");
@@ -1069,6 +1073,19 @@ gd_status launch_chain(ChainList &c, const GdJob *d_jobs, int step0, int n_steps
   if (e != hipSuccess) return hip_fail(e, "stepping kernel launch");
   c.steps += (unsigned)n_steps;  // the counters hold what was launched
   return GD_OK;
+}
+
+gd_status launch_keep(bool back, const GdJob *d_jobs, const GdBlock *d_blocks, int n_blocks, unsigned *area,
+                      const unsigned *failed, int step, hipStream_t s) {
+  if (n_blocks <= 0) return GD_OK;
+  if (back)
+    hipLaunchKernelGGL(gd_keep_kernel<true>, dim3(n_blocks), dim3(256), 0, s, d_jobs, d_blocks, area, failed,
+                       (unsigned)step);
+  else
+    hipLaunchKernelGGL(gd_keep_kernel<false>, dim3(n_blocks), dim3(256), 0, s, d_jobs, d_blocks, area, failed,
+                       (unsigned)step);
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? GD_OK : hip_fail(e, "keep kernel launch");
 }
 
 gd_status launch_swap(int axis, const GdJob *d_jobs, const GdBlock *d_blocks, int n_blocks,
@@ -1600,9 +1617,11 @@ struct RecSink {
 // copied; dump k + 2 reuses the half only after the host has taken it.
 // chain: the stepping kernel may be used.  *again: one of its waits ran out of
 // time, nothing was handed over of this dump or later ones (*handed dumps were,
-// or had been before), and the run is to be repeated without it.
+// or had been before), and the run is to go on without it from MC step *from, the
+// last one whose state was kept (0: from the start).
 static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
-                          gd_replica_out *out, gd_stats *stats, const bool chain, int *handed, bool *again) {
+                          gd_replica_out *out, gd_stats *stats, const bool chain, int *from, int *handed,
+                          bool *again) {
   if (!j || !mc || mc->steps_total < 0 || mc->steps_per_exchange < 0) return GD_ERR_ARG;
   gd_status st = ensure_device();
   if (st != GD_OK) return st;
@@ -1701,14 +1720,16 @@ static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
       chain_max = 0;
     }
   }
-  // hand dump k (ring half b, copied to the host) to the sink, each dump once;
-  // false: the stepping kernel failed in it or before
+  // hand dump k (ring half b, copied to the host) to the sink, each dump once
+  const auto hand = [&](int k, int b) {
+    if (k < *handed) return;
+    sink->fn(sink->user, k, k * spd, g.R, spd, h_half[b], h_cnt[b]);
+    *handed = k + 1;
+  };
+  // false: the stepping kernel failed, in it or before or since
   const auto deliver = [&](int k, int b) {
     if (chain_max > 0 && *h_fail[b]) return false;
-    if (k >= *handed) {
-      sink->fn(sink->user, k, k * spd, g.R, spd, h_half[b], h_cnt[b]);
-      *handed = k + 1;
-    }
+    hand(k, b);
     return true;
   };
   const unsigned *d_fail = j->chain.d_sync + GD_SY_FAILED;
@@ -1769,11 +1790,17 @@ static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
       c.steps = 0;
     }
     c.stale = true;  // until this run has ended well
+    if (j->keep_used && (e = hipMemsetAsync(j->d_keep, 0, sizeof(unsigned), s)) != hipSuccess)
+      return hip_fail(e, "kept state");
+    j->keep_used = false;
   }
   // initial energies (MonteCarlo_d with s2max = 1)
   hipLaunchKernelGGL(gd_start_job_kernel, dim3(j->n_blocks), dim3(256), 0, s, g, j->d_job);
   if ((e = hipGetLastError()) != hipSuccess) st = hip_fail(e, "start kernel launch");
-  if (chain_max > 0) {
+  if (*from > 0) {
+    if (st == GD_OK)
+      st = launch_keep(true, j->d_job, j->d_blocks, j->n_blocks, j->d_keep, nullptr, *from, s);
+  } else if (chain_max > 0) {
     if (st == GD_OK && mc->steps_total == 0) st = launch_chain(j->chain, j->d_job, 0, 1, true, s);
   } else {
     if (st == GD_OK) st = launch_pair(g.lc, j->d_job, j->d_items, j->n_items, s);
@@ -1782,7 +1809,8 @@ static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
   if (st == GD_OK && multi && timing) st = tspan.mark_ref(s);
   int pending = -1;  // streamed dump whose copy is in flight
   int chain_steps = 0;  // MC steps (and initial pass) taken by the stepping kernel
-  for (int s1 = 0, k = 0; s1 < mc->steps_total && st == GD_OK; s1 += spd, ++k) {
+  double since = 0.0;   // work since the state was kept
+  for (int k = *from / spd, s1 = k * spd; s1 < mc->steps_total && st == GD_OK; s1 += spd, ++k) {
     const int b = k & 1;
     if (record) {
       e = hipMemsetAsync(g.rec_n + (size_t)b * g.Rp, 0, (size_t)g.Rp * sizeof(int), s);
@@ -1793,7 +1821,7 @@ static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
     }
     if (multi && (st = fork()) != GD_OK) break;
     const int s_end = std::min(mc->steps_total, s1 + spd);
-    for (int step = s1; step < s_end; ++step) {
+    for (int step = std::max(s1, *from); step < s_end; ++step) {
       const bool timed = timing && step % kTimedEvery == 0;
       if (chain_max > 0) {
         // up to the next exchange point or the dump's end; the initial pass
@@ -1801,6 +1829,13 @@ static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
         const bool init = step == 0;
         int n = std::min(s_end - step, chain_max - (init ? 1 : 0));
         if (n_rounds > 0) n = std::min(n, spe - step % spe);
+        // kept where a dump of records starts, whose counts are zero
+        if (since >= kKeepWork && (!record || step == s1)) {
+          if ((st = launch_keep(false, j->d_job, j->d_blocks, j->n_blocks, j->d_keep, d_fail, step, s)) != GD_OK) break;
+          j->keep_used = true;
+          since = 0.0;
+        }
+        since += j->chain.work(n);
         if (timing && (st = tp.begin(s)) != GD_OK) break;
         if ((st = launch_chain(j->chain, j->d_job, step, n + (init ? 1 : 0), init, s)) != GD_OK) break;
         if (timing && (st = tp.end(s)) != GD_OK) break;
@@ -1870,10 +1905,7 @@ static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
         st = hip_fail(e, "record copy");
         break;
       }
-      if (!deliver(pending, pending & 1)) {
-        pending = -1;
-        break;
-      }
+      if (!deliver(pending, pending & 1)) break;
     }
     pending = k;
   }
@@ -1894,8 +1926,14 @@ static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
   if (st == GD_OK && chain_max > 0) {
     *again = *res.fail != 0;
     j->chain.stale = *again;
+    unsigned kept = 0;
+    if (*again && j->keep_used && (e = hipMemcpy(&kept, j->d_keep, sizeof kept, hipMemcpyDeviceToHost)) != hipSuccess)
+      st = hip_fail(e, "kept state");
+    *from = (int)kept;
   }
-  if (st == GD_OK && !*again && sink && !sink->blocking && pending >= 0) deliver(pending, pending & 1);
+  // the last dump; of a run that goes on from a kept state, one that ended before it
+  if (st == GD_OK && sink && !sink->blocking && pending >= 0 && (!*again || (pending + 1) * (long long)spd <= *from))
+    hand(pending, pending & 1);
   if (st == GD_OK && timing) st = multi ? tspan.collect(np) : tp.collect();
   const auto t1 = std::chrono::steady_clock::now();
   if (st != GD_OK || *again) return st;
@@ -1924,12 +1962,12 @@ static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
 
 static gd_status dock_impl(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
                            gd_replica_out *out, gd_stats *stats) {
-  int handed = 0;
+  int from = 0, handed = 0;
   bool again = false;
-  gd_status st = dock_run(j, mc, sink, out, stats, true, &handed, &again);
+  gd_status st = dock_run(j, mc, sink, out, stats, true, &from, &handed, &again);
   if (st == GD_OK && again) {
     again = false;
-    st = dock_run(j, mc, sink, out, stats, false, &handed, &again);
+    st = dock_run(j, mc, sink, out, stats, false, &from, &handed, &again);
   }
   return st;
 }

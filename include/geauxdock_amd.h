@@ -290,8 +290,10 @@ gd_status gd_tiling_get(const gd_job *job, gd_tiling *t);
  * lists are rebuilt). */
 gd_status gd_job_set_streams(gd_job *job, int n_streams);
 /* Bound of one wait inside the stepping kernel (seconds, 0 to 60, default 2) in
- * runs and batches of the job.  A run that exceeds it, as when other processes'
- * kernels hold the device, is repeated by launches. */
+ * runs and batches of the job, those under way included.  A run that exceeds it, as
+ * when other processes' kernels hold the device, goes on by launches from a state
+ * that it kept (about every 0.2 s, in a run that records at a dump's start; before the
+ * first, from its start): the results are the same bits. */
 gd_status gd_job_set_step_wait(gd_job *job, double seconds);
 gd_status gd_tiling_set(gd_job *job, const gd_tiling *t);
 /* Sweep atoms per lane x protein tile counts on `job` for `steps` MC steps
@@ -337,8 +339,8 @@ typedef struct {
  * results and usage queries never wait for a device sweep. */
 gd_status gd_server_create(const gd_server_config *cfg, gd_server **out);
 /* gd_job_set_step_wait for the server's sweeps.  When a wait exceeds the bound, the
- * active requests begin again and the server steps by launches from then on:
- * the results are the same bits. */
+ * sweep is taken again, and it and the next 255 by launches: the results are the
+ * same bits. */
 gd_status gd_server_set_step_wait(gd_server *server, double seconds);
 gd_status gd_server_destroy(gd_server *s);
 /* Device bytes a complex will occupy as a plain job (host-side estimate of
