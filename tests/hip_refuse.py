@@ -11,11 +11,13 @@ SHIM = r"""
 #define _GNU_SOURCE
 #include <dlfcn.h>
 #include <stddef.h>
+#include <string.h>
 typedef struct { unsigned x, y, z; } dim;
-static long g_pass = -1;                 /* kernel launches until one is refused (-1: none is) */
+static long g_pass = -1;                 /* launches of the stepping kernel until one is refused (-1: none is) */
+static const void *g_step;               /* the stepping kernel's host function */
 static size_t g_host = (size_t)-1, g_dev = (size_t)-1;  /* most bytes of a pinned / device allocation */
 static int g_err, g_n_host, g_n_dev;
-void refuse_launch_after(long n) { g_pass = n; }
+void refuse_stepping_after(long n) { g_pass = n; }
 void refuse_pinned_over(size_t n) { g_host = n; g_n_host = 0; }
 void refuse_device_over(size_t n) { g_dev = n; g_n_dev = 0; }
 int refused_pinned(void) { return g_n_host; }
@@ -25,10 +27,16 @@ static void *real(const char *name) {
   if (!h) h = dlopen("libamdhip64.so.7", RTLD_LAZY | RTLD_NOLOAD);
   return h ? dlsym(h, name) : 0;
 }
+void __hipRegisterFunction(void *m, const void *host, char *device, const char *name, unsigned n, void *tid, void *bid,
+                           dim *block, dim *grid, int *size) {
+  typedef void (*fn)(void *, const void *, char *, const char *, unsigned, void *, void *, dim *, dim *, int *);
+  if (strstr(name, "gd_chain_kernel")) g_step = host;
+  ((fn)real("__hipRegisterFunction"))(m, host, device, name, n, tid, bid, block, grid, size);
+}
 int hipLaunchKernel(const void *f, dim grid, dim block, void **args, size_t lds, void *s) {
   static int (*r)(const void *, dim, dim, void **, size_t, void *);
-  if (g_pass == 0) { g_pass = -1; return g_err = 9; }
-  if (g_pass > 0) --g_pass;
+  if (f == g_step && g_pass == 0) { g_pass = -1; return g_err = 9; }
+  if (f == g_step && g_pass > 0) --g_pass;
   if (!r) r = (int (*)(const void *, dim, dim, void **, size_t, void *))real("hipLaunchKernel");
   return r(f, grid, block, args, lds, s);
 }
@@ -56,7 +64,7 @@ HEAD = """
 import ctypes as C, sys
 import numpy as np
 shim = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
-shim.refuse_launch_after.argtypes = [C.c_long]
+shim.refuse_stepping_after.argtypes = [C.c_long]
 shim.refuse_pinned_over.argtypes = [C.c_size_t]
 shim.refuse_device_over.argtypes = [C.c_size_t]
 NONE = 2 ** 64 - 1
