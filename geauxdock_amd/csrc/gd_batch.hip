@@ -543,8 +543,7 @@ gd_status batch_run(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, gd_repl
     stats->ms_pair_span = tp.n ? tp.ms / tp.n : 0.0;
     if (chain_steps > 0) stats->n_pair_launch = chain_steps, stats->ms_pair_span = tp.ms / chain_steps;
   }
-  out_copy(jobs.data(), outs.data(), n_jobs, res);
-  return GD_OK;
+  return out_copy(jobs.data(), outs.data(), n_jobs, res, s);
 }
 
 gd_status batch_dock_impl(gd_job **jobs, int n_jobs, const gd_mc_param *mc, gd_replica_out *out,
@@ -1285,7 +1284,7 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
   gd_status rs = out_launch(djobs.data(), douts.data(), (int)done.size(), nullptr, hs, res);
   e = hipStreamSynchronize(hs);
   if (rs == GD_OK && e != hipSuccess) rs = hip_fail(e, "results");
-  if (rs == GD_OK) out_copy(djobs.data(), douts.data(), (int)done.size(), res);
+  if (rs == GD_OK) rs = out_copy(djobs.data(), douts.data(), (int)done.size(), res, hs);
   for (ServJob *j : done) {
     const double rsteps = (double)j->job->h.R * j->done_steps;
     gd_job_destroy(j->job);

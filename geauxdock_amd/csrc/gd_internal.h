@@ -153,15 +153,18 @@ void noalloc_host_make();
 float *noalloc_host();
 // Results of jobs whose runs are done in stream order: out_launch queues the
 // kernel that gathers them (and the word *d_fail, if given), out_copy hands them
-// over once the stream was waited for.  out[k] may be null.
+// over once the stream was waited for.  Results of more than kHostPoolBytes, or for
+// which there is no pinned memory, are copied row by row.  out[k] may be null.
 struct OutStage {
   HostBuf buf;
   std::vector<size_t> at;    // word offset of each job
   const unsigned *fail = nullptr;
+  unsigned fail_word = 0;
+  bool by_copies = false;
 };
 gd_status out_launch(gd_job *const *jobs, gd_replica_out *const *out, int n, const unsigned *d_fail, hipStream_t s,
                      OutStage &o);
-void out_copy(gd_job *const *jobs, gd_replica_out *const *out, int n, const OutStage &o);
+gd_status out_copy(gd_job *const *jobs, gd_replica_out *const *out, int n, const OutStage &o, hipStream_t s);
 float far_r2_threshold(double pmf0, double el1);
 // nb, nb_list: see gd_pair_kernel.
 gd_status launch_pair(int lc, const GdJob *d_jobs, const GdItem *d_items, int n_items, hipStream_t s, int nb = 0,
@@ -178,9 +181,10 @@ struct EvalBufs {
 size_t eval_carve(const GdJob &g, int nb, char *base, EvalBufs *b);
 constexpr size_t kEvalHostWords = 2 + 6 + 10 + 9;  // host words of a pose: inputs, results
 // One pass over cnt poses on the job's stream, waited for: setup, pair, reduce
-// and finish kernels.  host: kEvalHostWords words a pose that kernels read and write.
+// and finish kernels.  host: kEvalHostWords words a pose that kernels read and write;
+// without, dev: as many on the device, to and from which the caller's arrays are copied.
 gd_status eval_pass(gd_job *j, const EvalBufs &b, int cnt, const int *conf, const float *pose, float *terms,
-                    float *raw, float *host);
+                    float *raw, float *host, float *dev);
 gd_status launch_exchange(const GdJob *d_jobs, int round, hipStream_t s);  // of one job
 size_t chain_sync_bytes(int n_blocks);
 // Steps that one launch may take (0: this list is stepped by launches).

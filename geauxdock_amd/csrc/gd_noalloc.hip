@@ -8,7 +8,7 @@
 // Same kernels and the same tiling as gd_energy_eval, so the results are the
 // same bits.  Poses run in passes of whole 64-lane blocks that fit the scratch
 // and the device's host buffer for inputs and results, which was made with its
-// first job.  Every call on a GPU shares both: calls that overlap on one GPU race
+// first job (without it they are copied).  Every call on a GPU shares both: calls that overlap on one GPU race
 // (the scratch keeps the last call's contents).
 #include <hip/hip_runtime.h>
 
@@ -68,10 +68,6 @@ extern "C" gd_status gd_energy_eval_noalloc(gd_job *j, int n, const int *conf, c
   void *base = nullptr;
   if ((st = scratch_ptr(&base)) != GD_OK) return st;
   float *host = gdr::noalloc_host();
-  if (!host) {
-    gdr::set_error("gd_energy_eval_noalloc: no host buffer (out of memory when the job was made)");
-    return GD_ERR_HIP;
-  }
   if (one_block_bytes(g) > (size_t)GD_NOALLOC_SCRATCH_BYTES) {
     char buf[200];
     std::snprintf(buf, sizeof buf,
@@ -84,13 +80,19 @@ extern "C" gd_status gd_energy_eval_noalloc(gd_job *j, int n, const int *conf, c
   // blocks of a pass: as many as fit the scratch and the host buffer
   int nb = (int)(gdr::kNoallocHostBytes / (64 * gdr::kEvalHostWords * sizeof(float)));
   if (nb > (n - 1) / 64 + 1) nb = (n - 1) / 64 + 1;
-  while (gdr::eval_carve(g, nb, nullptr, nullptr) > (size_t)GD_NOALLOC_SCRATCH_BYTES) --nb;  // one block fits
+  // without a host buffer (there was no memory for it) inputs and results are copied
+  // through the scratch
+  const auto pass_bytes = [&](int k) {
+    return gdr::eval_carve(g, k, nullptr, nullptr) + (host ? 0 : (size_t)k * 64 * gdr::kEvalHostWords * sizeof(float));
+  };
+  while (pass_bytes(nb) > (size_t)GD_NOALLOC_SCRATCH_BYTES) --nb;  // one block fits
+  float *dev = host ? nullptr : (float *)((char *)base + gdr::eval_carve(g, nb, nullptr, nullptr));
   gdr::EvalBufs b;
   gdr::eval_carve(g, nb, (char *)base, &b);
   for (int at = 0; at < n && st == GD_OK; at += nb * 64) {
     const int cnt = n - at < nb * 64 ? n - at : nb * 64;
     st = gdr::eval_pass(j, b, cnt, conf + 2 * (size_t)at, pose + 6 * (size_t)at, terms + 10 * (size_t)at,
-                        raw ? raw + 9 * (size_t)at : nullptr, host);
+                        raw ? raw + 9 * (size_t)at : nullptr, host, dev);
   }
   return st;
 }

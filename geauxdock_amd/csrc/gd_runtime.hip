@@ -1234,8 +1234,14 @@ gd_status out_launch(gd_job *const *jobs, gd_replica_out *const *out, int n, con
       words += ((size_t)jobs[k]->h.R * GD_PACK_W + 15) / 16 * 16;
     }
   if (words == 16 && !d_fail) return GD_OK;
-  gd_status st = o.buf.acquire(words * sizeof(float));
-  if (st != GD_OK) return st;
+  gd_status st = GD_OK;
+  o.by_copies = words * sizeof(float) > kHostPoolBytes || o.buf.acquire(words * sizeof(float)) != GD_OK;
+  if (o.by_copies) {
+    if (!d_fail) return GD_OK;
+    o.fail = &o.fail_word;
+    const hipError_t e = hipMemcpyAsync(&o.fail_word, d_fail, sizeof(unsigned), hipMemcpyDeviceToHost, s);
+    return e == hipSuccess ? GD_OK : hip_fail(e, "stepping kernel status");
+  }
   float *base = (float *)o.buf.p;
   if (d_fail) o.fail = (unsigned *)base;
   GdPackList list;
@@ -1287,40 +1293,87 @@ size_t eval_carve(const GdJob &g, int nb, char *base, EvalBufs *b) {
 }
 
 gd_status eval_pass(gd_job *j, const EvalBufs &b, int cnt, const int *conf, const float *pose, float *terms,
-                    float *raw, float *host) {
+                    float *raw, float *host, float *dev) {
   const int nb = (cnt + 63) / 64;
+  float *const io = host ? host : dev;
   hipStream_t s = j->stream;
   GdJob x = j->h;  // the job's tables, the evaluation's lanes and buffers
   x.R = cnt;
   x.Rp = nb * 64;
   x.ligi = b.ligi, x.prti = b.prti, x.prop = b.prop, x.coords = b.coords;
   x.part_lin = b.plin, x.part_hpc = b.phpc, x.part_mcs = b.pmcs, x.fin_part = b.fin;
-  int *h_conf = (int *)host;
-  float *h_pose = host + 2 * (size_t)cnt;
-  x.ev_terms = host + 8 * (size_t)cnt;  // written over the link by the finish kernel
-  x.ev_raw = host + 18 * (size_t)cnt;
+  int *h_conf = (int *)io;
+  float *h_pose = io + 2 * (size_t)cnt;
+  x.ev_terms = io + 8 * (size_t)cnt;  // written over the link by the finish kernel
+  x.ev_raw = io + 18 * (size_t)cnt;
   x.rec = nullptr;
   x.rec_cap = 0;
   x.record = 0;
-  std::memcpy(h_conf, conf, (size_t)cnt * 2 * sizeof(int));
-  std::memcpy(h_pose, pose, (size_t)cnt * 6 * sizeof(float));
+  hipError_t e = hipSuccess;
+  if (host) {
+    std::memcpy(h_conf, conf, (size_t)cnt * 2 * sizeof(int));
+    std::memcpy(h_pose, pose, (size_t)cnt * 6 * sizeof(float));
+  } else if ((e = hipMemcpyAsync(h_conf, conf, (size_t)cnt * 2 * sizeof(int), hipMemcpyHostToDevice, s)) !=
+                 hipSuccess ||
+             (e = hipMemcpyAsync(h_pose, pose, (size_t)cnt * 6 * sizeof(float), hipMemcpyHostToDevice, s)) !=
+                 hipSuccess) {
+    return hip_fail(e, "evaluation inputs");
+  }
   hipLaunchKernelGGL(gd_eval_setup_kernel, dim3(nb), dim3(1024), 0, s, x, b.job, (const int *)h_conf,
                      (const float *)h_pose, cnt);
-  hipError_t e = hipGetLastError();
+  e = hipGetLastError();
   gd_status st = e == hipSuccess ? GD_OK : hip_fail(e, "eval setup kernel launch");
   if (st == GD_OK) st = launch_pair(x.lc, b.job, j->d_items, x.nL * x.nG * nb, s, nb, j->h.Rp / 64);
   if (st == GD_OK) st = launch_finish(b.job, nullptr, nb, GD_MODE_EVAL, 0, s);
+  if (!host && st == GD_OK &&
+      ((e = hipMemcpyAsync(terms, x.ev_terms, (size_t)cnt * 10 * sizeof(float), hipMemcpyDeviceToHost, s)) !=
+           hipSuccess ||
+       (raw && (e = hipMemcpyAsync(raw, x.ev_raw, (size_t)cnt * 9 * sizeof(float), hipMemcpyDeviceToHost, s)) !=
+                   hipSuccess)))
+    st = hip_fail(e, "evaluation results");
   e = hipStreamSynchronize(s);
   if (st == GD_OK && e != hipSuccess) st = hip_fail(e, "energy evaluation");
-  if (st != GD_OK) return st;
+  if (st != GD_OK || !host) return st;
   std::memcpy(terms, x.ev_terms, (size_t)cnt * 10 * sizeof(float));
   if (raw) std::memcpy(raw, x.ev_raw, (size_t)cnt * 9 * sizeof(float));
   return GD_OK;
 }
 
-void out_copy(gd_job *const *jobs, gd_replica_out *const *out, int n, const OutStage &o) {
+// Results of a job row by row of the device's arrays.
+static gd_status out_rows(const GdJob &g, const gd_replica_out &q, hipStream_t s) {
+  const size_t R = g.R, Rp = g.Rp;
+  std::vector<float> row(R);
+  const auto down = [&](void *to, const void *from) -> gd_status {
+    hipError_t e = hipMemcpyAsync(to, from, R * 4, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    return e == hipSuccess ? GD_OK : hip_fail(e, "results");
+  };
+  gd_status st = GD_OK;
+  const auto turned = [&](float *to, const float *from, int n) {  // [n][Rp] to [R][n]
+    for (int i = 0; to && i < n && st == GD_OK; ++i)
+      if ((st = down(row.data(), from + (size_t)i * Rp)) == GD_OK)
+        for (size_t r = 0; r < R; ++r) to[r * n + i] = row[r];
+  };
+  turned(q.movematrix, g.mm, 6);
+  turned(q.energy, g.en, 10);
+  const struct {
+    void *to;
+    const void *from;
+  } rows[] = {{q.best_energy, g.best}, {q.idx_tmp, g.tmpi},   {q.n_accept, g.nacc},  {q.n_exchange, g.nexc},
+              {q.is_accept, g.acc},    {q.n_swap_lig, g.nswp}, {q.n_swap_prt, g.nswp + Rp}};
+  for (const auto &x : rows)
+    if (x.to && st == GD_OK) st = down(x.to, x.from);
+  return st;
+}
+
+gd_status out_copy(gd_job *const *jobs, gd_replica_out *const *out, int n, const OutStage &o, hipStream_t s) {
   for (int k = 0; k < n; ++k) {
     if (!out[k]) continue;
+    if (o.by_copies) {
+      const gd_status st = out_rows(jobs[k]->h, *out[k], s);
+      if (st != GD_OK) return st;
+      continue;
+    }
     const size_t R = jobs[k]->h.R;
     const float *p = (const float *)o.buf.p + o.at[k];
     const gd_replica_out &q = *out[k];
@@ -1337,6 +1390,7 @@ void out_copy(gd_job *const *jobs, gd_replica_out *const *out, int n, const OutS
     cp(q.n_swap_lig, p + 21 * R, R);
     cp(q.n_swap_prt, p + 22 * R, R);
   }
+  return GD_OK;
 }
 
 // A job of its own (plain tiling, its own stream), or, with a stream, one that
@@ -1576,13 +1630,29 @@ gd_status gd_energy_eval(gd_job *j, int n, const int *conf, const float *pose, f
       }
     }
   }
+  // inputs and results: at most the pool's bytes a pass; without pinned memory, through
+  // a device buffer
+  lanes = std::min(lanes, (int)(kHostPoolBytes / (64 * kEvalHostWords * sizeof(float))) * 64);
+  const size_t io_bytes = (size_t)std::min(n, lanes) * kEvalHostWords * sizeof(float);
   HostBuf host;
-  if ((st = host.acquire((size_t)std::min(n, lanes) * kEvalHostWords * sizeof(float))) != GD_OK) return st;
+  struct DevBuf {
+    void *p = nullptr;
+    ~DevBuf() {
+      if (p) hipFree(p);
+    }
+  } dev;
+  if (host.acquire(io_bytes) != GD_OK) {
+    const hipError_t e = hipMalloc(&dev.p, io_bytes);
+    if (e != hipSuccess) {
+      dev.p = nullptr;
+      return hip_fail(e, "evaluation buffers");
+    }
+  }
   std::vector<float> oc;
   for (int base = 0; base < n && st == GD_OK; base += lanes) {
     const int cnt = std::min(lanes, n - base);
     st = eval_pass(j, b, cnt, conf + 2 * (size_t)base, pose + 6 * (size_t)base, terms + 10 * (size_t)base,
-                   raw ? raw + 9 * (size_t)base : nullptr, (float *)host.p);
+                   raw ? raw + 9 * (size_t)base : nullptr, (float *)host.p, (float *)dev.p);
     if (st != GD_OK || !coords) continue;
     const int W = (cnt + 63) / 64 * 64;  // lanes of the pass
     oc.resize((size_t)3 * L * W);
@@ -1956,8 +2026,7 @@ static gd_status dock_run(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
       stats->ms_step_period = stats->ms_pair_span = tp.ms / chain_steps;
     }
   }
-  out_copy(&j, &out, 1, res);
-  return GD_OK;
+  return out_copy(&j, &out, 1, res, s);
 }
 
 static gd_status dock_impl(gd_job *j, const gd_mc_param *mc, const RecSink *sink,
@@ -1989,8 +2058,7 @@ gd_status gd_job_replicas(gd_job *j, gd_replica_out *out) {
   gd_status st = out_launch(&j, &out, 1, nullptr, j->stream, res);
   const hipError_t e = hipStreamSynchronize(j->stream);
   if (st == GD_OK && e != hipSuccess) st = hip_fail(e, "results");
-  if (st == GD_OK) out_copy(&j, &out, 1, res);
-  return st;
+  return st == GD_OK ? out_copy(&j, &out, 1, res, j->stream) : st;
 }
 
 gd_status gd_dock_records(gd_job *j, int cap, float *rec, int *count) {

@@ -86,3 +86,51 @@ assert errors >= 1
 for a, b in zip(want, got):
     same(a, b)
 """)
+
+
+def test_no_pinned_memory(tmp_path):
+    """No pinned memory at all from the first call on: evaluations, runs, batches,
+    the served requests and the read-back give what they give with it."""
+    hip_refuse.run(tmp_path, _SERVE.replace("want, errors = serve({})\nassert errors == 0", "") + """
+from tests.oracle_ffi import random_poses
+ip, fp = C.POINTER(C.c_int), C.POINTER(C.c_float)
+small = g.synth_complex(300, 9, 3, 2, 1, seed=1, ene=ene)
+large = g.synth_complex(4001, 46, 5, 11, 4, floor_temp=0.05, ceiling_temp=0.3, seed=4, ene=ene)
+
+def everything():
+    got = []
+    for job in (small, large):
+        dev = g.DeviceJob(job)
+        for n in (1, 130, 2500):
+            conf, pose = random_poses(job, n, seed=n, trans=2.0)
+            conf, pose = np.ascontiguousarray(conf, np.int32), np.ascontiguousarray(pose, np.float32)
+            got += list(dev.eval(conf, pose, want_coords=True))
+            terms, raw = np.zeros((n, 10), np.float32), np.zeros((n, 9), np.float32)
+            for r in (raw.ctypes.data_as(fp), None):
+                g.check(g.lib().gd_energy_eval_noalloc(dev.h, n, conf.ctypes.data_as(ip), pose.ctypes.data_as(fp),
+                                                       terms.ctypes.data_as(fp), r), "noalloc")
+            got += [terms, raw]
+        for wait in (2.0, 0.0):  # 0: the failure word comes by a copy, too
+            dev.set_step_wait(wait)
+            out, st = dev.dock(g.make_mc(24, steps_per_exchange=7, seed=3, axes=("temp", "lig", "prt")))
+            back = dev.replicas()
+            for o in (out, back):
+                got += [getattr(o, f).copy() for f in FIELDS]
+        outs = [g.host.ReplicaOut(job.n_rep)]
+        mc = g.make_mc(9, steps_per_exchange=4, seed=3)
+        g.check(g.lib().gd_batch_dock(C.byref(dev.h), 1, C.byref(mc), C.byref(outs[0].c), None), "batch")
+        got += [getattr(outs[0], f).copy() for f in FIELDS]
+        dev.close()
+    outs, errors = serve({})
+    assert errors == 0
+    return got + [getattr(o, f).copy() for o in outs for f in FIELDS]
+
+shim.refuse_pinned_over(0)
+a = everything()
+assert shim.refused_pinned() > 0
+shim.refuse_pinned_over(NONE)
+b = everything()
+assert len(a) == len(b)
+for x, y in zip(a, b):
+    assert np.array_equal(x, y)
+""")

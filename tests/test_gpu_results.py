@@ -59,3 +59,24 @@ def test_results_of_long_lists(ene):
                 assert np.array_equal(getattr(one[0], f), getattr(outs[k], f)), (k, f)
     for d in devs:
         d.close()
+
+
+def test_large_results(ene):
+    """196,608 replicas, whose results (18 MB) are copied row by row: every replica's
+    energies are those of the evaluation at its pose, and the ladders hold each
+    temperature once."""
+    nl, np_, nt = 64, 32, 96
+    job = g.synth_complex(16, 2, nl, np_, nt, floor_temp=0.05, ceiling_temp=0.3, seed=6, ene=ene)
+    dev = g.DeviceJob(job)
+    n = nl * np_ * nt
+    out, _ = dev.dock(g.make_mc(3, steps_per_exchange=1, seed=2, axes=("temp", "lig")))
+    r = np.arange(n)
+    lig, p = r % nl, r // (nl * nt)
+    terms, _, _ = dev.eval(np.stack([lig, p], 1).astype(np.int32), out.movematrix)
+    assert np.array_equal(out.energy, terms)
+    assert (out.best_energy <= out.energy[:, 9]).all()
+    assert 0 < out.n_accept.sum() <= 3 * n and set(np.unique(out.is_accept)) <= {0, 1}
+    assert out.n_exchange.sum() > 0 and out.n_swap_lig.sum() > 0 and not out.n_swap_prt.any()
+    ladders = np.sort(out.idx_tmp.reshape(np_, nt, nl).transpose(0, 2, 1), axis=2)
+    assert (ladders == np.arange(nt)).all()
+    dev.close()
