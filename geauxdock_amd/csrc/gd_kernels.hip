@@ -1174,7 +1174,7 @@ __device__ __forceinline__ void gd_reduce_wave(GdJobC &J, const int r, const int
     gd_reduce_shape<AG, true, true, 2, 12>(J, r, wi, q0, n, acc);
   } else if (small && n <= 4 && nG <= 16 && nL <= 16) {
     gd_reduce_shape<AG, true, true, 4, 16>(J, r, wi, q0, n, acc);
-  } else if (n <= 4 && nG <= 20 && nL <= 20) {
+  } else if (n <= 4 && nG <= 20 && nL <= 20 && gd_rows_fit(20, Rp)) {  // 2^26 replicas: 16 rows fit
     gd_reduce_shape<AG, false, false, 4, 20>(J, r, wi, q0, n, acc);
   } else {
 #pragma unroll

@@ -3,6 +3,9 @@
 #pragma once
 #include "gd_rng.h"
 
+// The offset of any lane in n rows of Rp floats each fits 32 bits, in bytes.
+GD_HD bool gd_rows_fit(int n, int Rp) { return (uint64_t)n * (uint64_t)Rp <= (1ull << 30); }
+
 // Queue entries [at, at + n) of the stepping kernel lie in a queue of `limit`.  `at`
 // is a difference of two counters that run on from launch to launch: after a
 // launch that failed it can be negative (the launch queued fewer entries than the

@@ -18,6 +18,20 @@ def _run(tmp_path, body):
     assert r.returncode == 0, r.stdout
 
 
+def test_rows_fit(tmp_path):
+    """Row offsets are 32 bits: 16 rows and fewer fit at every replica count that is
+    accepted (2^26), and 20 rows up to the last count whose last lane does."""
+    _run(tmp_path, """
+  for (long long Rp : {64ll, 1ll << 20, 53687040ll, 53687104ll, (1ll << 26) - 64, 1ll << 26})
+    for (int n : {1, 2, 4, 8, 12, 16, 20}) {
+      const long long last = ((n - 1) * Rp + Rp - 1) * 4 + 3;  // its last byte
+      bad += gd_rows_fit(n, (int)Rp) != (last < (1ll << 32));
+      bad += n <= 16 && !gd_rows_fit(n, (int)Rp);
+    }
+  bad += gd_rows_fit(20, 1 << 26);
+""")
+
+
 def test_queue_room(tmp_path):
     """Entries before the queue's start are refused also where their end wraps to
     its first ones: 8 blocks' entries queued one launch of one step late."""
