@@ -637,10 +637,12 @@ extern "C" gd_status gd_autotune(gd_job *j, int steps, gd_tiling *best, double *
   return GD_OK;
 }
 
-// Shared launches: protein tile points x persistent-grid waves per CU (4 atoms
-// per lane), each candidate a whole batched run of `steps` MC steps of the
-// given jobs (graph-captured as gd_batch_dock runs them); the shortest run
-// wins.  The jobs are left at the shared tiling of the table.
+// Shared launches, 4 atoms per lane, each candidate a whole batched run of `steps`
+// MC steps of the given jobs: the protein tile points as gd_batch_dock steps them
+// (by the stepping kernel where the lists suit it), then, at the best of these, the
+// waves per CU of the persistent grid of launches (for lists that do not suit it, and
+// swap passes).  The shortest run wins.  The jobs are left at the shared tiling of
+// the table.
 extern "C" gd_status gd_autotune_shared(gd_job **jobs, int n_jobs, int steps, gd_tiling *best,
                                         double *best_ms) {
   if (!jobs || n_jobs <= 0 || steps <= 0) return GD_ERR_ARG;
@@ -648,20 +650,23 @@ extern "C" gd_status gd_autotune_shared(gd_job **jobs, int n_jobs, int steps, gd
   if (st != GD_OK) return st;
   std::vector<gd_mc_param> mc(n_jobs, tune_mc(steps));
   for (int k = 0; k < n_jobs; ++k) mc[k].job_id = (uint32_t)k;
-  double best_t = 1e300;
+  double t = 0.0, best_t = 1e300, best_launches = 1e300;
   int best_pt = 0, best_w = 0;
-  for (int pt : {32, 40, 48, 64, 80, 96, 128})
-    for (int w : {16, 24, 32}) {
-      if ((st = batch_dock_impl(jobs, n_jobs, mc.data(), nullptr, nullptr, pt, w)) != GD_OK) return st;
-      const auto t0 = std::chrono::steady_clock::now();
-      if ((st = batch_dock_impl(jobs, n_jobs, mc.data(), nullptr, nullptr, pt, w)) != GD_OK) return st;
-      const double t = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-      if (t < best_t) {
-        best_t = t;
-        best_pt = pt;
-        best_w = w;
-      }
-    }
+  const auto run = [&](int pt, int w) {  // w 0: as batches are stepped; else by launches of that grid
+    gd_status r = batch_dock_impl(jobs, n_jobs, mc.data(), nullptr, nullptr, pt, w);
+    const auto t0 = std::chrono::steady_clock::now();
+    if (r == GD_OK) r = batch_dock_impl(jobs, n_jobs, mc.data(), nullptr, nullptr, pt, w);
+    t = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+    return r;
+  };
+  for (int pt : {32, 40, 48, 64, 80, 96, 128}) {
+    if ((st = run(pt, 0)) != GD_OK) return st;
+    if (t < best_t) best_t = t, best_pt = pt;
+  }
+  for (int w : {16, 24, 32}) {
+    if ((st = run(best_pt, w)) != GD_OK) return st;
+    if (t < best_launches) best_launches = t, best_w = w;
+  }
   for (int k = 0; k < n_jobs; ++k)
     if ((st = shared_tiling(jobs[k], 0)) != GD_OK) return st;
   if (best) {

@@ -11,8 +11,9 @@ alone.
   shared launches (batches, serving): for each (L, P) bucket of the screening
       sizes (L 12-80, P 1,500-9,000), gd_autotune_shared on a batch of 16
       complexes of a screen (one target, ligands of the bucket, 10 x 11 x 4
-      replicas), 32 MC steps per candidate: protein tile points x persistent
-      waves per CU.  The waves per CU most buckets pick is kept for all.
+      replicas), 32 MC steps per candidate: protein tile points, then the
+      persistent grid's waves per CU.  The waves per CU most buckets pick is
+      kept for all.
   one job per launch: for each (chunks, P, R) bucket of the configurations'
       plain jobs (L 12-80 in 4-atom chunks, R = 25, 220, 440, 880, 1,760),
       gd_autotune on a synthetic complex on the library's default streams, 128

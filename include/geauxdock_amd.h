@@ -302,9 +302,10 @@ gd_status gd_tiling_set(gd_job *job, const gd_tiling *t);
  * reference's counterpart, the disabled CalcThreadBlockShape of
  * backend_gpu/kernel_cuda_l2_util.cu:40-67, is a formula). */
 gd_status gd_autotune(gd_job *job, int steps, gd_tiling *best, double *best_ms);
-/* Sweep the tiling of shared launches (protein tile points x persistent-grid
- * waves per CU, 4 atoms per lane) on a batch of these jobs, `steps` MC steps
- * per candidate; returns the fastest.  Nothing process-wide changes: the
+/* Sweep the tiling of shared launches (4 atoms per lane) on a batch of these jobs,
+ * `steps` MC steps per candidate: protein tile points as gd_batch_dock steps the
+ * batch (*best_ms is its time with the fastest), then, with these, the waves per CU
+ * of the persistent grid of launches.  Nothing process-wide changes: the
  * library's tilings come from its tuned table (geauxdock_amd/tune.py writes
  * it from these sweeps). */
 gd_status gd_autotune_shared(gd_job **jobs, int n_jobs, int steps, gd_tiling *best, double *best_ms);
