@@ -59,6 +59,33 @@ def test_plain(ene, shape, spe):
     dev.close()
 
 
+@pytest.mark.parametrize("blocking", [False, True])
+@pytest.mark.parametrize("dump,spe", [(5, 4), (1, 0), (7, 7), (20, 3)])
+def test_streamed(ene, dump, spe, blocking):
+    """Every dump is handed over once, and is that of a run by launches: whole runs
+    that fail in their first dump, on a job that steps by the kernel before and
+    after."""
+    dev = g.DeviceJob(_job(ene, FOUR))
+    mc = g.make_mc(20, steps_per_dump=dump, steps_per_exchange=spe, seed=3, axes=("temp", "lig"))
+    runs = []
+    for way in ("kernel", "failing", "kernel", "launches"):
+        dev.set_step_wait(0.0 if way == "failing" else 2.0)
+        if way == "launches":
+            dev.set_streams(1)
+        dumps = []
+        out, st = dev.dock_stream(mc, lambda k, s0, rec, cnt: dumps.append((k, s0, rec, cnt)), blocking=blocking)
+        assert (st.n_pair_launch == 21) == (way == "kernel"), (way, st.n_pair_launch)
+        runs.append((out, dumps))
+    assert [d[:2] for d in runs[0][1]] == [(k, s) for k, s in enumerate(range(0, 20, dump))]
+    for out, dumps in runs[1:]:
+        _same(runs[0][0], out)
+        assert [d[:2] for d in dumps] == [d[:2] for d in runs[0][1]]
+        for a, b in zip(dumps, runs[0][1]):
+            keep = np.arange(a[2].shape[1])[None, :] < a[3][:, None]
+            assert np.array_equal(a[3], b[3]) and np.array_equal(a[2][keep], b[2][keep])
+    dev.close()
+
+
 @pytest.mark.parametrize("spe", [1, 3])
 def test_batch(ene, spe):
     devs = [g.DeviceJob(_job(ene, s, seed=k + 1)) for k, s in enumerate([FOUR, (300, 9, 3, 2, 1), SEVEN])]
