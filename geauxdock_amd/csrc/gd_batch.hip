@@ -1,10 +1,12 @@
-// gd_batch.hip -- many complexes in shared launches: batched docking
-// (persistent work-queue pair kernel, graph-captured sweep segments), the
-// tiling autotuner, and the continuous-batching serving loop.
+// gd_batch.hip -- many complexes in shared launches: batched docking (the
+// stepping kernel; for lists that do not suit it the persistent work-queue pair
+// kernel and graph-captured segments), the tiling autotuner, and the
+// continuous-batching serving loop.
 //
 // A "batch" concatenates the device structs of its jobs into one array, and
-// their work items and 64-replica blocks into one list each, so one pair,
-// one reduce and one finish launch advance every job by one MC step.  Each job
+// their work items and 64-replica blocks into one list each, so one launch of the
+// stepping kernel advances every job to the next exchange point, or one pair, one
+// reduce and one finish launch by one MC step.  Each job
 // keeps its own tiling, replica order, Philox stream (seed, job_id) and step
 // counter (launch step - step0), so a job computes bit-identical results
 // alone or inside any batch.  The reference has no counterpart: its MPI

@@ -1,6 +1,9 @@
 // gd_kernels.hip -- hand-written gfx950 kernels of the Monte Carlo hot path.
 //
-// One MC step of every replica is three launches:
+// One MC step of every replica is a pair, a reduce and a finish phase: the work of
+// gd_chain_kernel, which takes all steps between two exchange points in one launch
+// (jobs and lists of several 64-replica blocks, 4 atoms per lane), or three launches
+// a step:
 //   gd_pair_kernel   one 8-wave work group per item (64 replicas x one
 //                    ligand-atom chunk x eight protein tiles, one per wave):
 //                    PRT pair terms, the tiles' slices of the KDE anchors and
@@ -20,8 +23,9 @@
 //                    (Philox4x32-10, counter-based).
 // plus gd_start_kernel (replica table and ligands of a run's start),
 // gd_eval_setup_kernel (the poses of an energy evaluation as lanes),
-// gd_pack_kernel (results to the host), gd_exchange_kernel (temperature swaps) and
-// the pose-swap kernels gd_swap_propose_kernel / gd_swap_accept_kernel.
+// gd_pack_kernel (results to the host), gd_keep_kernel (the state of a run kept
+// aside), gd_exchange_kernel (temperature swaps) and the pose-swap kernels
+// gd_swap_propose_kernel / gd_swap_accept_kernel.
 //
 // The reference computes the same quantities in one CUDA block per replica
 // (backend_gpu/kernel_cuda_l1_montecarlo.cu:29-536); here the pair loop

@@ -2,14 +2,15 @@
 // no allocation at all, for callers that cannot allocate device memory
 // (code under HIP graph capture, tight serving loops, harnesses that forbid
 // it).  The kernels' scratch -- the evaluation's copy of the job struct, its
-// poses, transformed ligands and partial sums -- lives in one file-scope device array of GD_NOALLOC_SCRATCH_BYTES, held by
-// every GPU the library runs on until the process ends.
+// poses, transformed ligands and partial sums -- lives in one file-scope device
+// array of GD_NOALLOC_SCRATCH_BYTES, held by every GPU the library runs on until
+// the process ends.
 //
 // Same kernels and the same tiling as gd_energy_eval, so the results are the
 // same bits.  Poses run in passes of whole 64-lane blocks that fit the scratch
 // and the device's host buffer for inputs and results, which was made with its
-// first job (without it they are copied).  Every call on a GPU shares both: calls that overlap on one GPU race
-// (the scratch keeps the last call's contents).
+// first job (without it they are copied).  Every call on a GPU shares both: calls
+// that overlap on one GPU race (the scratch keeps the last call's contents).
 #include <hip/hip_runtime.h>
 
 #include <cstdio>

@@ -202,7 +202,8 @@ gd_status gd_energy_eval(gd_job *job, int n_pose, const int *conf, const float *
  * the reference.  The kernels' scratch (partial sums, poses, transformed ligands)
  * lives in one static device array of GD_NOALLOC_SCRATCH_BYTES per GPU, and
  * inputs and results pass through one host buffer per GPU, made with its first
- * job; both are held until the process ends.  Poses run in passes of 64-pose
+ * job (or are copied, where there was no memory for it); both are held until the
+ * process ends.  Poses run in passes of 64-pose
  * blocks that fit them, and a job whose single block needs more scratch returns
  * GD_ERR_SIZE.  Same results, bit for bit, as gd_energy_eval (terms[n][10],
  * raw[n][9] optional; no coordinates).  The job's replica state is not touched.
@@ -262,8 +263,8 @@ void gd_record_csv_write(void *writer, int dump, int step_begin, int n_rep, int 
 /* Closes the file; returns GD_ERR_IO if any write failed. */
 gd_status gd_record_csv_close(gd_record_csv *writer);
 
-/* Many complexes in one launch sequence (persistent work-queue pair kernel,
- * graph-captured sweep segments).  mc[i] / out[i] per job. */
+/* Many complexes in one launch sequence (the stepping kernel, or the persistent
+ * work-queue pair kernel and graph-captured segments).  mc[i] / out[i] per job. */
 gd_status gd_batch_dock(gd_job **jobs, int n_jobs, const gd_mc_param *mc,
                         gd_replica_out *out, gd_stats *stats);
 
