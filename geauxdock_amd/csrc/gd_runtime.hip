@@ -1551,6 +1551,8 @@ gd_status gd_stepping_shape(int n_cu, int n_jobs, int n_rep, int lig_chunks, int
                             int *slots) {
   if (n_cu < 1 || n_jobs < 1 || n_rep < 1 || lig_chunks < 1 || tile_groups < 1 || !finishers || !slots)
     return GD_ERR_ARG;
+  if (n_cu > (1 << 20) || n_jobs > (1 << 20) || n_rep > (1 << 26) || (double)n_jobs * (n_rep + 63) / 64 * lig_chunks * tile_groups > 1e9)
+    return GD_ERR_SIZE;
   GdJob g;
   std::memset(&g, 0, sizeof g);
   g.Rp = (n_rep + 63) / 64 * 64;

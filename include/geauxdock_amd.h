@@ -237,7 +237,7 @@ gd_status gd_dock_records(gd_job *job, int cap, float *rec, int *count);
  * count[n_rep] gives the entries used in each row.  Called on the thread that
  * runs gd_dock_stream, once per dump and in dump order; the arrays are valid
  * only during the call, and the callback must not call the library on the
- * same job. */
+ * same job (but for gd_job_set_step_wait). */
 typedef void (*gd_record_fn)(void *user, int dump, int step_begin, int n_rep, int cap,
                              const float *rec, const int *count);
 enum { GD_STREAM_BLOCKING = 1 };

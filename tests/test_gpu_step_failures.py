@@ -4,6 +4,8 @@ above the line from which plain runs step by the kernel, which the counts of tim
 launches show: the kernel counts every step and the initial pass, launches 1 step
 in 16."""
 import ctypes as C
+import threading
+import time
 
 import numpy as np
 import pytest
@@ -219,8 +221,12 @@ def test_streamed_run_goes_on(ene, blocking):
     dev.close()
 
 
+def _timed(run):
+    t = time.perf_counter()
+    return run(), time.perf_counter() - t
+
+
 def _fail_after(devs, run, seconds):
-    import threading
     t = threading.Timer(seconds, lambda: [d.set_step_wait(0.0) for d in devs])
     t.start()
     try:
@@ -231,13 +237,13 @@ def _fail_after(devs, run, seconds):
 
 
 def test_plain_run_goes_on(ene):
-    """More launches than the device's queue holds, so that the bound changes part of
-    the way."""
+    """More launches than the device's queue holds, so that the bound, set to 0 after
+    half the time, counts for the later ones."""
     dev = g.DeviceJob(_job(ene, FOUR))
     mc = g.make_mc(30000, steps_per_exchange=2, seed=3, axes=("temp", "lig", "prt"))
-    want, st = dev.dock(mc)
+    (want, st), seconds = _timed(lambda: dev.dock(mc))
     assert st.n_pair_launch == 30001
-    out, st = _fail_after([dev], lambda: dev.dock(mc), 0.7)
+    out, st = _fail_after([dev], lambda: dev.dock(mc), seconds / 2)
     _same(want, out)
     assert 0 < st.n_pair_launch <= 2 * (22000 // 16 + 1), st.n_pair_launch
     dev.close()
@@ -249,8 +255,8 @@ def test_plain_run_goes_on(ene):
 def test_batch_goes_on(ene, steps, stats):
     devs = [g.DeviceJob(_job(ene, s, seed=k + 1)) for k, s in enumerate([SEVEN, (300, 9, 3, 2, 1), SEVEN])]
     mcs = [g.make_mc(n, steps_per_exchange=48, seed=3, job_id=k, axes=("temp", "lig")) for k, n in enumerate(steps)]
-    want, _ = _batch(devs, mcs)
-    got, st = _fail_after(devs[:1], lambda: _batch(devs, mcs, stats=stats), 0.55)
+    (want, _), seconds = _timed(lambda: _batch(devs, mcs))
+    got, st = _fail_after(devs[:1], lambda: _batch(devs, mcs, stats=stats), 0.6 * seconds)
     for a, b in zip(want, got):
         _same(a, b)
     if stats:  # by launches from a kept state on

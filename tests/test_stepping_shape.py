@@ -26,3 +26,4 @@ def test_arguments():
     f = C.c_int()
     assert g.lib().gd_stepping_shape(0, 1, 1, 1, 1, C.byref(f), C.byref(f)) == abi.GD_ERR_ARG
     assert g.lib().gd_stepping_shape(1, 1, 1, 1, 1, None, C.byref(f)) == abi.GD_ERR_ARG
+    assert g.lib().gd_stepping_shape(256, 1, 1 << 26, 1 << 20, 1, C.byref(f), C.byref(f)) == abi.GD_ERR_SIZE
