@@ -74,8 +74,10 @@ struct BatchLists {
   bool suits = false, with_turn = false;  // the lists suit it; they were made with its turn
   double wait_s = GD_CHAIN_WAIT_S;  // bound of its waits (in a batch a job's, if shorter)
   bool failed = false;       // it failed on lists that were rebuilt since
-  void *qmem = nullptr;      // its counters, then its queue; grows only
-  size_t sync_bytes = 0, queue_bytes = 0;
+  void *qmem = nullptr;      // its counters, its queue, then room for kept state (keeps); grows only
+  size_t sync_bytes = 0, queue_bytes = 0, keep_size = 0;
+  bool keeps = false;
+  unsigned *keep() const { return (unsigned *)((char *)qmem + sync_bytes + queue_bytes); }
   BatchLists() = default;
   BatchLists(const BatchLists &) = delete;
   BatchLists &operator=(const BatchLists &) = delete;
@@ -84,7 +86,8 @@ struct BatchLists {
     if (qmem) (void)hipFree(qmem);
   }
   // Counters and queue for the lists of `chain`.  The queue
-  // keeps its contents: entries of earlier launches hold earlier epochs.
+  // keeps its contents: entries of earlier launches hold earlier epochs.  So does the
+  // kept state, also where the rest grows or there is no memory for that.
   gd_status chain_memory(hipStream_t s) {
     if (qmem && chain.epoch > 0) {
       unsigned f = 0;
@@ -93,17 +96,21 @@ struct BatchLists {
       if (e != hipSuccess) return hip_fail(e, "stepping kernel status");
       failed = failed || f != 0;
     }
-    const size_t bs = (chain_sync_bytes(chain.n_blocks) + 255) / 256 * 256, bq = chain.queue_bytes();
+    const size_t bs = (chain_sync_bytes(chain.n_blocks) + 255) / 256 * 256,
+                 bq = chain.queue_bytes(), bk = keeps ? keep_bytes(chain.n_blocks) : 0;
     hipError_t e = hipSuccess;
-    if (bs > sync_bytes || bq > queue_bytes) {
-      if (qmem) (void)hipFree(qmem);
-      qmem = nullptr;
-      sync_bytes = std::max(sync_bytes, bs), queue_bytes = std::max(queue_bytes, bq);
-      if ((e = hipMalloc(&qmem, sync_bytes + queue_bytes)) != hipSuccess) {
-        sync_bytes = queue_bytes = 0;
-        return hip_fail(e, "hipMalloc stepping queue");
+    if (bs > sync_bytes || bq > queue_bytes || bk > keep_size) {
+      const size_t ns = std::max(sync_bytes, bs), nq = std::max(queue_bytes, bq), nk = std::max(keep_size, bk);
+      void *to = nullptr;
+      if ((e = hipMalloc(&to, ns + nq + nk)) != hipSuccess) return hip_fail(e, "hipMalloc stepping queue");
+      if (qmem) {
+        if (keep_size > 0) e = hipMemcpyAsync((char *)to + ns + nq, keep(), keep_size, hipMemcpyDeviceToDevice, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        (void)hipFree(qmem);
       }
-      e = hipMemsetAsync(qmem, 0, sync_bytes + queue_bytes, s);
+      qmem = to;
+      sync_bytes = ns, queue_bytes = nq, keep_size = nk;
+      if (e == hipSuccess) e = hipMemsetAsync(qmem, 0, sync_bytes + queue_bytes, s);
     } else {
       e = hipMemsetAsync(qmem, 0, sync_bytes, s);
     }
@@ -198,7 +205,7 @@ struct BatchLists {
   }
 };
 
-// Device memory for the state that a batch or a server keeps (launch_keep).
+// Device memory for the state that a batch keeps (launch_keep): it outlives the lists.
 struct KeepArea {
   unsigned *mem = nullptr;
   size_t bytes = 0;
@@ -777,7 +784,6 @@ struct gd_server {
   BatchLists lists;
   bool dirty = true;
   int launch_sweeps = 0;         // sweeps by launches to come, after a wait of the stepping kernel ran out of time
-  KeepArea keep;                 // the active jobs' state at the sweep's first launch of it
   int lc = kSharedLc;
   std::chrono::steady_clock::time_point t0;
   // host input pipeline: file requests parsed by a loader thread
@@ -862,6 +868,7 @@ extern "C" gd_status gd_server_create(const gd_server_config *cfg, gd_server **o
     return hip_fail(e, "hipStreamCreate");
   }
   gdr::host_pool_users(1);
+  s->lists.keeps = true;
   *out = s;
   return GD_OK;
 }
@@ -1152,7 +1159,6 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
   // and the steps they had taken
   std::vector<ServJob *> kept;
   std::vector<int> kept_steps;
-  bool no_keep = false;
   for (int k = 0; k < s->cfg.sweep_steps && st == GD_OK; ++k) {
     std::vector<int> act;
     std::vector<gd_job *> jobs;
@@ -1170,16 +1176,13 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
       s->dirty = false;
     }
     // by the stepping kernel up to the next exchange point or end of any job
-    if (turn.mine && s->lists.chain_max > 0 && kept.empty() && !no_keep) {
-      no_keep = s->keep.make(s->lists.n_blocks, hs) != GD_OK;  // no memory: by launches
-      if (!no_keep) {
-        if ((st = launch_keep(false, s->lists.d_jobs, s->lists.d_blocks, s->lists.n_blocks, s->keep.mem,
-                              (const unsigned *)s->lists.qmem + GD_SY_FAILED, 1, hs)) != GD_OK)
-          break;
-        for (int q : act) kept.push_back(s->active[q]), kept_steps.push_back(s->active[q]->done_steps);
-      }
+    const bool chain = turn.mine && s->lists.chain_max > 0;
+    if (chain && kept.empty()) {
+      if ((st = launch_keep(false, s->lists.d_jobs, s->lists.d_blocks, s->lists.n_blocks, s->lists.keep(),
+                            (const unsigned *)s->lists.qmem + GD_SY_FAILED, 1, hs)) != GD_OK)
+        break;
+      for (int q : act) kept.push_back(s->active[q]), kept_steps.push_back(s->active[q]->done_steps);
     }
-    const bool chain = turn.mine && s->lists.chain_max > 0 && !no_keep;
     int n = 1;
     if (chain) {
       n = std::min(s->lists.chain_max, s->cfg.sweep_steps - k);
@@ -1240,7 +1243,7 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
       BatchLists B;
       e = hipMemsetAsync(s->lists.qmem, 0, s->lists.sync_bytes, hs);
       st = e == hipSuccess ? B.build(jobs, all, hs, nullptr) : hip_fail(e, "stepping kernel counters");
-      if (st == GD_OK) st = launch_keep(true, B.d_jobs, B.d_blocks, B.n_blocks, s->keep.mem, nullptr, 1, hs);
+      if (st == GD_OK) st = launch_keep(true, B.d_jobs, B.d_blocks, B.n_blocks, s->lists.keep(), nullptr, 1, hs);
       e = hipStreamSynchronize(hs);
       if (st == GD_OK && e != hipSuccess) st = hip_fail(e, "kept state");
       s->dirty = true;
