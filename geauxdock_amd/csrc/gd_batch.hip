@@ -87,7 +87,9 @@ struct BatchLists {
   }
   // Counters and queue for the lists of `chain`.  The queue
   // keeps its contents: entries of earlier launches hold earlier epochs.  So does the
-  // kept state, also where the rest grows or there is no memory for that.
+  // kept state, also where the rest grows or there is no memory for that.  A queue of
+  // 1 MB is what most lists ask for, a little more or less (ChainList::shape): with less
+  // it grew by a little as jobs left the lists.
   gd_status chain_memory(hipStream_t s) {
     if (qmem && chain.epoch > 0) {
       unsigned f = 0;
@@ -97,7 +99,7 @@ struct BatchLists {
       failed = failed || f != 0;
     }
     const size_t bs = (chain_sync_bytes(chain.n_blocks) + 255) / 256 * 256,
-                 bq = chain.queue_bytes(), bk = keeps ? keep_bytes(chain.n_blocks) : 0;
+                 bq = std::max(chain.queue_bytes(), (size_t)1 << 20), bk = keeps ? keep_bytes(chain.n_blocks) : 0;
     hipError_t e = hipSuccess;
     if (bs > sync_bytes || bq > queue_bytes || bk > keep_size) {
       const size_t ns = std::max(sync_bytes, bs), nq = std::max(queue_bytes, bq), nk = std::max(keep_size, bk);
