@@ -474,6 +474,7 @@ gd_status batch_run(gd_job **jobs_in, int n_jobs, const gd_mc_param *mc, gd_repl
     if (act.size() != (size_t)B.n_jobs) {
       // shrink the lists to the jobs still running; their step0 stays 0
       if ((st = B.build(jobs, act, s, stepping)) != GD_OK) break;
+      if (B.failed) break;  // the counters are new and hold no mark of it: nothing more is to be kept
     }
     int n = 1;
     const bool chain = B.chain_max > 0;
@@ -1174,8 +1175,9 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
         (stepping && s->lists.suits && turn.take() && !s->lists.with_turn)) {
       for (int q : act) jobs[q]->h.step0 = s->active[q]->step0;
       s->dirty = true;  // until they are whole
-      if ((st = s->lists.build(jobs, act, hs, stepping)) != GD_OK) return st;
+      if ((st = s->lists.build(jobs, act, hs, stepping)) != GD_OK) break;
       s->dirty = false;
+      if (s->lists.failed) break;
     }
     // by the stepping kernel up to the next exchange point or end of any job
     const bool chain = turn.mine && s->lists.chain_max > 0;
@@ -1194,10 +1196,7 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
         n = std::min(n, j->mc.steps_total - j->done_steps);
         if (spe > 0) n = std::min(n, spe - j->done_steps % spe);
       }
-      if ((st = launch_chain(s->lists.chain, s->lists.d_jobs, s->launch_step, n, false, hs)) != GD_OK) {
-        (void)hipStreamSynchronize(hs);
-        return st;  // the steps were not taken: the next call takes them
-      }
+      if ((st = launch_chain(s->lists.chain, s->lists.d_jobs, s->launch_step, n, false, hs)) != GD_OK) break;
     }
     std::vector<int> round(act.size(), -1);
     for (int q = 0; q < (int)act.size(); ++q) {
@@ -1222,47 +1221,49 @@ extern "C" gd_status gd_server_step(gd_server *s, int *n_active, int *n_done) {
     if (any_done) s->dirty = true;
   }
   hipError_t e = hipStreamSynchronize(hs);
-  if (st == GD_OK && e != hipSuccess) st = hip_fail(e, "sweep");
-  if (st != GD_OK) return st;
-  if (turn.mine && s->lists.qmem) {
+  if (e != hipSuccess) return hip_fail(e, "sweep");
+  if (!kept.empty()) {
     unsigned f = 0;
     e = hipMemcpy(&f, (unsigned *)s->lists.qmem + GD_SY_FAILED, sizeof f, hipMemcpyDeviceToHost);
     if (e != hipSuccess) return hip_fail(e, "stepping kernel status");
-    if (f || s->lists.failed) {
-      // a wait ran out of time: the jobs go on from the state that was kept, by
-      // launches (the same bits: a job's draws are a function of its own steps)
-      s->launch_sweeps = kLaunchSweeps;
+    const bool late = f || s->lists.failed;
+    if (late || st != GD_OK) {
+      // a wait ran out of time, or a launch was refused: the jobs go on from the state
+      // that was kept, in the first case by launches (the same bits: a job's draws are a
+      // function of its own steps).  Job by job, which takes no memory
+      if (late) s->launch_sweeps = kLaunchSweeps;
       s->lists.failed = false;
-      std::vector<gd_job *> jobs;
-      std::vector<int> all;
-      for (size_t q = 0; q < kept.size(); ++q) {
-        ServJob *j = kept[q];
-        j->done_steps = kept_steps[q];
-        j->job->h.step0 = j->step0 = s->launch_step - j->done_steps;
-        jobs.push_back(j->job);
-        all.push_back((int)q);
-      }
-      BatchLists B;
-      e = hipMemsetAsync(s->lists.qmem, 0, s->lists.sync_bytes, hs);
-      st = e == hipSuccess ? B.build(jobs, all, hs, nullptr) : hip_fail(e, "stepping kernel counters");
-      if (st == GD_OK) st = launch_keep(true, B.d_jobs, B.d_blocks, B.n_blocks, s->lists.keep(), nullptr, 1, hs);
-      e = hipStreamSynchronize(hs);
-      if (st == GD_OK && e != hipSuccess) st = hip_fail(e, "kept state");
       s->dirty = true;
-      if (st != GD_OK) {
+      e = hipMemsetAsync(s->lists.qmem, 0, s->lists.sync_bytes, hs);
+      gd_status rs = e == hipSuccess ? GD_OK : hip_fail(e, "stepping kernel counters");
+      unsigned *area = s->lists.keep();
+      for (size_t q = 0; q < kept.size() && rs == GD_OK; ++q) {
+        ServJob *j = kept[q];
+        gd_job *job = j->job;
+        j->done_steps = kept_steps[q];
+        job->h.step0 = j->step0 = s->launch_step - j->done_steps;
+        e = hipMemcpyAsync(job->d_job, &job->h, sizeof(GdJob), hipMemcpyHostToDevice, hs);
+        rs = e == hipSuccess ? launch_keep(true, job->d_job, job->d_blocks, job->n_blocks, area, nullptr, 1, hs)
+                             : hip_fail(e, "kept state");
+        area += (size_t)job->n_blocks * GD_KEEP_ROWS * 64;
+      }
+      e = hipStreamSynchronize(hs);
+      if (rs == GD_OK && e != hipSuccess) rs = hip_fail(e, "kept state");
+      if (rs != GD_OK) {
         // neither steps nor state to go on from: report each
         std::lock_guard<std::mutex> lk(s->mu);
         for (ServJob *j : kept) {
-          fail_request(s, j->ticket, st, j->t_submit, j->t_admit);
+          fail_request(s, j->ticket, rs, j->t_submit, j->t_admit);
           s->used -= j->foot;
           s->active.erase(std::find(s->active.begin(), s->active.end(), j));
           gd_job_destroy(j->job);
           delete j;
         }
-        return st;
+        return rs;
       }
     }
   }
+  if (st != GD_OK) return st;
   // (4) convergence: a job's sweep ends every sweep_steps of its own steps
   if (s->cfg.converge_sweeps > 0) {
     for (ServJob *j : s->active) {

@@ -47,7 +47,7 @@ def serve(refuse):
     done = errors = 0
     for k in range(40):
         if k in refuse:
-            refuse[k]()
+            refuse[k](s)
         na, nd, n, res = C.c_int(), C.c_int(), C.c_int(), (abi.gd_job_result * 8)()
         errors += g.lib().gd_server_step(s, C.byref(na), C.byref(nd)) != 0
         shim.refuse_device_over(NONE)
@@ -70,18 +70,33 @@ def test_refused_sweep(tmp_path, after):
     """The first or second stepping launch of a sweep is refused: the call is an
     error, and the next ones take the steps that it did not."""
     hip_refuse.run(tmp_path, _SERVE + """
-got, errors = serve({1: lambda: shim.refuse_stepping_after(%d)})
+got, errors = serve({1: lambda s: shim.refuse_stepping_after(%d)})
 assert errors == 1
 for a, b in zip(want, got):
     same(a, b)
 """ % after)
 
 
+def test_refused_sweep_after_a_time_out(tmp_path):
+    """The first stepping launch of a sweep runs out of time and the second is refused:
+    the sweep is taken again from its start."""
+    hip_refuse.run(tmp_path, _SERVE + """
+def both(s):
+    g.check(g.lib().gd_server_set_step_wait(s, 0.0), "wait")
+    shim.refuse_stepping_after(1)
+
+got, errors = serve({1: both, 2: lambda s: g.check(g.lib().gd_server_set_step_wait(s, 2.0), "wait")})
+assert errors == 1
+for a, b in zip(want, got):
+    same(a, b)
+""")
+
+
 def test_refused_lists(tmp_path):
     """No memory for the lists of a sweep whose jobs have changed: an error, and
     the lists are made by the next call."""
     hip_refuse.run(tmp_path, _SERVE + """
-got, errors = serve({k: lambda: shim.refuse_device_over(0) for k in range(1, 8)})
+got, errors = serve({k: lambda s: shim.refuse_device_over(0) for k in range(1, 8)})
 assert errors >= 1
 for a, b in zip(want, got):
     same(a, b)

@@ -263,3 +263,20 @@ def test_batch_goes_on(ene, steps, stats):
         assert 0 < st.n_pair_launch <= 10000 // 16, st.n_pair_launch
     for d in devs:
         d.close()
+
+
+def test_batch_fails_before_its_list_shrinks(ene):
+    """Only the job that ends at step 9,000 bounds the waits to 0, from step 6,000 or so
+    on: the launches after it has left the list run in time, on a state that is not
+    to be kept."""
+    devs = [g.DeviceJob(_job(ene, SEVEN, seed=k + 1)) for k in range(2)]
+    mcs = [g.make_mc(n, steps_per_exchange=48, seed=3, job_id=k, axes=("temp", "lig"))
+           for k, n in enumerate((26000, 9000))]
+    _, first = _timed(lambda: _batch(devs, [mcs[1], mcs[1]]))
+    want, _ = _batch(devs, mcs)
+    got, st = _fail_after(devs[1:], lambda: _batch(devs, mcs, stats=True), 0.7 * first)
+    assert 0 < st.n_pair_launch < 26000 // 16
+    for a, b in zip(want, got):
+        _same(a, b)
+    for d in devs:
+        d.close()
